@@ -20,6 +20,7 @@
 #include "kh_batch.h"
 #include "kh_fused.h"
 #include "kh_launch.h"
+#include "kh_transfer.h"
 #include "kh_zwave.h"
 
 using namespace kh;
@@ -159,6 +160,7 @@ struct kh_run {
     int             *bid   = nullptr;   // np: body of each bead
     double          *flo   = nullptr;   // np x 3: LJ force from partners of higher index
     std::vector<int> sek_host;          // the packed Sekibun offsets (host copy, for the initial block)
+    RowStage         stage;             // pinned staging of the field transfers
     // measurement
     bool                               timing = false;
     std::map<std::string, KernelTimes> times;
@@ -972,74 +974,37 @@ struct Step {
 
 // ------------------------------------------------------------ transfers
 // host reference layout [NX][NY][NZ_] (real in k < NZ) <-> device [NX][NY][NZ]
-int upload_real(kh_run *r, void *dev, const double *host) {
-    const Grid &g   = r->g;
-    const int   nz_ = 2 * g.nzh;
-    if (!r->mixed) {
-        KH_HIP(hipMemcpy2DAsync(dev, sizeof(double) * g.nz, host, sizeof(double) * nz_, sizeof(double) * g.nz,
-                                (size_t)g.nx * g.ny, hipMemcpyHostToDevice, r->stream));
-        KH_HIP(hipStreamSynchronize(r->stream));
-    } else {
-        std::vector<float> tmp((size_t)g.nreal);
-        for (long long row = 0; row < (long long)g.nx * g.ny; row++)
-            for (int k = 0; k < g.nz; k++) tmp[(size_t)row * g.nz + k] = (float)host[(size_t)row * nz_ + k];
-        KH_HIP(hipMemcpyAsync(dev, tmp.data(), sizeof(float) * tmp.size(), hipMemcpyHostToDevice, r->stream));
-        KH_HIP(hipStreamSynchronize(r->stream));
-    }
-    return KH_OK;
-}
-int download_real(kh_run *r, double *host, const void *dev) {
-    const Grid &g   = r->g;
-    const int   nz_ = 2 * g.nzh;
-    if (!r->mixed) {
-        KH_HIP(hipMemcpy2DAsync(host, sizeof(double) * nz_, dev, sizeof(double) * g.nz, sizeof(double) * g.nz,
-                                (size_t)g.nx * g.ny, hipMemcpyDeviceToHost, r->stream));
-        KH_HIP(hipStreamSynchronize(r->stream));
-    } else {
-        std::vector<float> tmp((size_t)g.nreal);
-        KH_HIP(hipMemcpyAsync(tmp.data(), dev, sizeof(float) * tmp.size(), hipMemcpyDeviceToHost, r->stream));
-        KH_HIP(hipStreamSynchronize(r->stream));
-        for (long long row = 0; row < (long long)g.nx * g.ny; row++)
-            for (int k = 0; k < g.nz; k++) host[(size_t)row * nz_ + k] = tmp[(size_t)row * g.nz + k];
-    }
-    for (long long row = 0; row < (long long)g.nx * g.ny; row++)
-        for (int k = g.nz; k < nz_; k++) host[(size_t)row * nz_ + k] = 0.0;
-    return KH_OK;
+RowField real_rows(kh_run *r, const void *dev, const double *host) {
+    const Grid &g = r->g;
+    return {const_cast<void *>(dev), const_cast<double *>(host), (long long)g.nx * g.ny, g.nz, g.nz, 2 * g.nzh,
+            r->mixed != 0};
 }
 // spectral: host rows of NZ_ = 2 nzh doubles ((re,im) of kz at [2kz]),
-// device rows nzp complex apart (padding left untouched); FP32 runs convert
-int upload_spec(kh_run *r, void *dev, const double *host) {
-    const Grid     &g    = r->g;
-    const long long rows = (long long)g.nx * g.ny;
-    if (!r->mixed) {
-        KH_HIP(hipMemcpy2DAsync(dev, sizeof(double) * 2 * g.nzp, host, sizeof(double) * 2 * g.nzh,
-                                sizeof(double) * 2 * g.nzh, (size_t)rows, hipMemcpyHostToDevice, r->stream));
-    } else {
-        std::vector<float> tmp((size_t)g.nspec * 2, 0.f);
-        for (long long row = 0; row < rows; row++)
-            for (int k = 0; k < 2 * g.nzh; k++)
-                tmp[(size_t)row * 2 * g.nzp + k] = (float)host[(size_t)row * 2 * g.nzh + k];
-        KH_HIP(hipMemcpyAsync(dev, tmp.data(), sizeof(float) * tmp.size(), hipMemcpyHostToDevice, r->stream));
-    }
-    KH_HIP(hipStreamSynchronize(r->stream));
+// device rows nzp complex apart (padding left untouched)
+RowField spec_rows(kh_run *r, const void *dev, const double *host) {
+    const Grid &g = r->g;
+    return {const_cast<void *>(dev), const_cast<double *>(host), (long long)g.nx * g.ny, 2 * g.nzp, 2 * g.nzh,
+            2 * g.nzh, r->mixed != 0};
+}
+int move(kh_run *r, const RowField *f, int n, bool to_host) {
+    KH_HIP(move_rows(r->stage, r->device, f, n, to_host, r->stream));
     return KH_OK;
 }
+int upload_real(kh_run *r, void *dev, const double *host) {
+    const RowField f = real_rows(r, dev, host);
+    return move(r, &f, 1, false);
+}
+int download_real(kh_run *r, double *host, const void *dev) {
+    const RowField f = real_rows(r, dev, host);
+    return move(r, &f, 1, true);
+}
+int upload_spec(kh_run *r, void *dev, const double *host) {
+    const RowField f = spec_rows(r, dev, host);
+    return move(r, &f, 1, false);
+}
 int download_spec(kh_run *r, double *host, const void *dev) {
-    const Grid     &g    = r->g;
-    const long long rows = (long long)g.nx * g.ny;
-    if (!r->mixed) {
-        KH_HIP(hipMemcpy2DAsync(host, sizeof(double) * 2 * g.nzh, dev, sizeof(double) * 2 * g.nzp,
-                                sizeof(double) * 2 * g.nzh, (size_t)rows, hipMemcpyDeviceToHost, r->stream));
-        KH_HIP(hipStreamSynchronize(r->stream));
-    } else {
-        std::vector<float> tmp((size_t)g.nspec * 2);
-        KH_HIP(hipMemcpyAsync(tmp.data(), dev, sizeof(float) * tmp.size(), hipMemcpyDeviceToHost, r->stream));
-        KH_HIP(hipStreamSynchronize(r->stream));
-        for (long long row = 0; row < rows; row++)
-            for (int k = 0; k < 2 * g.nzh; k++)
-                host[(size_t)row * 2 * g.nzh + k] = tmp[(size_t)row * 2 * g.nzp + k];
-    }
-    return KH_OK;
+    const RowField f = spec_rows(r, dev, host);
+    return move(r, &f, 1, true);
 }
 
 void *field_buffer(kh_run *r, int field) {
@@ -1078,6 +1043,7 @@ int free_run(kh_run *r) {
         (void)hipEventDestroy(p.b);
     }
     for (auto e : r->event_pool) (void)hipEventDestroy(e);
+    r->stage.release();
     if (r->stream) (void)hipStreamDestroy(r->stream);
     delete r;
     return KH_OK;
@@ -1709,8 +1675,8 @@ static int settle_zeta(kh_run *r) {
 int kh_set_fluid(kh_run *r, const double *z0, const double *z1, const double uk_dc[3]) {
     if (!r || !z0 || !z1 || !uk_dc) return fail(KH_ERR_ARG, "NULL argument");
     r->zeta_lazy = 0;  // every mode is overwritten
-    KH_TRY(upload_spec(r, r->zeta[0], z0));
-    KH_TRY(upload_spec(r, r->zeta[1], z1));
+    const RowField f[2] = {spec_rows(r, r->zeta[0], z0), spec_rows(r, r->zeta[1], z1)};
+    KH_TRY(move(r, f, 2, false));
     r->zeta_dirty = 1;
     KH_HIP(hipMemcpy(r->ukdc, uk_dc, 3 * sizeof(double), hipMemcpyHostToDevice));
     return KH_OK;
@@ -1719,8 +1685,8 @@ int kh_set_fluid(kh_run *r, const double *z0, const double *z1, const double uk_
 int kh_get_fluid(kh_run *r, double *z0, double *z1, double uk_dc[3]) {
     if (!r || !z0 || !z1 || !uk_dc) return fail(KH_ERR_ARG, "NULL argument");
     KH_TRY(settle_zeta(r));
-    KH_TRY(download_spec(r, z0, r->zeta[0]));
-    KH_TRY(download_spec(r, z1, r->zeta[1]));
+    const RowField f[2] = {spec_rows(r, r->zeta[0], z0), spec_rows(r, r->zeta[1], z1)};
+    KH_TRY(move(r, f, 2, true));
     KH_HIP(hipMemcpy(uk_dc, r->ukdc, 3 * sizeof(double), hipMemcpyDeviceToHost));
     return KH_OK;
 }
