@@ -9,8 +9,7 @@ bool fft_length_supported(int L);
 
 // Single passes (each one kernel launch).
 template <typename T>
-// kzvalid >= 0: only kz < kzvalid is written (the wavefront engine; other
-// lengths write every kz)
+// kzvalid >= 0: only kz < kzvalid is written
 hipError_t fft_z_r2c(const Grid &g, const T *in, cpx<T> *out, hipStream_t s, int kzvalid = -1);
 // kzvalid >= 0: modes kz >= kzvalid are taken as zero (not read)
 template <typename T>
@@ -22,7 +21,7 @@ struct ZIO {
     T            *out[5];
 };
 template <typename T>
-// mask: see zw_c2r (ignored by the LDS engine, which writes every point)
+// mask: see zw_c2r
 hipError_t fft_z_c2r_multi(const Grid &g, const ZIO<T> &io, int ncomp, hipStream_t s, int kzvalid = -1,
                            const T *mask = nullptr, Occ occ = {});
 template <typename T, bool FWD>

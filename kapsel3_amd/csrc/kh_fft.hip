@@ -10,9 +10,9 @@
 // Forward = z-pass (two real rows packed into one complex row, r2c), then
 // in-place complex passes along y and along x. Inverse = x, y, then z c2r,
 // with the 1/(NX NY NZ) normalisation folded into the last pass. Every pass
-// reads and writes each field element once, staging a tile in LDS:
-//   z pass : a contiguous block of rows (fully coalesced both ways)
-//   y/x    : a tile of C neighbouring columns (C*elem = 128 B per row)
+// reads and writes each field element once: the z passes on the
+// wavefront-scope engine (kh_zwave.hip), the y and x passes a tile of C
+// neighbouring columns (C*elem = 128 B per row) staged in LDS.
 #include "kh_fft.h"
 #include "kh_fft_engine.h"
 #include "kh_zwave.h"
@@ -24,112 +24,12 @@ template <typename T>
 struct FftTile;
 template <>
 struct FftTile<double> {
-    static constexpr int C     = 8;     // columns per y/x tile (128 B rows)
-    static constexpr int ZELEM = 2048;  // complex points per z-pass block
+    static constexpr int C = 8;  // columns per y/x tile (128 B rows)
 };
 template <>
 struct FftTile<float> {
-    static constexpr int C     = 16;
-    static constexpr int ZELEM = 4096;
+    static constexpr int C = 16;
 };
-
-// ---------------------------------------------------------------- z pass
-// Block of 2P consecutive real rows = P complex lines (rows 2p and 2p+1 are
-// the real and imaginary parts of line p).
-template <typename T, int L>
-struct ZPass {
-    static constexpr int NT  = PassThreads<T>::value;
-    static constexpr int P   = (FftTile<T>::ZELEM / L) > 0 ? FftTile<T>::ZELEM / L : 1;
-    static constexpr int NZH = L / 2 + 1;
-    static constexpr int BS  = ColStride<T, P>::value;
-    static constexpr int SZ  = (L * BS > P * (L + 2)) ? L * BS : P * (L + 2);  // FFT tile or staged rows
-    static constexpr int NR  = (2 * P * L + NT - 1) / NT;                     // real points per thread
-    static constexpr int NC  = (P * L + NT - 1) / NT;                         // complex points per thread
-};
-
-template <typename T, int L>
-__global__ __launch_bounds__(PassThreads<T>::value) void k_fft_z_r2c(const T *__restrict__ in,
-                                                                     cpx<T> *__restrict__ out, long long nrows,
-                                                                     int pitch) {
-    using Z = ZPass<T, L>;
-    constexpr int NT = Z::NT, P = Z::P, NZH = Z::NZH, BS = Z::BS;
-    __shared__ cpx<T> s[Z::SZ], tw[L];
-    fill_twiddles<T, L, NT>(tw);
-    const long long row0 = (long long)blockIdx.x * (2 * P);
-    const T        *src  = in + row0 * L;
-    T               v[Z::NR];
-#pragma unroll
-    for (int i = 0; i < Z::NR; i++) {
-        const int e = threadIdx.x + i * NT;
-        v[i]        = (e < 2 * P * L && row0 + e / L < nrows) ? src[e] : (T)0;
-    }
-#pragma unroll
-    for (int i = 0; i < Z::NR; i++) {
-        const int e = threadIdx.x + i * NT;
-        if (e < 2 * P * L) {
-            const int rl = e / L, n = e - rl * L;
-            reinterpret_cast<T *>(&s[n * BS + (rl >> 1)])[rl & 1] = v[i];
-        }
-    }
-    __syncthreads();
-    fft_cols_ip<T, L, P, BS, NT, true>(s, tw);
-    cpx<T> *dst = out + row0 * pitch;
-    for (int e = threadIdx.x; e < 2 * P * NZH; e += NT) {
-        const int rl = e / NZH, k = e - rl * NZH;
-        if (row0 + rl >= nrows) break;
-        const int    p  = rl >> 1;
-        const cpx<T> Zk = s[k * BS + p];
-        const cpx<T> Zm = cconj(s[((L - k) % L) * BS + p]);
-        cpx<T>       o;
-        if (rl & 1) {  // -i/2 (Z - Zm)
-            const cpx<T> d = csub(Zk, Zm);
-            o              = cmk(d.y * (T)0.5, -d.x * (T)0.5);
-        } else {
-            o = cscale(cadd(Zk, Zm), (T)0.5);
-        }
-        dst[rl * pitch + k] = o;
-    }
-}
-
-template <typename T, int L>
-__global__ __launch_bounds__(PassThreads<T>::value) void k_fft_z_c2r(ZIO<T> io, long long nrows, T scale,
-                                                                     int kzvalid, int pitch, Grid bg) {
-    if (batch_skip(bg)) return;
-    const cpx<T> *__restrict__ in  = brun(io.in[blockIdx.y], bg);  // one component per grid row
-    T *__restrict__            out = brun(io.out[blockIdx.y], bg);
-    using Z = ZPass<T, L>;
-    constexpr int NT = Z::NT, P = Z::P, NZH = Z::NZH, BS = Z::BS;
-    __shared__ cpx<T> s[Z::SZ], tw[L];
-    fill_twiddles<T, L, NT>(tw);
-    const long long row0 = (long long)blockIdx.x * (2 * P);
-    const cpx<T>   *src  = in + row0 * pitch;
-    for (int e = threadIdx.x; e < 2 * P * NZH; e += NT) {  // modes kz >= kzvalid are zero
-        const int rl = e / NZH, k = e - rl * NZH;
-        s[e]         = (row0 + rl < nrows && k < kzvalid) ? src[rl * pitch + k] : cmk((T)0, (T)0);
-    }
-    __syncthreads();
-    cpx<T> zv[Z::NC];
-#pragma unroll
-    for (int i = 0; i < Z::NC; i++) {
-        const int e = threadIdx.x + i * NT;
-        if (e < P * L) zv[i] = hermitian_pair<T, L>(s, e / L, e % L);
-    }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < Z::NC; i++) {
-        const int e = threadIdx.x + i * NT;
-        if (e < P * L) s[(e % L) * BS + e / L] = zv[i];
-    }
-    __syncthreads();
-    fft_cols_ip<T, L, P, BS, NT, false>(s, tw);
-    T *dst = out + row0 * L;
-    for (int e = threadIdx.x; e < 2 * P * L; e += NT) {
-        const int rl = e / L, n = e - rl * L;
-        if (row0 + rl >= nrows) break;
-        const cpx<T> z = s[n * BS + (rl >> 1)];
-        dst[e]         = ((rl & 1) ? z.y : z.x) * scale;
-    }
-}
 
 // ------------------------------------------------------------ y / x pass
 // Lines of L points at stride `lstride`; a tile is C consecutive columns.
@@ -182,39 +82,6 @@ bool fft_length_supported(int L) {
     }
 }
 
-template <typename T>
-static hipError_t launch_z_r2c(int L, const T *in, cpx<T> *out, long long nrows, int pitch, hipStream_t s) {
-    switch (L) {
-#define KH_CASE(n)                                                                       \
-    case n: {                                                                            \
-        constexpr int P  = ZPass<T, n>::P;                                               \
-        long long     nb = (nrows + 2 * P - 1) / (2 * P);                                \
-        hipLaunchKernelGGL((k_fft_z_r2c<T, n>), dim3((unsigned)nb), dim3(ZPass<T, n>::NT), 0, s, in, out, nrows, pitch); \
-        return hipGetLastError();                                                        \
-    }
-        KH_FOR_EACH_L(KH_CASE)
-#undef KH_CASE
-        default: return hipErrorInvalidValue;
-    }
-}
-
-template <typename T>
-static hipError_t launch_z_c2r(int L, const ZIO<T> &io, int ncomp, long long nrows, T scale, int kzvalid,
-                               int pitch, hipStream_t s, const Grid &bg) {
-    switch (L) {
-#define KH_CASE(n)                                                                       \
-    case n: {                                                                            \
-        constexpr int P  = ZPass<T, n>::P;                                               \
-        long long     nb = (nrows + 2 * P - 1) / (2 * P);                                \
-        hipLaunchKernelGGL((k_fft_z_c2r<T, n>), dim3((unsigned)nb, ncomp, batch_z(bg)), dim3(ZPass<T, n>::NT), 0, s, io, nrows, scale, kzvalid, pitch, bg); \
-        return hipGetLastError();                                                        \
-    }
-        KH_FOR_EACH_L(KH_CASE)
-#undef KH_CASE
-        default: return hipErrorInvalidValue;
-    }
-}
-
 template <typename T, bool FWD>
 static hipError_t launch_strided(int L, cpx<T> *data, long long lstride, int ncols, long long ostride, int nouter,
                                  hipStream_t s) {
@@ -235,8 +102,7 @@ static hipError_t launch_strided(int L, cpx<T> *data, long long lstride, int nco
 
 template <typename T>
 hipError_t fft_z_r2c(const Grid &g, const T *in, cpx<T> *out, hipStream_t s, int kzvalid) {
-    if (zw_supported(g.nz)) return zw_r2c<T>(g.nz, in, out, (long long)g.nx * g.ny, g.nzp, s, kzvalid);
-    return launch_z_r2c<T>(g.nz, in, out, (long long)g.nx * g.ny, g.nzp, s);
+    return zw_r2c<T>(g.nz, in, out, (long long)g.nx * g.ny, g.nzp, s, kzvalid);
 }
 template <typename T>
 hipError_t fft_z_c2r(const Grid &g, const cpx<T> *in, T *out, hipStream_t s, int kzvalid) {
@@ -250,10 +116,7 @@ hipError_t fft_z_c2r_multi(const Grid &g, const ZIO<T> &io, int ncomp, hipStream
                            Occ occ) {
     const T   scale = (T)(1.0 / ((double)g.nx * (double)g.ny * (double)g.nz));
     const int kzv   = kzvalid < 0 ? g.nzh : kzvalid;
-    if (zw_supported(g.nz))
-        return zw_c2r<T>(g.nz, io, ncomp, (long long)g.nx * g.ny, scale, kzv, g.nzp, s, mask, nullptr, &g, occ);
-    if (occ.w) return hipErrorInvalidValue;
-    return launch_z_c2r<T>(g.nz, io, ncomp, (long long)g.nx * g.ny, scale, kzv, g.nzp, s, g);
+    return zw_c2r<T>(g.nz, io, ncomp, (long long)g.nx * g.ny, scale, kzv, g.nzp, s, mask, nullptr, &g, occ);
 }
 // y: lines along y at stride nzp, columns kz < nzh, one outer block per x
 template <typename T, bool FWD>

@@ -11,7 +11,7 @@
 //   z passes : read/write only kz < TRN_Z
 // Pointwise work between two passes on the same axis is fused into one
 // kernel: the real-space quadratic products sit between the inverse and the
-// forward z pass (k_z_adv), the construction of u_hat from zeta sits in
+// forward z pass (k_zw_adv), the construction of u_hat from zeta sits in
 // front of the inverse x pass (k_x_zeta2u_inv), and the projection, the
 // addition of u* and the curl sit behind the forward x pass (k_x_f_zeta).
 #include "kh_fft_engine.h"
@@ -46,18 +46,6 @@ struct XZTile {
     static constexpr int C  = sizeof(T) == 4 ? 8 : XTile<T>::C;
     static constexpr int NT = sizeof(T) == 4 ? 256 : XTile<T>::NT;
 };
-
-template <typename T>
-struct ZTile;
-template <>
-struct ZTile<double> {
-    static constexpr int ELEM = 2048;  // complex points per z block
-};
-template <>
-struct ZTile<float> {
-    static constexpr int ELEM = 2048;
-};
-
 
 // ------------------------------------------------------------------------
 // Column passes. Y mode: outer block = x, line along y, columns kz < ncols.
@@ -230,172 +218,6 @@ __global__ __launch_bounds__(XZTile<T>::NT) void k_x_zeta2u_inv(
             const int e = threadIdx.x + i * NT;
             const int n = e / C, c = e - n * C;
             if (e < C * L && kz0 + c < g.trn_z) out[d][base + n * lstride + c] = s[n * BS + c];
-        }
-        __syncthreads();
-    }
-}
-
-// ------------------------------------------------------------------------
-// z pass of the advection term: three half-spectrum rows per (x,y) (kz <
-// TRN_Z nonzero) -> inverse z -> u in registers -> the five products of
-// U2advection_k (operate_omega.cxx:31-47) -> forward z -> five half spectra
-// (kz < TRN_Z written). Two real rows share one complex line.
-template <typename T, int L>
-__global__ __launch_bounds__(PassThreads<T>::value) void k_z_adv(
-    Grid g, const cpx<T> *__restrict__ s0g, const cpx<T> *__restrict__ s1g, const cpx<T> *__restrict__ s2g,
-    cpx<T> *__restrict__ p0, cpx<T> *__restrict__ p1, cpx<T> *__restrict__ p2, cpx<T> *__restrict__ p3,
-    cpx<T> *__restrict__ p4, T scale) {
-    if (batch_skip(g)) return;
-    s0g = brun(s0g, g), s1g = brun(s1g, g), s2g = brun(s2g, g);
-    p0 = brun(p0, g), p1 = brun(p1, g), p2 = brun(p2, g), p3 = brun(p3, g), p4 = brun(p4, g);
-    constexpr int NT  = PassThreads<T>::value;
-    constexpr int P   = (ZTile<T>::ELEM / L) > 0 ? ZTile<T>::ELEM / L : 1;
-    constexpr int NZH = L / 2 + 1;
-    constexpr int NPT = (P * L + NT - 1) / NT;
-    constexpr int BS  = ColStride<T, P>::value;
-    constexpr int SZ  = (L * BS > P * (L + 2)) ? L * BS : P * (L + 2);
-    __shared__ cpx<T> s[SZ], tw[L];
-    fill_twiddles<T, L, NT>(tw);
-    const long long nrows  = (long long)g.nx * g.ny;
-    const long long row0   = (long long)blockIdx.x * (2 * P);
-    const int       kzv    = g.trn_z;
-    const cpx<T>   *src[3] = {s0g, s1g, s2g};
-    cpx<T>          U[3][NPT];  // (row 2p, row 2p+1) of component d at z = n, point e = p*L + n
-    for (int d = 0; d < 3; d++) {
-        for (int e = threadIdx.x; e < 2 * P * NZH; e += NT) {
-            const int rl = e / NZH, k = e - rl * NZH;
-            s[e]         = (row0 + rl < nrows && k < kzv) ? src[d][(row0 + rl) * g.nzp + k] : cmk((T)0, (T)0);
-        }
-        __syncthreads();
-        cpx<T> zv[NPT];
-#pragma unroll
-        for (int i = 0; i < NPT; i++) {
-            const int e = threadIdx.x + i * NT;
-            if (e < P * L) zv[i] = hermitian_pair<T, L>(s, e / L, e % L);
-        }
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < NPT; i++) {
-            const int e = threadIdx.x + i * NT;
-            if (e < P * L) s[(e % L) * BS + e / L] = zv[i];
-        }
-        __syncthreads();
-        fft_cols_ip<T, L, P, BS, NT, false>(s, tw);
-#pragma unroll
-        for (int i = 0; i < NPT; i++) {
-            const int e = threadIdx.x + i * NT;
-            U[d][i]     = (e < P * L) ? cscale(s[(e % L) * BS + e / L], scale) : cmk((T)0, (T)0);
-        }
-        __syncthreads();
-    }
-    cpx<T> *dst[5] = {p0, p1, p2, p3, p4};
-    for (int q = 0; q < 5; q++) {
-#pragma unroll
-        for (int i = 0; i < NPT; i++) {
-            const int e = threadIdx.x + i * NT;
-            if (e >= P * L) continue;
-            cpx<T> v;
-            // .x = row 2p, .y = row 2p+1
-            const cpx<T> u1 = U[0][i], u2 = U[1][i], u3 = U[2][i];
-            if (q == 0)
-                v = cmk(u2.x * u3.x, u2.y * u3.y);
-            else if (q == 1)
-                v = cmk(u3.x * u1.x, u3.y * u1.y);
-            else if (q == 2)
-                v = cmk(u1.x * u2.x, u1.y * u2.y);
-            else if (q == 3)
-                v = cmk((u2.x - u3.x) * (u2.x + u3.x), (u2.y - u3.y) * (u2.y + u3.y));
-            else
-                v = cmk((u3.x - u1.x) * (u3.x + u1.x), (u3.y - u1.y) * (u3.y + u1.y));
-            s[(e % L) * BS + e / L] = v;
-        }
-        __syncthreads();
-        fft_cols_ip<T, L, P, BS, NT, true>(s, tw);
-        for (int e = threadIdx.x; e < 2 * P * NZH; e += NT) {
-            const int rl = e / NZH, k = e - rl * NZH;
-            if (row0 + rl >= nrows) break;
-            if (k >= kzv) continue;
-            const int    p  = rl >> 1;
-            const cpx<T> Zk = s[k * BS + p];
-            const cpx<T> Zm = cconj(s[((L - k) % L) * BS + p]);
-            cpx<T>       v;
-            if (rl & 1) {
-                const cpx<T> d = csub(Zk, Zm);
-                v              = cmk(d.y * (T)0.5, -d.x * (T)0.5);
-            } else {
-                v = cscale(cadd(Zk, Zm), (T)0.5);
-            }
-            dst[q][(row0 + rl) * g.nzp + k] = v;
-        }
-        __syncthreads();
-    }
-}
-
-// ------------------------------------------------------------------------
-// z pass of the rigidity force: f = up - min(phi_sum, 1) u*
-// (Make_f_particle_dt_nonsole, f_particle.h:35-54; make_phi.cxx:248-259),
-// forward z per component, kz < TRN_Z written.
-template <typename T, int L>
-__global__ __launch_bounds__(PassThreads<T>::value) void k_z_force(
-    Grid g, const T *__restrict__ up0, const T *__restrict__ up1, const T *__restrict__ up2,
-    const T *__restrict__ phis, const T *__restrict__ us0, const T *__restrict__ us1, const T *__restrict__ us2,
-    cpx<T> *__restrict__ f0, cpx<T> *__restrict__ f1, cpx<T> *__restrict__ f2) {
-    if (batch_skip(g)) return;
-    up0 = brun(up0, g), up1 = brun(up1, g), up2 = brun(up2, g), phis = brun(phis, g);
-    us0 = brun(us0, g), us1 = brun(us1, g), us2 = brun(us2, g);
-    f0 = brun(f0, g), f1 = brun(f1, g), f2 = brun(f2, g);
-    constexpr int NT  = PassThreads<T>::value;
-    constexpr int P   = (ZTile<T>::ELEM / L) > 0 ? ZTile<T>::ELEM / L : 1;
-    constexpr int NZH = L / 2 + 1;
-    constexpr int NR  = (2 * P * L + NT - 1) / NT;  // real points per thread
-    constexpr int BS  = ColStride<T, P>::value;
-    __shared__ cpx<T> s[L * BS], tw[L];
-    fill_twiddles<T, L, NT>(tw);
-    const long long nrows = (long long)g.nx * g.ny;
-    const long long row0  = (long long)blockIdx.x * (2 * P);
-    const T        *UP[3] = {up0, up1, up2}, *US[3] = {us0, us1, us2};
-    cpx<T>         *dst[3] = {f0, f1, f2};
-    // real point e = rl*L + n of the block (contiguous rows)
-    T ph[NR];
-#pragma unroll
-    for (int i = 0; i < NR; i++) {
-        const int e = threadIdx.x + i * NT;
-        ph[i]       = (e < 2 * P * L && row0 + e / L < nrows) ? fmin(phis[row0 * L + e], (T)1) : (T)0;
-    }
-    for (int d = 0; d < 3; d++) {
-        T a[NR], b[NR];
-#pragma unroll
-        for (int i = 0; i < NR; i++) {
-            const int  e  = threadIdx.x + i * NT;
-            const bool ok = e < 2 * P * L && row0 + e / L < nrows;
-            a[i]          = ok ? UP[d][row0 * L + e] : (T)0;
-            b[i]          = ok && US[d] ? US[d][row0 * L + e] : (T)0;
-        }
-#pragma unroll
-        for (int i = 0; i < NR; i++) {
-            const int e = threadIdx.x + i * NT;
-            if (e < 2 * P * L) {
-                const int rl = e / L, n = e - rl * L;
-                reinterpret_cast<T *>(&s[n * BS + (rl >> 1)])[rl & 1] = a[i] - ph[i] * b[i];
-            }
-        }
-        __syncthreads();
-        fft_cols_ip<T, L, P, BS, NT, true>(s, tw);
-        for (int e = threadIdx.x; e < 2 * P * NZH; e += NT) {
-            const int rl = e / NZH, k = e - rl * NZH;
-            if (row0 + rl >= nrows) break;
-            if (k >= g.trn_z) continue;
-            const int    p  = rl >> 1;
-            const cpx<T> Zk = s[k * BS + p];
-            const cpx<T> Zm = cconj(s[((L - k) % L) * BS + p]);
-            cpx<T>       v;
-            if (rl & 1) {
-                const cpx<T> dd = csub(Zk, Zm);
-                v               = cmk(dd.y * (T)0.5, -dd.x * (T)0.5);
-            } else {
-                v = cscale(cadd(Zk, Zm), (T)0.5);
-            }
-            dst[d][(row0 + rl) * g.nzp + k] = v;
         }
         __syncthreads();
     }
@@ -702,22 +524,18 @@ __global__ void k_zeta_clean(Grid g, cpx<T> *__restrict__ z0, cpx<T> *__restrict
 
 // zeta += (a0, a1) and uk_dc += dc: the projected slip field's vorticity
 // and mean velocity, added after the slip iteration.
-// With kept_only, (a0, a1) are read at the 2/3-kept modes only (they hold
-// nothing else).
+// (a0, a1) hold the 2/3-kept modes only.
 template <typename T>
 __global__ void k_zeta_add(Grid g, cpx<T> *__restrict__ z0, cpx<T> *__restrict__ z1, const cpx<T> *__restrict__ a0,
-                           const cpx<T> *__restrict__ a1, double *__restrict__ ukdc, const double *__restrict__ dc,
-                           int kept_only) {
+                           const cpx<T> *__restrict__ a1, double *__restrict__ ukdc, const double *__restrict__ dc) {
     const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (idx == 0)
         for (int d = 0; d < 3; d++) ukdc[d] += dc[d];
-    if (idx >= g.nspec || (int)(idx % g.nzp) >= g.nzh) return;
-    if (kept_only) {
-        const int       kz   = (int)(idx % g.nzp);
-        const long long rest = idx / g.nzp;
-        const int       j = (int)(rest % g.ny), i = (int)(rest / g.ny);
-        if (!kept_mode(g, kx_of(g, i), ky_of(g, j), kz)) return;
-    }
+    if (idx >= g.nspec) return;
+    const int       kz   = (int)(idx % g.nzp);
+    const long long rest = idx / g.nzp;
+    const int       j = (int)(rest % g.ny), i = (int)(rest / g.ny);
+    if (!kept_mode(g, kx_of(g, i), ky_of(g, j), kz)) return;
     z0[idx] = cadd(z0[idx], a0[idx]);
     z1[idx] = cadd(z1[idx], a1[idx]);
 }
@@ -779,45 +597,14 @@ hipError_t x_zeta2u_inv(const Grid &g, const cpx<T> *z0, const cpx<T> *z1, cpx<T
 
 template <typename T>
 hipError_t z_adv(const Grid &g, cpx<T> *const s3[3], cpx<T> *const p5[5], hipStream_t s) {
-    const long long nrows = (long long)g.nx * g.ny;
-    const T         scale = (T)(1.0 / ((double)g.nx * (double)g.ny * (double)g.nz));
-    if (zw_supported(g.nz)) return zw_adv<T>(g, s3, p5, scale, s);
-    switch (g.nz) {
-#define KH_CASE(n)                                                                                                 \
-    case n: {                                                                                                      \
-        constexpr int P = (ZTile<T>::ELEM / n) > 0 ? ZTile<T>::ELEM / n : 1;                                       \
-        hipLaunchKernelGGL((k_z_adv<T, n>), dim3((unsigned)((nrows + 2 * P - 1) / (2 * P)), 1, batch_z(g)), dim3(PassThreads<T>::value), 0, s, g, \
-                           s3[0], s3[1], s3[2], p5[0], p5[1], p5[2], p5[3], p5[4], scale);                         \
-        return hipGetLastError();                                                                                  \
-    }
-        KH_FOR_EACH_L(KH_CASE)
-#undef KH_CASE
-        default: return hipErrorInvalidValue;
-    }
+    const T scale = (T)(1.0 / ((double)g.nx * (double)g.ny * (double)g.nz));
+    return zw_adv<T>(g, s3, p5, scale, s);
 }
-
-bool z_force_clears(const Grid &g) { return zw_supported(g.nz); }
 
 template <typename T>
 hipError_t z_force(const Grid &g, T *const up[3], T *phis, T *const us[3], cpx<T> *const f[3], int clear,
                    int *tick, hipStream_t s, T *const us2[3], const int *skip, Occ occ) {
-    const long long nrows = (long long)g.nx * g.ny;
-    if (zw_supported(g.nz)) return zw_force<T>(g, up, phis, us, f, clear, tick, s, us2, skip, occ);
-    if (clear || tick || us2 || skip || occ.w) return hipErrorInvalidValue;
-    T *const none[3] = {nullptr, nullptr, nullptr};
-    if (!us) us = none;
-    switch (g.nz) {
-#define KH_CASE(n)                                                                                                   \
-    case n: {                                                                                                        \
-        constexpr int P = (ZTile<T>::ELEM / n) > 0 ? ZTile<T>::ELEM / n : 1;                                         \
-        hipLaunchKernelGGL((k_z_force<T, n>), dim3((unsigned)((nrows + 2 * P - 1) / (2 * P)), 1, batch_z(g)), dim3(PassThreads<T>::value), 0, s, g, \
-                           up[0], up[1], up[2], phis, us[0], us[1], us[2], f[0], f[1], f[2]);                        \
-        return hipGetLastError();                                                                                    \
-    }
-        KH_FOR_EACH_L(KH_CASE)
-#undef KH_CASE
-        default: return hipErrorInvalidValue;
-    }
+    return zw_force<T>(g, up, phis, us, f, clear, tick, s, us2, skip, occ);
 }
 
 template <typename T>
@@ -872,9 +659,9 @@ hipError_t x_slip(const Grid &g, cpx<T> *const f[3], cpx<T> *a0, cpx<T> *a1, dou
 
 template <typename T>
 hipError_t zeta_add(const Grid &g, cpx<T> *z0, cpx<T> *z1, const cpx<T> *a0, const cpx<T> *a1, double *ukdc,
-                    const double *dc, hipStream_t s, int kept_only) {
+                    const double *dc, hipStream_t s) {
     hipLaunchKernelGGL(k_zeta_add<T>, dim3((unsigned)((g.nspec + 255) / 256)), dim3(256), 0, s, g, z0, z1, a0, a1, ukdc,
-                       dc, kept_only);
+                       dc);
     return hipGetLastError();
 }
 
@@ -900,7 +687,7 @@ hipError_t zeta_clean(const Grid &g, cpx<T> *z0, cpx<T> *z1, hipStream_t s) {
     template hipError_t x_adv_ns<T>(const Grid &, const Comps<T> &, cpx<T> *, cpx<T> *, double, double, hipStream_t); \
     template hipError_t zeta_clean<T>(const Grid &, cpx<T> *, cpx<T> *, hipStream_t);                               \
     template hipError_t zeta_add<T>(const Grid &, cpx<T> *, cpx<T> *, const cpx<T> *, const cpx<T> *, double *,      \
-                                    const double *, hipStream_t, int);
+                                    const double *, hipStream_t);
 KH_INST(double)
 KH_INST(float)
 #undef KH_INST

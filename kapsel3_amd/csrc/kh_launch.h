@@ -26,7 +26,7 @@ hipError_t f_nonsole(long long n, T *const up[3], const T *phisum, T *const u[3]
 template <typename T>
 hipError_t add3(long long n, T *const u[3], T *const f[3], hipStream_t s);
 template <typename T>
-hipError_t fill(long long n, T *p, T v, hipStream_t s, const Grid *batch = nullptr);
+hipError_t fill(long long n, T *p, T v, hipStream_t s);
 
 // kh_shear.hip (the Lees-Edwards step; gd = strain of the oblique grid)
 template <typename T>
@@ -34,8 +34,6 @@ hipError_t obl_zeta_to_u(const Grid &g, cpx<T> *z0, cpx<T> *z1, cpx<T> *u0, cpx<
                          double *ukdc, int fixmask, int truncate, double gd, hipStream_t s);
 template <typename T>
 hipError_t obl_zeta_to_omega(const Grid &g, const cpx<T> *z0, const cpx<T> *z1, cpx<T> *const o[3], hipStream_t s);
-template <typename T>
-hipError_t obl_cross(long long n, T *const u[3], T *const w[3], hipStream_t s);
 template <typename T>
 hipError_t obl_adv_ns(const Grid &g, cpx<T> *const F[3], const cpx<T> *w1, cpx<T> *z0, cpx<T> *z1, double rate,
                       double gd, double dmy0, double dmy1, hipStream_t s);
@@ -79,7 +77,7 @@ hipError_t velocity(const PParams &pp, DevParticle *P, int ab2, double h, hipStr
                     double nio = 0.0);
 hipError_t thermostat(const PParams &pp, DevParticle *P, uint64_t seed, uint32_t stream, const int *d_ts, double niv,
                       double nio, hipStream_t s);
-hipError_t tick(int *d_ts, hipStream_t s, const Grid *batch = nullptr);
+hipError_t tick(int *d_ts, hipStream_t s);
 // the sheared step's stress record from the per-particle partials and the
 // nacc Reynolds partials of k_obl_to_cart
 hipError_t obl_record(const PParams &pp, const double *acc, long long nacc, const ShearRec &h, double *last,

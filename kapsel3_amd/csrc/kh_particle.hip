@@ -1498,13 +1498,11 @@ hipError_t rigid_velocity(const PParams &pp, DevParticle *P, const RigidArgs &ra
 }
 
 // jikan.ts += 1 on the device (the step counter the noise stream is keyed by)
-__global__ void k_tick(int *__restrict__ d_ts, Grid bg) {
-    if (batch_skip(bg)) return;
-    if (threadIdx.x == 0 && blockIdx.x == 0) *brun(d_ts, bg) += 1;
+__global__ void k_tick(int *__restrict__ d_ts) {
+    if (threadIdx.x == 0) *d_ts += 1;
 }
-hipError_t tick(int *d_ts, hipStream_t s, const Grid *batch) {
-    const Grid bg = batch ? *batch : Grid{};
-    hipLaunchKernelGGL(k_tick, dim3(1, 1, batch_z(bg)), dim3(64), 0, s, d_ts, bg);
+hipError_t tick(int *d_ts, hipStream_t s) {
+    hipLaunchKernelGGL(k_tick, dim3(1), dim3(64), 0, s, d_ts);
     return hipGetLastError();
 }
 

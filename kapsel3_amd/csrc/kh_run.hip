@@ -116,15 +116,13 @@ struct kh_run {
     int         *d_ts         = nullptr;  // jikan.ts on the device (noise counter)
     double      *slipeps      = nullptr;  // slip convergence measure (1 double)
     double      *xs           = nullptr;  // compact particle positions (np x 4)
-    bool         zclear       = false;    // the fused step's z_force leaves u_p and phi_sum zero
-    bool         pclean       = false;    // u_p and phi_sum are zero now
+    bool         pclean       = false;    // u_p and phi_sum are zero now (the fused step's z_force leaves them so)
     double      *slipdc       = nullptr;  // k = 0 mode of the projected slip field (3 doubles)
     int          slip_iters   = 0;        // iterations of the last slip loop decided on the host
     long long    slip_iters_host = 0, slip_loops_host = 0;  // totals of the loops decided on the host
-    // the fused step's slip loop decided on the device (power-of-two NZ >= 32):
+    // the fused step's slip loop is decided on the device:
     // int flag[2] (converged, iterations this step), then unsigned long long
     // stat[2] (total iterations, loops) at byte 16
-    bool         slip_dev     = false;
     int         *slipflag     = nullptr;
     double      *traj         = nullptr;  // per-step particle record (x, v) for traj_steps steps
     int          traj_steps   = 0;
@@ -250,6 +248,8 @@ struct Timed {
         KH_HIP(call);                \
     } while (0)
 
+void drop_graph(kh_run *r);
+
 // ------------------------------------------------------------ the step
 // the run's occupancy bits of the 4-point z vectors
 static inline Occ occ_of(const kh_run *r) { return Occ{(unsigned long long *)r->occ, r->occw}; }
@@ -280,7 +280,7 @@ struct Step {
     // the mask reads they save (a 4-point vector is 16 bytes there, and
     // z_force's clearing stores into lines it has not read are slower).
     static bool occ_on(const kh_run *r) {
-        return occ_kept<T>() && r->zclear && !r->slip && !r->rigid && !r->pp.obl;
+        return occ_kept<T>() && !r->slip && !r->rigid && !r->pp.obl;
     }
     static int zero(kh_run *r, T *p) {
         KH_LAUNCH("fill", (fill<T>(r->g.nreal, p, (T)0, r->stream)));
@@ -408,10 +408,8 @@ struct Step {
     // The slip iteration of Time_evolution_hydro (sp_3d_ns.cxx:121-161):
     // Make_particle_momentum_factor, then until converged (or slip_iter_max)
     // slip scatter -> Solenoidal_u -> Calc_f_slip -> up += u -> (first pass:
-    // LJ + gravity) -> velocity with the slip force; finally u := up. In the
-    // fused step zeta also takes the curl of the projected slip field (its
-    // u_hat is rebuilt from zeta later), and uk_dc its k = 0 mode.
-    static int slip_iteration(kh_run *r, int ab2, bool fused) {
+    // LJ + gravity) -> velocity with the slip force; finally u := up.
+    static int slip_iteration(kh_run *r, int ab2) {
         T *u[3] = {U(r, 0), U(r, 1), U(r, 2)}, *up[3] = {UP(r, 0), UP(r, 1), UP(r, 2)};
         KH_LAUNCH("slip_moments", slip_moments<T>(r->pp, r->dp, u, r->stream));
         KH_LAUNCH("slip_update", slip_update(r->pp, r->dp, 0, 0, r->stream));
@@ -423,9 +421,6 @@ struct Step {
             KH_LAUNCH("slip_scatter", slip_scatter<T>(r->pp, r->dp, u, up, r->stream));
             for (int d = 0; d < 3; d++) KH_TRY(r2c(r, up[d], S(r, d)));
             KH_LAUNCH("solenoidal", (solenoidal<T>(r->g, S(r, 0), S(r, 1), S(r, 2), r->stream)));
-            if (fused)
-                KH_LAUNCH("slip_zeta", (u_to_zeta<T>(r->g, S(r, 0), S(r, 1), S(r, 2), S(r, 3), S(r, 4), r->slipdc,
-                                                     r->stream)));
             for (int d = 0; d < 3; d++) KH_TRY(c2r(r, S(r, d), up[d]));
             KH_LAUNCH("f_slip", f_slip<T>(r->pp, r->dp, up, coef, r->stream));
             KH_LAUNCH("add3", (add3<T>(r->g.nreal, up, u, r->stream)));
@@ -446,9 +441,7 @@ struct Step {
         r->slip_iters_host += iter;
         r->slip_loops_host++;
         for (int d = 0; d < 3; d++) std::swap(r->ureal[d], r->up[d]);  // Swap_mem(u, up)
-        if (fused)
-            KH_LAUNCH("zeta_add", (zeta_add<T>(r->g, Z(r, 0), Z(r, 1), S(r, 3), S(r, 4), r->ukdc, r->slipdc,
-                                               r->stream)));
+        drop_graph(r);  // captured steps hold the buffers as they were
         return KH_OK;
     }
 
@@ -497,7 +490,7 @@ struct Step {
                 KH_LAUNCH("slip_update", slip_update(r->pp, r->dp, iter + 1, 1, s, skip));
         }
         KH_LAUNCH("reset_forces", reset_forces(r->pp, r->dp, s));
-        KH_LAUNCH("zeta_add", (zeta_add<T>(g, Z(r, 0), Z(r, 1), S(r, 3), S(r, 4), r->ukdc, r->slipdc, s, 1)));
+        KH_LAUNCH("zeta_add", (zeta_add<T>(g, Z(r, 0), Z(r, 1), S(r, 3), S(r, 4), r->ukdc, r->slipdc, s)));
         return KH_OK;
     }
 
@@ -540,7 +533,7 @@ struct Step {
     // Reset_phi / Reset_u (the previous fused step's z_force already left
     // u_p and phi_sum zero), then the position update and the phi scatter
     static int particles_begin(kh_run *r, int ab2) {
-        if (!(r->zclear && r->pclean)) {
+        if (!r->pclean) {
             for (int d = 0; d < 3; d++) KH_TRY(zero(r, UP(r, d)));
             KH_TRY(zero(r, PS(r)));
             KH_LAUNCH("fill", (fill<double>((long long)r->occw * r->g.nx * r->g.ny, (double *)r->occ, 0.0, r->stream)));
@@ -592,9 +585,8 @@ struct Step {
         cpx<T>     *s3[3]  = {S(r, 0), S(r, 1), S(r, 2)};
         Comps<T>    c5{{S(r, 0), S(r, 1), S(r, 2), S(r, 3), S(r, 4)}};
         T          *up3[3] = {UP(r, 0), UP(r, 1), UP(r, 2)}, *u3[3] = {U(r, 0), U(r, 1), U(r, 2)};
-        KH_LAUNCH("z_force", (z_force<T>(g, up3, PS(r), up_is_f ? nullptr : u3, s3, r->zclear ? 3 : 0,
-                                         r->zclear ? r->d_ts : nullptr, s, us2, nullptr, occ)));
-        if (!r->zclear) KH_LAUNCH("tick", tick(r->d_ts, s, &g));
+        KH_LAUNCH("z_force", (z_force<T>(g, up3, PS(r), up_is_f ? nullptr : u3, s3, 3, r->d_ts, s, us2, nullptr,
+                                         occ)));
         KH_LAUNCH("y_fwd_force", (cols_y<T, true>(g, c5, 3, 0, 1, s)));
         KH_LAUNCH("x_f_zeta", (x_f_zeta<T>(g, s3, Z(r, 0), Z(r, 1), r->ukdc, s)));
         return KH_OK;
@@ -624,27 +616,18 @@ struct Step {
         // The particles move and scatter phi first (the position update
         // reads only the particle state, so it commutes with the fluid
         // part): phi_sum is then known when u* is formed, and u* is written
-        // only where it is read. Squirmer runs with the slip loop decided on
-        // the host keep the reference's order.
-        const bool early = !r->slip || r->slip_dev;
+        // only where it is read.
         // plain spheres in FP64: the phi scatter marks the 4-point vectors it
         // reaches, and z_c2r and z_force read those bits instead of phi_sum
         const Occ occ = occ_on(r) ? occ_of(r) : Occ{};
         r->pp.occ     = occ;
-        if (early) KH_TRY(particles_begin(r, ab2));
+        KH_TRY(particles_begin(r, ab2));
         // squirmers read u* on the whole slip shell (|r - a| < xi/2), which
         // reaches points where phi has underflowed to 0: u* is written in full
-        KH_TRY(fused_fluid(r, g, early && !r->slip ? PS(r) : nullptr, occ));
-        if (!early) KH_TRY(particles_begin(r, ab2));
-        if (r->slip_dev) {  // the slip loop leaves up zero
+        KH_TRY(fused_fluid(r, g, !r->slip ? PS(r) : nullptr, occ));
+        if (r->slip) {  // the slip loop leaves up zero
             KH_TRY(calc_f_hydro(r));
             KH_TRY(slip_iteration_dev(r, ab2));
-            if (r->kbt > 0.) KH_TRY(thermo(r));
-            KH_TRY(scatter_up(r));
-        } else if (r->slip) {
-            KH_TRY(calc_f_hydro(r));
-            KH_TRY(slip_iteration(r, ab2, true));
-            for (int d = 0; d < 3; d++) KH_TRY(zero(r, UP(r, d)));
             if (r->kbt > 0.) KH_TRY(thermo(r));
             KH_TRY(scatter_up(r));
         } else if (r->rigid) {  // bead F_H, LJ, the bodies' update, u_p from the beads' rigid motion
@@ -655,8 +638,8 @@ struct Step {
             KH_TRY(plain_particles(r, ab2));
         }
         T *w3[3] = {W(r, 0), W(r, 1), W(r, 2)};  // squirmers: u = u* + the projected slip field
-        KH_TRY(fused_force(r, g, r->slip_dev ? w3 : nullptr, !r->slip && !r->rigid, occ));
-        r->pclean = r->zclear;
+        KH_TRY(fused_force(r, g, r->slip ? w3 : nullptr, !r->slip && !r->rigid, occ));
+        r->pclean = true;
         return KH_OK;
     }
 
@@ -674,10 +657,6 @@ struct Step {
         g.bactive     = b->active;
         hipStream_t s = r->stream;
         const SlotPart<T> *sp = (const SlotPart<T> *)b->dslots;
-        if (!r->zclear) {  // Reset_phi / Reset_u
-            for (int d = 0; d < 3; d++) KH_LAUNCH("fill", (fill<T>(g.nreal, UP(r, d), (T)0, s, &g)));
-            KH_LAUNCH("fill", (fill<T>(g.nreal, PS(r), (T)0, s, &g)));
-        }
         KH_LAUNCH("phi_scatter", (phi_scatter_batch<T>(sp, b->active, b->capacity, b->np_cap, r->jikan.dt_md,
                                                        r->jikan.hdt_md, s)));
         const Occ occ = occ_on(r) ? occ_of(r) : Occ{};
@@ -725,7 +704,7 @@ struct Step {
         KH_TRY(make_phi(r));
         KH_TRY(calc_f_hydro(r));
         if (r->slip)
-            KH_TRY(slip_iteration(r, ab2, false));
+            KH_TRY(slip_iteration(r, ab2));
         else
             KH_TRY(velocity_update(r, ab2));
         if (r->kbt > 0.) KH_TRY(thermo(r));
@@ -758,16 +737,10 @@ struct Step {
         return KH_OK;
     }
     // The same inverse transform of omega's three spectra, then u x omega
-    // (contravariant u and omega, covariant product) into out: fused into
-    // the z pass where the wavefront engine has the length, else a separate
-    // pass. u holds the real-space u.
+    // (contravariant u and omega, covariant product) into out, fused into
+    // the z pass. u holds the real-space u.
     static int c2r_kept3_cross(kh_run *r, cpx<T> *const sp[3], T *const u[3], T *const out[3]) {
         const Grid &g = r->g;
-        if (!zw_cross_supported(g.nz)) {
-            KH_TRY(c2r_kept3(r, sp, out));
-            KH_LAUNCH("obl_cross", (obl_cross<T>(g.nreal, u, out, r->stream)));
-            return KH_OK;
-        }
         Comps<T> c{{sp[0], sp[1], sp[2], nullptr, nullptr}};
         KH_LAUNCH("x_inv_kept", (cols_x<T, false>(g, c, 3, 1, 0, r->stream)));
         KH_LAUNCH("y_inv_kept", (cols_y<T, false>(g, c, 3, 1, 0, r->stream)));
@@ -960,7 +933,7 @@ struct Step {
             }
             case KH_FN_SLIP_ITERATION:
                 if (!r->slip) return fail(KH_ERR_STATE, "no slip species in this run");
-                return slip_iteration(r, r->jikan.ts != 0, false);
+                return slip_iteration(r, r->jikan.ts != 0);
             case KH_FN_OBL_NS_SOLVER:
             case KH_FN_OBL_ZETA_K2U:
             case KH_FN_OBL_U2ZETA_K:
@@ -1016,8 +989,6 @@ void *field_buffer(kh_run *r, int field) {
         default: return nullptr;
     }
 }
-
-void drop_graph(kh_run *r);
 
 int free_run(kh_run *r) {
     if (!r) return KH_OK;
@@ -1522,10 +1493,6 @@ int run_create(const kh_params *P, int np, char *arena, size_t arena_bytes, kh_r
         const int nh    = (int)P->a + (int)P->a_xi + 2, nmin = std::min(P->nx, std::min(P->ny, P->nz));
         pp.direct_dist = 2 * (nh + 2) <= nmin;
     }
-    // squirmer steps decide the slip loop on the device where the wavefront
-    // z engine and its masked inverse pass take NZ
-    r->slip_dev        = r->slip && zw_supported(g.nz) && g.nz >= 32;
-    r->zclear          = (!r->slip || r->slip_dev) && z_force_clears(g);
 
     CTime t0  = {0, 0.0, P->dt, P->dt * 0.5, P->dt, P->dt * 0.5};  // sp_3d_ns.cxx:782
     r->jikan  = t0;
@@ -1765,10 +1732,8 @@ int kh_step(kh_run *r, int nsteps) {
     if (nsteps < 0) return fail(KH_ERR_ARG, "negative step count");
     if (!r->shear) KH_TRY(settle_zeta(r));
     for (int s = 0; s < nsteps;) {
-        // (a slip loop decided on the host is not captured)
         const bool graph_ok = r->use_graph && !r->timing && r->step_path == KH_PATH_FUSED && r->jikan.ts > 0 &&
-                              !r->zeta_dirty && (!r->slip || r->slip_dev) && !r->shear &&
-                              (!r->zclear || r->pclean);
+                              !r->zeta_dirty && !r->shear && r->pclean;
         int done = 1;
         if (graph_ok && nsteps - s >= GRAPH_STEPS) {
             if (!r->graph_exec_k) KH_TRY(capture_steps(r, GRAPH_STEPS, &r->graph_k, &r->graph_exec_k));
@@ -2537,7 +2502,7 @@ int batch_step(kh_batch *b, int nsteps) {
         }
         for (kh_run *q : members) {
             q->pcache_valid = 1;
-            q->pclean       = q->zclear;
+            q->pclean       = true;
             for (int k = 0; k < done; k++) {
                 q->jikan.time += q->jikan.dt_fluid;  // sp_3d_ns.cxx:955
                 q->jikan.ts++;

@@ -182,20 +182,6 @@ __global__ __launch_bounds__(SH_NT) void k_obl_zeta_to_omega(Grid g, const cpx<T
     o2[idx] = c;
 }
 
-// u x omega of contravariant u and omega: covariant components
-// (operate_omega.cxx:113-137), in place into w.
-template <typename T>
-__global__ __launch_bounds__(SH_NT) void k_obl_cross(long long n, const T *__restrict__ u0, const T *__restrict__ u1,
-                                                     const T *__restrict__ u2, T *__restrict__ w0,
-                                                     T *__restrict__ w1, T *__restrict__ w2) {
-    const long long i = (long long)blockIdx.x * SH_NT + threadIdx.x;
-    if (i >= n) return;
-    const T a = u0[i], b = u1[i], c = u2[i], x = w0[i], y = w1[i], z = w2[i];
-    w0[i]     = b * z - c * y;
-    w1[i]     = c * x - a * z;
-    w2[i]     = a * y - b * x;
-}
-
 // The spectral end of Zeta_k2advection_k_OBL (operate_omega.cxx:139-154):
 // the shear terms -2 rate u_hat^y (1, g, 0), the curl (U_k2rotation_k,
 // fft_wrapper.cxx:893-935) and Omega_k2zeta_k_OBL (fft_wrapper.cxx:265-289),
@@ -488,11 +474,6 @@ hipError_t obl_zeta_to_omega(const Grid &g, const cpx<T> *z0, const cpx<T> *z1, 
     return hipGetLastError();
 }
 template <typename T>
-hipError_t obl_cross(long long n, T *const u[3], T *const w[3], hipStream_t s) {
-    hipLaunchKernelGGL(k_obl_cross<T>, dim3(sh_blocks(n)), dim3(SH_NT), 0, s, n, u[0], u[1], u[2], w[0], w[1], w[2]);
-    return hipGetLastError();
-}
-template <typename T>
 hipError_t obl_adv_ns(const Grid &g, cpx<T> *const F[3], const cpx<T> *w1, cpx<T> *z0, cpx<T> *z1, double rate,
                       double gd, double dmy0, double dmy1, hipStream_t s) {
     const long long nk = sh_nkept(g);
@@ -534,7 +515,6 @@ hipError_t obl_u_to_zeta(const Grid &g, const cpx<T> *u0, const cpx<T> *u1, cons
                                          double *, int, int, double, hipStream_t);                                   \
     template hipError_t obl_zeta_to_omega<T>(const Grid &, const cpx<T> *, const cpx<T> *, cpx<T> *const[3],         \
                                              hipStream_t);                                                           \
-    template hipError_t obl_cross<T>(long long, T *const[3], T *const[3], hipStream_t);                              \
     template hipError_t obl_adv_ns<T>(const Grid &, cpx<T> *const[3], const cpx<T> *, cpx<T> *, cpx<T> *, double,    \
                                       double, double, double, hipStream_t);                                          \
     template hipError_t obl_remap<T>(const Grid &, T *const[3], T *const[3], double, hipStream_t);                   \

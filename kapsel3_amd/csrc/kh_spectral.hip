@@ -221,9 +221,7 @@ __global__ __launch_bounds__(PW_NT) void k_add3(long long n, T *__restrict__ u0,
 
 // 16-byte stores; fields are hipMalloc'd (256-byte aligned)
 template <typename T>
-__global__ __launch_bounds__(PW_NT) void k_fill(long long n, T *__restrict__ p, T v, Grid bg) {
-    if (batch_skip(bg)) return;
-    p                  = brun(p, bg);
+__global__ __launch_bounds__(PW_NT) void k_fill(long long n, T *__restrict__ p, T v) {
     constexpr int   W  = 16 / sizeof(T);
     const long long i  = ((long long)blockIdx.x * PW_NT + threadIdx.x) * W;
     if (i + W <= n) {
@@ -281,10 +279,9 @@ hipError_t add3(long long n, T *const u[3], T *const f[3], hipStream_t s) {
     return hipGetLastError();
 }
 template <typename T>
-hipError_t fill(long long n, T *p, T v, hipStream_t s, const Grid *batch) {
-    constexpr int W  = 16 / sizeof(T);
-    const Grid    bg = batch ? *batch : Grid{};
-    hipLaunchKernelGGL(k_fill<T>, dim3(nblocks((n + W - 1) / W), 1, batch_z(bg)), dim3(PW_NT), 0, s, n, p, v, bg);
+hipError_t fill(long long n, T *p, T v, hipStream_t s) {
+    constexpr int W = 16 / sizeof(T);
+    hipLaunchKernelGGL(k_fill<T>, dim3(nblocks((n + W - 1) / W)), dim3(PW_NT), 0, s, n, p, v);
     return hipGetLastError();
 }
 
@@ -298,7 +295,7 @@ hipError_t fill(long long n, T *p, T v, hipStream_t s, const Grid *batch) {
                                      cpx<T> *, double *, hipStream_t);                                             \
     template hipError_t f_nonsole<T>(long long, T *const[3], const T *, T *const[3], T *const[3], hipStream_t);    \
     template hipError_t add3<T>(long long, T *const[3], T *const[3], hipStream_t);                                 \
-    template hipError_t fill<T>(long long, T *, T, hipStream_t, const Grid *);
+    template hipError_t fill<T>(long long, T *, T, hipStream_t);
 KH_INST(double)
 KH_INST(float)
 #undef KH_INST

@@ -1,8 +1,8 @@
 // kh_wave_fft.h -- wavefront-scope FFT of whole lines held in registers.
 //
-// A line of L complex points (L a power of two, 8..512) is owned by G = L/E
-// lanes of one wavefront, E points per lane; a 64-lane wavefront holds
-// W = 64/G lines. The transform is a Stockham decomposition L = R_0 R_1 ...
+// A line of L complex points (L a power of two, 8..512, or three times one,
+// 12..384) is owned by G = L/E lanes of one wavefront, E points per lane (G a
+// power of two); a 64-lane wavefront holds W = 64/G lines. The transform is a Stockham decomposition L = R_0 R_1 ...
 // with every radix dividing E: each stage does E/R radix-R butterflies in
 // registers, and the exchange between two stages goes through a per-line
 // LDS strip that only the owning wavefront touches, so no workgroup barrier
@@ -81,17 +81,70 @@ struct Dft<T, 16, FWD> {
     }
 };
 
+// DFT of 6 = 2 x 3 and of 12 = 3 x 4 points as prime-factor transforms: the
+// factors are coprime, so with n = N2 n1 + N1 n2 and k by the Chinese
+// remainder theorem no twiddles stand between them, and the index maps cost
+// nothing at compile time.
+template <typename T, bool FWD>
+struct Dft<T, 6, FWD> {
+    __device__ __forceinline__ static void run(cpx<T> *v) {
+        cpx<T> y[2][3];
+#pragma unroll
+        for (int n1 = 0; n1 < 2; n1++) {
+#pragma unroll
+            for (int n2 = 0; n2 < 3; n2++) y[n1][n2] = v[(3 * n1 + 2 * n2) % 6];
+            Dft<T, 3, FWD>::run(y[n1]);
+        }
+#pragma unroll
+        for (int k2 = 0; k2 < 3; k2++) {
+            v[(4 * k2) % 6]     = cadd(y[0][k2], y[1][k2]);
+            v[(3 + 4 * k2) % 6] = csub(y[0][k2], y[1][k2]);
+        }
+    }
+};
+
+template <typename T, bool FWD>
+struct Dft<T, 12, FWD> {
+    __device__ __forceinline__ static void run(cpx<T> *v) {
+        cpx<T> y[3][4];
+#pragma unroll
+        for (int n1 = 0; n1 < 3; n1++) {
+#pragma unroll
+            for (int n2 = 0; n2 < 4; n2++) y[n1][n2] = v[(4 * n1 + 3 * n2) % 12];
+            Dft<T, 4, FWD>::run(y[n1]);
+        }
+#pragma unroll
+        for (int k2 = 0; k2 < 4; k2++) {
+            cpx<T> b[3] = {y[0][k2], y[1][k2], y[2][k2]};
+            Dft<T, 3, FWD>::run(b);
+#pragma unroll
+            for (int k1 = 0; k1 < 3; k1++) v[(4 * k1 + 9 * k2) % 12] = b[k1];
+        }
+    }
+};
+
 struct WavePlan {
     int n;
     int r[8];
     int ns[8];
 };
 
-// L = E^a * rem with rem | E; REV reverses the radix order.
+// L = E^a * rem with rem | E, or, where 3 divides L (E = 12), 12 or 6 times
+// powers of four; REV reverses the radix order.
 __host__ __device__ constexpr WavePlan make_wave_plan(int L, int E, bool rev) {
     WavePlan p{};
     int      rs[8] = {};
     int      k = 0, m = L;
+    if (L % 3 == 0) {
+        int q = 0;  // L / 12 = 2^q
+        while ((12 << q) < L) q++;
+        rs[k++] = q % 2 ? 6 : 12;
+        m /= rs[0];
+        while (m > 1) {
+            rs[k++] = 4;
+            m /= 4;
+        }
+    }
     while (m >= E && m % E == 0) {
         rs[k++] = E;
         m /= E;
@@ -120,13 +173,17 @@ __host__ __device__ constexpr int wave_tw_off(const WavePlan &p, int s) {
 __host__ __device__ constexpr int wave_tw_size(const WavePlan &p) { return wave_tw_off(p, p.n); }
 
 // Points per lane: `pref` (16 for FP32, 8 for FP64 by default), at most L
-// and at least L/64 (a line fits one wavefront).
+// and at least L/64 (a line fits one wavefront); 12 where 3 divides L (the
+// radices 12, 6 and 4 divide it, and L/12 lanes fill wavefronts evenly).
 template <typename T, int L, int PREF = (sizeof(T) == 4 ? 16 : 8)>
 struct WaveE {
-    static constexpr int value = L < PREF ? L : (L / PREF > 64 ? L / 64 : PREF);
+    static constexpr int value = L % 3 == 0 ? 12 : L < PREF ? L : (L / PREF > 64 ? L / 64 : PREF);
 };
 
-__host__ __device__ constexpr bool wave_fft_ok(int L) { return L >= 8 && L <= 512 && (L & (L - 1)) == 0; }
+__host__ __device__ constexpr bool wave_fft_ok(int L) {
+    if (L % 3 == 0) return L >= 12 && L <= 384 && ((L / 3) & (L / 3 - 1)) == 0;
+    return L >= 8 && L <= 512 && (L & (L - 1)) == 0;
+}
 
 // LDS strip of one line in 128-byte groups (8 FP64 / 16 FP32 complex).
 // KH_WAVE_SWIZZLE 0: each group padded by one element; 1: no padding, the
@@ -191,7 +248,7 @@ struct WaveFft {
 #pragma unroll
         for (int b = 0; b < NB; b++) {
             const int j = g + G * b;
-            const int k = j & (Ns - 1);
+            const int k = (int)((unsigned)j % (unsigned)Ns);
             if constexpr (Ns > 1) {
 #pragma unroll
                 for (int r = 1; r < R; r++) {
@@ -205,8 +262,8 @@ struct WaveFft {
 #pragma unroll
             for (int b = 0; b < NB; b++) {
                 const int j    = g + G * b;
-                const int k    = j & (Ns - 1);
-                const int base = (j / Ns) * Ns * R + k;
+                const int k    = (int)((unsigned)j % (unsigned)Ns);
+                const int base = (j - k) * R + k;
 #pragma unroll
                 for (int r = 0; r < R; r++) buf[WavePad<T>::at(base + r * Ns)] = v[b * R + r];
             }

@@ -1,5 +1,4 @@
-// kh_zwave.h -- z passes on the wavefront-scope FFT engine (kh_zwave.hip),
-// used for power-of-two NZ from 8 to 512.
+// kh_zwave.h -- z passes on the wavefront-scope FFT engine (kh_zwave.hip).
 #pragma once
 
 #include "kh_common.h"
@@ -7,12 +6,11 @@
 
 namespace kh {
 
-bool zw_supported(int L);
 // rows of L reals -> half spectra (all L/2+1 modes); spectral rows `pitch` complex apart
 template <typename T>
 hipError_t zw_r2c(int L, const T *in, cpx<T> *out, long long nrows, int pitch, hipStream_t s, int kzv = -1);
 // half spectra (modes kz < kzv, rest zero) -> rows of L reals * scale; grid y = component.
-// mask (a real field, L >= 32): only 4-point vectors where it is nonzero are written
+// mask (a real field): only 4-point vectors where it is nonzero are written
 // (a non-null skip, masked passes only: nothing is done once *skip is nonzero;
 // a non-null batch, masked passes only: its batch fields make one launch
 // cover the batch's runs)
@@ -20,12 +18,11 @@ template <typename T>
 hipError_t zw_c2r(int L, const ZIO<T> &io, int ncomp, long long nrows, T scale, int kzv, int pitch,
                   hipStream_t s, const T *mask = nullptr, const int *skip = nullptr, const Grid *batch = nullptr,
                   Occ occ = {});
-// inverse z (3) -> advection products -> forward z (5), modes kz < TRN_Z
-// inverse z pass of omega fused with u x omega (lengths >= 32)
-bool zw_cross_supported(int L);
+// inverse z pass of omega fused with u x omega
 template <typename T>
 hipError_t zw_c2r_cross(int L, const ZIO<T> &io, const T *const u[3], long long nrows, T scale, int kzv, int pitch,
                         hipStream_t s);
+// inverse z (3) -> advection products -> forward z (5), modes kz < TRN_Z
 template <typename T>
 hipError_t zw_adv(const Grid &g, cpx<T> *const s3[3], cpx<T> *const p5[5], T scale, hipStream_t s);
 // f = up - min(phi_sum,1) u* -> forward z (3), modes kz < TRN_Z; u* = us +

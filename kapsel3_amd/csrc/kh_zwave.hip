@@ -1,5 +1,5 @@
-// kh_zwave.hip -- z passes on the wavefront-scope FFT engine (power-of-two
-// NZ from 8 to 512).
+// kh_zwave.hip -- z passes on the wavefront-scope FFT engine (every
+// supported NZ: 2^a and 3 2^a from 8 to 512).
 //
 // Rows along z are contiguous in both layouts (real R[x][y][z], spectral
 // S[x][y][kz]), so every lane reads its points straight from HBM in the
@@ -80,7 +80,7 @@ __device__ __forceinline__ void store_pair(const cpx<T> *v, const WaveLane<T, L,
         const int k = wl.g + G * t;
         if (k < kzv) {
             const cpx<T> Zk = wl.buf[WavePad<T>::at(k)];
-            const cpx<T> Zm = cconj(wl.buf[WavePad<T>::at((L - k) & (L - 1))]);
+            const cpx<T> Zm = cconj(wl.buf[WavePad<T>::at(k ? L - k : 0)]);
             const cpx<T> d  = csub(Zk, Zm);
             if (wl.okA) ra[k] = cscale(cadd(Zk, Zm), (T)0.5);
             if (wl.okB) rb[k] = cmk(d.y * (T)0.5, -d.x * (T)0.5);
@@ -509,9 +509,7 @@ __global__ __launch_bounds__(256) void k_zw_force(Grid g, ZForceIO<T> io, int cl
 }
 
 // ------------------------------------------------------------ launchers
-#define KH_FOR_EACH_WL(X) X(8) X(16) X(32) X(64) X(128) X(256) X(512)
-
-bool zw_supported(int L) { return wave_fft_ok(L); }
+#define KH_FOR_EACH_WL(X) X(8) X(12) X(16) X(24) X(32) X(48) X(64) X(96) X(128) X(192) X(256) X(384) X(512)
 
 // points per lane of each pass (the advection pass holds three components
 // in registers, so it may take fewer points per lane; the force pass, which
@@ -538,7 +536,7 @@ bool zw_supported(int L) { return wave_fft_ok(L); }
 // this many points per lane or fewer: at 8 (FP32 and FP64) the extra
 // registers cost less than the second read and transform of u2
 #ifndef KH_ADV_LIVE3_E
-#define KH_ADV_LIVE3_E 8
+#define KH_ADV_LIVE3_E 12
 #endif
 template <typename T, int L>
 struct ZwE {
@@ -572,19 +570,15 @@ template <typename T>
 hipError_t zw_c2r(int L, const ZIO<T> &io, int ncomp, long long nrows, T scale, int kzv, int pitch,
                   hipStream_t s, const T *mask, const int *skip, const Grid *batch, Occ occ) {
     const Grid bg     = batch ? *batch : Grid{};
-    const bool masked = (mask || occ.w) && L >= 32;
-    if (occ.w && !masked) return hipErrorInvalidValue;
+    const bool masked = mask || occ.w;
     if (batch_z(bg) > 1 && !masked) return hipErrorInvalidValue;  // only the masked pass is batched
     if (skip && !masked) return hipErrorInvalidValue;  // only the masked pass takes a skip flag
-    if (masked) {  // every length with 4 points per lane per row
+    if (masked) {
         switch (L) {
 #define KH_CASE(n)                                                                                              \
     case n:                                                                                                     \
-        if constexpr (n >= 32) {                                                                                \
-            hipLaunchKernelGGL((k_zw_c2r_masked<T, n, ZwE<T, n>::pass>), dim3(zw_blocks<T, n, ZwE<T, n>::pass>(nrows), 1, batch_z(bg)), dim3(256), 0, s, io, ncomp, mask, nrows, scale, kzv, pitch, skip, bg, occ); \
-            return hipGetLastError();                                                                           \
-        }                                                                                                       \
-        break;
+        hipLaunchKernelGGL((k_zw_c2r_masked<T, n, ZwE<T, n>::pass>), dim3(zw_blocks<T, n, ZwE<T, n>::pass>(nrows), 1, batch_z(bg)), dim3(256), 0, s, io, ncomp, mask, nrows, scale, kzv, pitch, skip, bg, occ); \
+        return hipGetLastError();
             KH_FOR_EACH_WL(KH_CASE)
 #undef KH_CASE
             default: return hipErrorInvalidValue;
@@ -601,19 +595,14 @@ hipError_t zw_c2r(int L, const ZIO<T> &io, int ncomp, long long nrows, T scale, 
     }
 }
 
-bool zw_cross_supported(int L) { return zw_supported(L) && L >= 32; }
-
 template <typename T>
 hipError_t zw_c2r_cross(int L, const ZIO<T> &io, const T *const u[3], long long nrows, T scale, int kzv, int pitch,
                         hipStream_t s) {
     switch (L) {
 #define KH_CASE(n)                                                                                              \
     case n:                                                                                                     \
-        if constexpr (n >= 32) {                                                                                \
-            hipLaunchKernelGGL((k_zw_c2r_cross<T, n, ZwE<T, n>::pass>), dim3(zw_blocks<T, n, ZwE<T, n>::pass>(nrows)), dim3(256), 0, s, io, u[0], u[1], u[2], nrows, scale, kzv, pitch); \
-            return hipGetLastError();                                                                           \
-        }                                                                                                       \
-        break;
+        hipLaunchKernelGGL((k_zw_c2r_cross<T, n, ZwE<T, n>::pass>), dim3(zw_blocks<T, n, ZwE<T, n>::pass>(nrows)), dim3(256), 0, s, io, u[0], u[1], u[2], nrows, scale, kzv, pitch); \
+        return hipGetLastError();
         KH_FOR_EACH_WL(KH_CASE)
 #undef KH_CASE
         default: break;
