@@ -65,9 +65,7 @@ def kernel_bytes(name, n, p, npts, sf, nphi=None, occ=None):
         "y_inv": cs * (3 * xcol + 3 * ycol),
         "z_adv": cs * (3 * ycol + 5 * ycol),
         "y_fwd_adv": cs * (5 * ycol + 5 * xcol),
-        "x_fwd_adv": cs * (5 * xcol + 5 * kept),
-        "adv_ns": cs * (5 + 2 + 2) * kept,
-        "x_adv_ns": cs * (5 * xcol + 2 * kept + 2 * kept),
+        "x_ns_u": cs * (5 * xcol + 2 * kept + 2 * kept + 3 * xcol),
         # u* is read only where phi_sum > 0 (F_H gather, rigidity force):
         # three spectra in, phi_sum everywhere, u* written at those points
         "z_c2r": cs * 3 * ycol + (bits if occ else sf * real) + sf * 3 * nphi,

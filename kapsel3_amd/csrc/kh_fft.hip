@@ -13,60 +13,33 @@
 // reads and writes each field element once: the z passes on the
 // wavefront-scope engine (kh_zwave.hip), the y and x passes a tile of C
 // neighbouring columns (C*elem = 128 B per row) staged in LDS.
+#include "kh_col_fft.h"
 #include "kh_fft.h"
-#include "kh_fft_engine.h"
 #include "kh_zwave.h"
 
 namespace kh {
-
-
-template <typename T>
-struct FftTile;
-template <>
-struct FftTile<double> {
-    static constexpr int C = 8;  // columns per y/x tile (128 B rows)
-};
-template <>
-struct FftTile<float> {
-    static constexpr int C = 16;
-};
 
 // ------------------------------------------------------------ y / x pass
 // Lines of L points at stride `lstride`; a tile is C consecutive columns.
 // Tile t of outer block o starts at data + o*ostride + t*C; `ncols` columns
 // are valid per outer block.
 template <typename T, int L, bool FWD>
-__global__ __launch_bounds__(PassThreads<T>::value) void k_fft_strided(cpx<T> *__restrict__ data, long long lstride,
-                                                                       int ncols, long long ostride, int tiles) {
-    constexpr int NT  = PassThreads<T>::value;
-    constexpr int C   = FftTile<T>::C;
-    constexpr int BS  = ColStride<T, C>::value;
-    constexpr int NPT = (C * L + NT - 1) / NT;
-    __shared__ cpx<T> s[L * BS], tw[L];
-    fill_twiddles<T, L, NT>(tw);
-    const int o = blockIdx.x / tiles, t = blockIdx.x - o * tiles;
-    const int c0 = t * C;
-    cpx<T>   *base = data + (long long)o * ostride + c0;
-    cpx<T>    v[NPT];
+__global__ __launch_bounds__((ColGeom<T, L>::NT)) void k_fft_strided(cpx<T> *__restrict__ data, long long lstride,
+                                                                   int ncols, long long ostride, int tiles) {
+    using F = ColFft<T, L, FWD, FWD>;
+    __shared__ cpx<T> s[F::BUF], tw[F::TW];
+    const int  o = blockIdx.x / tiles, t = blockIdx.x - o * tiles;
+    const int  g = threadIdx.x / F::C, c = threadIdx.x - g * F::C;
+    const bool ok   = t * F::C + c < ncols;
+    cpx<T>    *base = data + (long long)o * ostride + t * F::C + c;
+    cpx<T>     v[F::E];
 #pragma unroll
-    for (int i = 0; i < NPT; i++) {
-        const int e = threadIdx.x + i * NT;
-        const int n = e / C, c = e - n * C;
-        v[i] = (e < C * L && c0 + c < ncols) ? base[(long long)n * lstride + c] : cmk((T)0, (T)0);
-    }
+    for (int i = 0; i < F::E; i++) v[i] = ok ? base[(long long)F::in_point(g, i) * lstride] : cmk((T)0, (T)0);
+    F::fill_tw(tw);  // while the loads are in flight
+    F::run(v, s, tw, g, c);
 #pragma unroll
-    for (int i = 0; i < NPT; i++) {
-        const int e = threadIdx.x + i * NT;
-        if (e < C * L) s[(e / C) * BS + e % C] = v[i];
-    }
-    __syncthreads();
-    fft_cols_ip<T, L, C, BS, NT, FWD>(s, tw);
-#pragma unroll
-    for (int i = 0; i < NPT; i++) {
-        const int e = threadIdx.x + i * NT;
-        const int n = e / C, c = e - n * C;
-        if (e < C * L && c0 + c < ncols) base[(long long)n * lstride + c] = s[n * BS + c];
-    }
+    for (int i = 0; i < F::E; i++)
+        if (ok) base[(long long)F::out_point(g, i) * lstride] = v[i];
 }
 
 // ------------------------------------------------------------ launchers
@@ -85,15 +58,15 @@ bool fft_length_supported(int L) {
 template <typename T, bool FWD>
 static hipError_t launch_strided(int L, cpx<T> *data, long long lstride, int ncols, long long ostride, int nouter,
                                  hipStream_t s) {
-    constexpr int C     = FftTile<T>::C;
-    const int     tiles = (ncols + C - 1) / C;
-    const long long nb  = (long long)tiles * nouter;
     switch (L) {
-#define KH_CASE(n)                                                                                              \
-    case n:                                                                                                     \
-        hipLaunchKernelGGL((k_fft_strided<T, n, FWD>), dim3((unsigned)nb), dim3(PassThreads<T>::value), 0, s, data, lstride, ncols, \
-                           ostride, tiles);                                                                     \
-        return hipGetLastError();
+#define KH_CASE(n)                                                                                                 \
+    case n: {                                                                                                      \
+        using Geo       = ColGeom<T, n>;                                                                           \
+        const int tiles = (ncols + Geo::C - 1) / Geo::C;                                                           \
+        hipLaunchKernelGGL((k_fft_strided<T, n, FWD>), dim3((unsigned)((long long)tiles * nouter)), dim3(Geo::NT), \
+                           0, s, data, lstride, ncols, ostride, tiles);                                            \
+        return hipGetLastError();                                                                                  \
+    }
         KH_FOR_EACH_L(KH_CASE)
 #undef KH_CASE
         default: return hipErrorInvalidValue;

@@ -39,10 +39,11 @@ hipError_t z_force(const Grid &g, T *const up[3], T *phis, T *const us[3], cpx<T
 template <typename T>
 hipError_t x_slip(const Grid &g, cpx<T> *const f[3], cpx<T> *a0, cpx<T> *a1, double *dc, const int *skip,
                   hipStream_t s);
-// forward x (5 products) -> Omega + slaved-Euler update of zeta at the kept modes
+// forward x (5 products) -> Omega + slaved-Euler update of zeta at the kept
+// modes -> FIX_CELL, u*_hat -> inverse x, 3 components (u may be product buffers)
 template <typename T>
-hipError_t x_adv_ns(const Grid &g, const Comps<T> &prod, cpx<T> *z0, cpx<T> *z1, double dmy0, double dmy1,
-                    hipStream_t s);
+hipError_t x_ns_u(const Grid &g, const Comps<T> &prod, cpx<T> *z0, cpx<T> *z1, cpx<T> *const u[3], double *ukdc,
+                  double dmy0, double dmy1, int fixmask, hipStream_t s);
 // forward x (3) -> projection + u* + curl -> zeta, uk_dc
 template <typename T>
 hipError_t x_f_zeta(const Grid &g, cpx<T> *const f[3], cpx<T> *z0, cpx<T> *z1, double *ukdc, hipStream_t s);

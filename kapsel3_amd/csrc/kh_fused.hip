@@ -14,38 +14,24 @@
 // forward z pass (k_zw_adv), the construction of u_hat from zeta sits in
 // front of the inverse x pass (k_x_zeta2u_inv), and the projection, the
 // addition of u* and the curl sit behind the forward x pass (k_x_f_zeta).
-#include "kh_fft_engine.h"
+#include "kh_col_fft.h"
 #include "kh_fused.h"
 #include "kh_modes.h"
 #include "kh_zwave.h"
 
+#include <type_traits>
+
 namespace kh {
 
-template <typename T>
-struct ColTile;
-template <>
-struct ColTile<double> {
-    static constexpr int C = 8;  // 8 x 16 B = 128 B per line element
-};
-template <>
-struct ColTile<float> {
-    static constexpr int C = 16;  // 16 x 8 B = 128 B
-};
-
-// Column tile and workgroup size of the fused x passes (all components in
-// one workgroup)
-template <typename T>
-struct XTile {
-    static constexpr int C  = ColTile<T>::C;
-    static constexpr int NT = PassThreads<T>::value;
-};
-// zeta -> u_hat -> inverse x: FP32 runs narrower tiles on 4-wavefront
-// workgroups (more workgroups resident, a shorter last round)
-template <typename T>
-struct XZTile {
-    static constexpr int C  = sizeof(T) == 4 ? 8 : XTile<T>::C;
-    static constexpr int NT = sizeof(T) == 4 ? 256 : XTile<T>::NT;
-};
+// Element e of a spectral field. A field has at most 512 x 512 x 272 complex
+// elements, so byte offsets fit 32 bits: one offset register then serves every
+// field a lane reads at the same place (the field's base stays scalar), where
+// 64-bit addresses took a register pair per access.
+template <typename P>
+__device__ __forceinline__ P &at(P *field, unsigned e) {
+    using C = typename std::conditional<std::is_const<P>::value, const char, char>::type;
+    return *reinterpret_cast<P *>(reinterpret_cast<C *>(field) + e * (unsigned)sizeof(P));
+}
 
 // ------------------------------------------------------------------------
 // Column passes. Y mode: outer block = x, line along y, columns kz < ncols.
@@ -53,56 +39,69 @@ struct XZTile {
 // in_mask: rows whose wavenumber is truncated are taken as zero (not read).
 // out_mask: such rows are not written.
 template <typename T, int L, bool FWD, bool XMODE>
-__global__ __launch_bounds__(PassThreads<T>::value) void k_cols(Comps<T> comps, Grid g, int ncols, int in_mask,
-                                                                int out_mask, const int *__restrict__ skip) {
+__global__ __launch_bounds__((ColGeom<T, L>::NT)) void k_cols(Comps<T> comps, Grid g, int ncols, int in_mask,
+                                                            int out_mask, const int *__restrict__ skip) {
+    using F = ColFft<T, L, FWD, FWD>;
     if ((skip && *skip) || batch_skip(g)) return;
     cpx<T> *__restrict__ data = brun(comps.p[blockIdx.y], g);  // one component per grid row
-    constexpr int NT  = PassThreads<T>::value;
-    constexpr int C   = ColTile<T>::C;
-    constexpr int BS  = ColStride<T, C>::value;
-    constexpr int NPT = (C * L + NT - 1) / NT;
-    __shared__ cpx<T> s[L * BS], tw[L];
-    fill_twiddles<T, L, NT>(tw);
-    const int ntiles = (ncols + C - 1) / C;
-    const int o = blockIdx.x / ntiles, kz0 = (blockIdx.x - o * ntiles) * C;
-    long long base, lstride;
-    int       trn, nline;
+    __shared__ cpx<T> s[F::BUF], tw[F::TW];
+    const int ntiles = (ncols + F::C - 1) / F::C;
+    const int o = blockIdx.x / ntiles, kz0 = (blockIdx.x - o * ntiles) * F::C;
+    const int l = threadIdx.x / F::C, c = threadIdx.x - l * F::C;
+    unsigned base, lstride;
+    int      trn;
     if (XMODE) {
         const int j = kept_index(o, g.ny, g.trn_y);
-        base        = (long long)j * g.nzp + kz0;
-        lstride     = (long long)g.ny * g.nzp;
+        base        = (unsigned)j * g.nzp + kz0 + c;
+        lstride     = (unsigned)g.ny * g.nzp;
         trn         = g.trn_x;
-        nline       = g.nx;
     } else {
-        base    = (long long)o * g.ny * g.nzp + kz0;
+        base    = (unsigned)o * g.ny * g.nzp + kz0 + c;
         lstride = g.nzp;
         trn     = g.trn_y;
-        nline   = g.ny;
     }
-    cpx<T> v[NPT];
+    const bool ok = kz0 + c < ncols;
+    cpx<T>     v[F::E];
 #pragma unroll
-    for (int i = 0; i < NPT; i++) {
-        const int e = threadIdx.x + i * NT;
-        const int n = e / C, c = e - n * C;
-        const int k = (n > nline / 2) ? n - nline : n;
+    for (int i = 0; i < F::E; i++) {
+        const int n = F::in_point(l, i);
         v[i]        = cmk((T)0, (T)0);
-        if (e < C * L && kz0 + c < ncols && (!in_mask || kept1(k, trn))) v[i] = data[base + n * lstride + c];
+        if (ok && (!in_mask || kept1(n > L / 2 ? n - L : n, trn))) v[i] = at(data, base + n * lstride);
     }
+    F::fill_tw(tw);  // while the loads are in flight
+    F::run(v, s, tw, l, c);
 #pragma unroll
-    for (int i = 0; i < NPT; i++) {
-        const int e = threadIdx.x + i * NT;
-        if (e < C * L) s[(e / C) * BS + e % C] = v[i];
-    }
-    __syncthreads();
-    fft_cols_ip<T, L, C, BS, NT, FWD>(s, tw);
-#pragma unroll
-    for (int i = 0; i < NPT; i++) {
-        const int e = threadIdx.x + i * NT;
-        const int n = e / C, c = e - n * C;
-        const int k = (n > nline / 2) ? n - nline : n;
-        if (e < C * L && kz0 + c < ncols && (!out_mask || kept1(k, trn))) data[base + n * lstride + c] = s[n * BS + c];
+    for (int i = 0; i < F::E; i++) {
+        const int n = F::out_point(l, i);
+        if (ok && (!out_mask || kept1(n > L / 2 ? n - L : n, trn))) at(data, base + n * lstride) = v[i];
     }
 }
+
+// The tile of a fused x pass: workgroup -> kept (ky) row and kz columns, lane
+// -> column c and its E points of the line along x.
+template <typename T, int L>
+struct XTile {
+    using Geo = ColGeom<T, L>;
+    int       l, kz, j, iky;
+    bool      ok;
+    unsigned  base, lstride;
+    __device__ __forceinline__ explicit XTile(const Grid &g) {
+        const int ntiles = (g.trn_z + Geo::C - 1) / Geo::C;
+        const int o      = blockIdx.x / ntiles;
+        l                = threadIdx.x / Geo::C;
+        kz               = (blockIdx.x - o * ntiles) * Geo::C + (threadIdx.x - l * Geo::C);
+        j                = kept_index(o, g.ny, g.trn_y);
+        iky              = ky_of(g, j);
+        ok               = kz < g.trn_z;
+        lstride          = (unsigned)g.ny * g.nzp;
+        base             = (unsigned)j * g.nzp + kz;
+    }
+    __device__ __forceinline__ unsigned elem(int n) const { return base + (unsigned)n * lstride; }
+    __device__ __forceinline__ int  c() const { return threadIdx.x - l * Geo::C; }
+    __device__ __forceinline__ bool first() const { return blockIdx.x == 0; }  // holds (ky, kz) = (0, 0)
+    __device__ __forceinline__ static int ikx(int n) { return n > L / 2 ? n - L : n; }
+    __device__ __forceinline__ bool kept(const Grid &g, int n) const { return ok && kept1(ikx(n), g.trn_x); }
+};
 
 // ------------------------------------------------------------------------
 // u_hat from zeta (Zeta_k2u_k, fft_wrapper.cxx:591-688, on the truncated
@@ -153,137 +152,151 @@ __device__ __forceinline__ void zeta_to_uhat(const Grid &g, int ikx, int iky, in
 // inverse x pass of each component. fixmask: FIX_CELL zeroing of uk_dc
 // (sp_3d_ns.cxx:46-52), done by the block holding (ky,kz) = (0,0).
 template <typename T, int L>
-__global__ __launch_bounds__(XZTile<T>::NT) void k_x_zeta2u_inv(
+__global__ __launch_bounds__((ColGeom<T, L>::NT)) void k_x_zeta2u_inv(
     Grid g, const cpx<T> *__restrict__ z0, const cpx<T> *__restrict__ z1, cpx<T> *__restrict__ u0,
     cpx<T> *__restrict__ u1, cpx<T> *__restrict__ u2, double *__restrict__ ukdc, int fixmask) {
+    using F = ColFft<T, L, false, false>;
     if (batch_skip(g)) return;
     z0 = brun(z0, g), z1 = brun(z1, g), u0 = brun(u0, g), u1 = brun(u1, g), u2 = brun(u2, g);
     ukdc = brun(ukdc, g);
-    constexpr int NT  = XZTile<T>::NT;
-    constexpr int C   = XZTile<T>::C;
-    constexpr int BS  = ColStride<T, C>::value;
-    constexpr int NPT = (C * L + NT - 1) / NT;
-    __shared__ cpx<T> s[L * BS], tw[L];
+    __shared__ cpx<T> s[F::BUF], tw[F::TW];
     __shared__ double uk[3];
-    fill_twiddles<T, L, NT>(tw);
-    const int ntiles = (g.trn_z + C - 1) / C;
-    const int o = blockIdx.x / ntiles, kz0 = (blockIdx.x - o * ntiles) * C;
-    const int j = kept_index(o, g.ny, g.trn_y), iky = (j > g.hny) ? j - g.ny : j;
-    if (threadIdx.x == 0) {
-        for (int d = 0; d < 3; d++) uk[d] = (fixmask & (1 << d)) ? 0.0 : ukdc[d];
+    const XTile<T, L> t(g);
+    cpx<T>            D1[F::E], D2[F::E];
+#pragma unroll
+    for (int i = 0; i < F::E; i++) {
+        const int  n  = F::in_point(t.l, i);
+        const bool ok = t.kept(g, n);
+        D1[i]         = ok ? at(z0, t.elem(n)) : cmk((T)0, (T)0);
+        D2[i]         = ok ? at(z1, t.elem(n)) : cmk((T)0, (T)0);
+    }
+    F::fill_tw(tw);
+    if (threadIdx.x < 3) {
+        const bool fixed = fixmask & (1 << threadIdx.x);
+        uk[threadIdx.x]  = fixed ? 0.0 : ukdc[threadIdx.x];
+        if (fixed && t.first()) ukdc[threadIdx.x] = 0.0;
     }
     __syncthreads();
-    if (fixmask && j == 0 && kz0 == 0 && threadIdx.x == 0)
-        for (int d = 0; d < 3; d++)
-            if (fixmask & (1 << d)) ukdc[d] = 0.0;
-    const long long lstride = (long long)g.ny * g.nzp;
-    const long long base    = (long long)j * g.nzp + kz0;
-    cpx<T>          D1[NPT], D2[NPT];
+    cpx<T> U[3][F::E];
 #pragma unroll
-    for (int i = 0; i < NPT; i++) {
-        const int p = threadIdx.x + i * NT;
-        const int n = p / C, c = p - n * C, kz = kz0 + c;
-        const int ikx = (n > g.hnx) ? n - g.nx : n;
-        const bool ok = p < C * L && kz < g.trn_z && kept1(ikx, g.trn_x);
-        D1[i]         = ok ? z0[base + n * lstride + c] : cmk((T)0, (T)0);
-        D2[i]         = ok ? z1[base + n * lstride + c] : cmk((T)0, (T)0);
-    }
-    cpx<T> U[3][NPT];
-#pragma unroll
-    for (int i = 0; i < NPT; i++) {
-        const int p = threadIdx.x + i * NT;
-        const int n = p / C, c = p - n * C, kz = kz0 + c;
-        const int ikx = (n > g.hnx) ? n - g.nx : n;
+    for (int i = 0; i < F::E; i++) {
+        const int n = F::in_point(t.l, i);
         U[0][i] = U[1][i] = U[2][i] = cmk((T)0, (T)0);
-        if (p < C * L && kz < g.trn_z && kept1(ikx, g.trn_x)) {
+        if (t.kept(g, n)) {
             cpx<T> u[3];
-            zeta_to_uhat<T>(g, ikx, iky, kz, D1[i], D2[i], uk, u);
+            zeta_to_uhat<T>(g, t.ikx(n), t.iky, t.kz, D1[i], D2[i], uk, u);
             U[0][i] = u[0];
             U[1][i] = u[1];
             U[2][i] = u[2];
+            __builtin_amdgcn_sched_barrier(0);  // one mode's FP64 temporaries at a time
         }
     }
     cpx<T> *out[3] = {u0, u1, u2};
 #pragma unroll
     for (int d = 0; d < 3; d++) {
+        F::run(U[d], s, tw, t.l, t.c());
 #pragma unroll
-        for (int i = 0; i < NPT; i++) {
-            const int p = threadIdx.x + i * NT;
-            if (p < C * L) s[(p / C) * BS + p % C] = U[d][i];
-        }
-        __syncthreads();
-        fft_cols_ip<T, L, C, BS, NT, false>(s, tw);
-#pragma unroll
-        for (int i = 0; i < NPT; i++) {
-            const int e = threadIdx.x + i * NT;
-            const int n = e / C, c = e - n * C;
-            if (e < C * L && kz0 + c < g.trn_z) out[d][base + n * lstride + c] = s[n * BS + c];
-        }
-        __syncthreads();
+        for (int i = 0; i < F::E; i++)
+            if (t.ok) at(out[d], t.elem(F::out_point(t.l, i))) = U[d][i];
     }
 }
 
 // ------------------------------------------------------------------------
 // Forward x pass of the five advection products on the kept (ky,kz)
-// columns, then per kept mode Omega_k2zeta_k + the slaved-Euler update of
-// zeta (NS_solver_slavedEuler, fluid_solver.cxx:348-374): the products are
-// never written back in spectral form.
-template <typename T, int L>
-__global__ __launch_bounds__(XTile<T>::NT) void k_x_adv_ns(Grid g, Comps<T> prod, cpx<T> *__restrict__ z0,
-                                                                    cpx<T> *__restrict__ z1, double dmy0,
-                                                                    double dmy1) {
-    if (batch_skip(g)) return;
-    for (int q = 0; q < 5; q++) prod.p[q] = brun(prod.p[q], g);
-    z0 = brun(z0, g), z1 = brun(z1, g);
-    constexpr int NT  = XTile<T>::NT;
-    constexpr int C   = XTile<T>::C;
-    constexpr int BS  = ColStride<T, C>::value;
-    constexpr int NPT = (C * L + NT - 1) / NT;
-    __shared__ cpx<T> s[L * BS], tw[L];
-    fill_twiddles<T, L, NT>(tw);
-    const int ntiles = (g.trn_z + C - 1) / C;
-    const int o = blockIdx.x / ntiles, kz0 = (blockIdx.x - o * ntiles) * C;
-    const int j = kept_index(o, g.ny, g.trn_y), iky = (j > g.hny) ? j - g.ny : j;
-    const long long lstride = (long long)g.ny * g.nzp;
-    const long long base    = (long long)j * g.nzp + kz0;
-    cpx<T>          Ph[5][NPT];
+// columns, per kept mode Omega_k2zeta_k + the slaved-Euler update of zeta
+// (NS_solver_slavedEuler, fluid_solver.cxx:348-374), FIX_CELL's zeroing of
+// uk_dc (sp_3d_ns.cxx:46-52) and u*_hat of the new zeta, then the inverse x
+// pass of its three components: neither the products' spectra nor the new zeta
+// are read back from memory. Each product is folded into the two rows of Omega
+// its mode stores as soon as it is transformed (8 FP64 registers a mode
+// instead of 20), while the next one's loads are in flight. Bound by memory
+// latency at two or three workgroups a CU. Against the launches it replaces
+// (products' x pass, slaved Euler, zeta -> u_hat): 256^3 mixed 136 -> 103 us
+// (3.1 TB/s), 256^3 FP64 199 -> 157 us (4.1 TB/s), 192^3 mixed 61 -> 34 us,
+// 512^3 mixed 1320 -> 735 us.
+template <typename T, int L, int Q>
+__device__ __forceinline__ void adv_products(const Grid &g, const XTile<T, L> &t, const Comps<T> &prod,
+                                             cpx<T> (&v)[2][ColGeom<T, L>::E], cpx<double> (&acc)[ColGeom<T, L>::E][2],
+                                             cpx<T> *s, const cpx<T> *tw) {
+    using F = ColFft<T, L, true, true>;
+    if constexpr (Q < 5) {
+        if constexpr (Q + 1 < 5) {
+            const cpx<T> *src = brun(prod.p[Q + 1], g);
+            unsigned      e0  = t.elem(F::in_point(t.l, 0));
+            asm volatile("" : "+v"(e0));  // these loads come after the previous product's fold, not all five at once
 #pragma unroll
-    for (int q = 0; q < 5; q++) {
-        const cpx<T> *src = prod.p[q];
-        cpx<T>        v[NPT];
-#pragma unroll
-        for (int i = 0; i < NPT; i++) {
-            const int e = threadIdx.x + i * NT;
-            const int n = e / C, c = e - n * C;
-            v[i]        = (e < C * L && kz0 + c < g.trn_z) ? src[base + n * lstride + c] : cmk((T)0, (T)0);
+            for (int i = 0; i < F::E; i++)
+                v[(Q + 1) & 1][i] =
+                    t.ok ? at(src, e0 + (unsigned)(F::in_point(0, i)) * t.lstride) : cmk((T)0, (T)0);
         }
+        F::run(v[Q & 1], s, tw, t.l, t.c());
+        int l = t.l;
+        asm volatile("" : "+v"(l));  // wavenumbers are worked out again for each product, not kept in registers
 #pragma unroll
-        for (int i = 0; i < NPT; i++) {
-            const int e = threadIdx.x + i * NT;
-            if (e < C * L) s[(e / C) * BS + e % C] = v[i];
+        for (int i = 0; i < F::E; i++) {
+            adv_fold<Q, T>(g, XTile<T, L>::ikx(F::out_point(l, i)), t.iky, t.kz, v[Q & 1][i], acc[i]);
+            // done here: else the compiler moves the sums to where they are
+            // used, below the mode's condition, and keeps all five products
+            asm volatile("" : "+v"(acc[i][0].x), "+v"(acc[i][0].y), "+v"(acc[i][1].x), "+v"(acc[i][1].y));
         }
-        __syncthreads();
-        fft_cols_ip<T, L, C, BS, NT, true>(s, tw);
-#pragma unroll
-        for (int i = 0; i < NPT; i++) {
-            const int p = threadIdx.x + i * NT;
-            if (p < C * L) Ph[q][i] = s[(p / C) * BS + p % C];
-        }
-        __syncthreads();
+        adv_products<T, L, Q + 1>(g, t, prod, v, acc, s, tw);
     }
+}
+template <typename T, int L>
+__global__ __launch_bounds__((ColGeom<T, L>::NT), (ColGeom<T, L>::WAVES)) void k_x_ns_u(Grid g, Comps<T> prod, cpx<T> *__restrict__ z0,
+                                                                cpx<T> *__restrict__ z1, cpx<T> *u0, cpx<T> *u1,
+                                                                cpx<T> *u2, double *__restrict__ ukdc, double dmy0,
+                                                                double dmy1, int fixmask) {
+    using F  = ColFft<T, L, true, true>;
+    using Fi = ColFft<T, L, false, false>;
+    static_assert(F::RN == Fi::R0, "forward output layout must be the inverse input layout");
+    if (batch_skip(g)) return;
+    z0 = brun(z0, g), z1 = brun(z1, g), ukdc = brun(ukdc, g);
+    __shared__ cpx<T> s[F::BUF], tw[F::TW], twi[Fi::TW];
+    __shared__ double uk[3];
+    const XTile<T, L> t(g);
+    cpx<double>       acc[F::E][2];
+    {
+        cpx<T>        v[2][F::E];
+        const cpx<T> *src = brun(prod.p[0], g);
 #pragma unroll
-    for (int i = 0; i < NPT; i++) {
-        const int p = threadIdx.x + i * NT;
-        if (p >= C * L) continue;
-        const int n = p / C, c = p - n * C, kz = kz0 + c;
-        const int ikx = (n > g.hnx) ? n - g.nx : n;
-        if (kz >= g.trn_z || !kept1(ikx, g.trn_x)) continue;
-        const long long idx  = base + n * lstride + c;
-        const cpx<T>    a[5] = {Ph[0][i], Ph[1][i], Ph[2][i], Ph[3][i], Ph[4][i]};
-        cpx<T>          x0 = z0[idx], x1 = z1[idx];
-        slaved_euler_mode<T>(g, ikx, iky, kz, a, dmy0, dmy1, x0, x1);
-        z0[idx] = x0;
-        z1[idx] = x1;
+        for (int i = 0; i < F::E; i++) {
+            v[0][i]   = t.ok ? at(src, t.elem(F::in_point(t.l, i))) : cmk((T)0, (T)0);
+            acc[i][0] = acc[i][1] = {0.0, 0.0};
+        }
+        F::fill_tw(tw);  // while the loads are in flight
+        Fi::fill_tw(twi);
+        if (threadIdx.x < 3) {
+            const bool fixed = fixmask & (1 << threadIdx.x);
+            uk[threadIdx.x]  = fixed ? 0.0 : ukdc[threadIdx.x];
+            if (fixed && t.first()) ukdc[threadIdx.x] = 0.0;
+        }
+        __syncthreads();
+        adv_products<T, L, 0>(g, t, prod, v, acc, s, tw);
+    }
+    cpx<T> U[3][F::E];
+#pragma unroll
+    for (int i = 0; i < F::E; i++) {
+        const int n = F::out_point(t.l, i);
+        U[0][i] = U[1][i] = U[2][i] = cmk((T)0, (T)0);
+        if (t.kept(g, n)) {
+            cpx<T> x0 = at(z0, t.elem(n)), x1 = at(z1, t.elem(n)), u[3];
+            slaved_euler_acc<T>(g, t.ikx(n), t.iky, t.kz, acc[i], dmy0, dmy1, x0, x1);
+            at(z0, t.elem(n)) = x0;
+            at(z1, t.elem(n)) = x1;
+            zeta_to_uhat<T>(g, t.ikx(n), t.iky, t.kz, x0, x1, uk, u);
+            U[0][i] = u[0];
+            U[1][i] = u[1];
+            U[2][i] = u[2];
+        }
+    }
+    cpx<T> *out[3] = {brun(u0, g), brun(u1, g), brun(u2, g)};
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        Fi::run(U[d], s, twi, t.l, t.c());
+#pragma unroll
+        for (int i = 0; i < Fi::E; i++)
+            if (t.ok) at(out[d], t.elem(Fi::out_point(t.l, i))) = U[d][i];
     }
 }
 
@@ -292,59 +305,37 @@ __global__ __launch_bounds__(XTile<T>::NT) void k_x_adv_ns(Grid g, Comps<T> prod
 // kept mode: truncation + Solenoidal_uk (operate_omega.cxx:171-195), the sum
 // with u* rebuilt from zeta (the reference's U2zeta_k of u* + f), and
 // U_k2zeta_k (fft_wrapper.cxx:407-476). Writes zeta at the kept modes and
-// uk_dc += f_hat(0).
+// uk_dc += f_hat(0). With the lines in registers 94 to 146 of them instead of
+// 220, so two to three workgroups a CU: 512^3 mixed 1104 -> 381 us (3.5 TB/s),
+// 256^3 mixed 61 -> 52 us, FP64 83 -> 76 us (4.5 TB/s).
 template <typename T, int L>
-__global__ __launch_bounds__(XTile<T>::NT) void k_x_f_zeta(Grid g, cpx<T> *__restrict__ f0,
-                                                                    cpx<T> *__restrict__ f1, cpx<T> *__restrict__ f2,
-                                                                    cpx<T> *__restrict__ z0, cpx<T> *__restrict__ z1,
-                                                                    double *__restrict__ ukdc) {
+__global__ __launch_bounds__((ColGeom<T, L>::NT)) void k_x_f_zeta(Grid g, const cpx<T> *__restrict__ f0,
+                                                                const cpx<T> *__restrict__ f1,
+                                                                const cpx<T> *__restrict__ f2, cpx<T> *__restrict__ z0,
+                                                                cpx<T> *__restrict__ z1, double *__restrict__ ukdc) {
+    using F = ColFft<T, L, true, true>;
     if (batch_skip(g)) return;
     f0 = brun(f0, g), f1 = brun(f1, g), f2 = brun(f2, g), z0 = brun(z0, g), z1 = brun(z1, g), ukdc = brun(ukdc, g);
-    constexpr int NT  = XTile<T>::NT;
-    constexpr int C   = XTile<T>::C;
-    constexpr int BS  = ColStride<T, C>::value;
-    constexpr int NPT = (C * L + NT - 1) / NT;
-    __shared__ cpx<T> s[L * BS], tw[L];
+    __shared__ cpx<T> s[F::BUF], tw[F::TW];
     __shared__ double uk[3];
-    fill_twiddles<T, L, NT>(tw);
-    const int ntiles = (g.trn_z + C - 1) / C;
-    const int o = blockIdx.x / ntiles, kz0 = (blockIdx.x - o * ntiles) * C;
-    const int j = kept_index(o, g.ny, g.trn_y), iky = (j > g.hny) ? j - g.ny : j;
+    const XTile<T, L> t(g);
+    const cpx<T>     *src[3] = {f0, f1, f2};
+    cpx<T>            Fh[3][F::E];
+#pragma unroll
+    for (int d = 0; d < 3; d++)
+#pragma unroll
+        for (int i = 0; i < F::E; i++)
+            Fh[d][i] = t.ok ? at(src[d], t.elem(F::in_point(t.l, i))) : cmk((T)0, (T)0);
+    F::fill_tw(tw);  // while the loads are in flight
     if (threadIdx.x < 3) uk[threadIdx.x] = ukdc[threadIdx.x];
-    const long long lstride = (long long)g.ny * g.nzp;
-    const long long base    = (long long)j * g.nzp + kz0;
-    cpx<T>         *F[3]    = {f0, f1, f2};
-    cpx<T>          Fh[3][NPT];
-    for (int d = 0; d < 3; d++) {
-        cpx<T> v[NPT];
+    __syncthreads();
 #pragma unroll
-        for (int i = 0; i < NPT; i++) {
-            const int e = threadIdx.x + i * NT;
-            const int n = e / C, c = e - n * C;
-            v[i]        = (e < C * L && kz0 + c < g.trn_z) ? F[d][base + n * lstride + c] : cmk((T)0, (T)0);
-        }
+    for (int d = 0; d < 3; d++) F::run(Fh[d], s, tw, t.l, t.c());
 #pragma unroll
-        for (int i = 0; i < NPT; i++) {
-            const int e = threadIdx.x + i * NT;
-            if (e < C * L) s[(e / C) * BS + e % C] = v[i];
-        }
-        __syncthreads();
-        fft_cols_ip<T, L, C, BS, NT, true>(s, tw);
-#pragma unroll
-        for (int i = 0; i < NPT; i++) {
-            const int p = threadIdx.x + i * NT;
-            if (p < C * L) Fh[d][i] = s[(p / C) * BS + p % C];
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int i = 0; i < NPT; i++) {
-        const int p = threadIdx.x + i * NT;
-        if (p >= C * L) continue;
-        const int n = p / C, c = p - n * C, kz = kz0 + c;
-        const int ikx = (n > g.hnx) ? n - g.nx : n;
-        if (kz >= g.trn_z || !kept1(ikx, g.trn_x)) continue;
-        const long long idx = base + n * lstride + c;
+    for (int i = 0; i < F::E; i++) {
+        const int n = F::out_point(t.l, i), ikx = t.ikx(n), iky = t.iky, kz = t.kz;
+        if (!t.kept(g, n)) continue;
+        const unsigned idx = t.elem(n);
         const double    kx = ikx * g.wave_x, ky = iky * g.wave_y, kzz = kz * g.wave_z;
         const double    K2  = (g.wave_x * ikx) * (g.wave_x * ikx) + (g.wave_y * iky) * (g.wave_y * iky) +
                           (g.wave_z * kz) * (g.wave_z * kz);
@@ -357,7 +348,7 @@ __global__ __launch_bounds__(XTile<T>::NT) void k_x_f_zeta(Grid g, cpx<T> *__res
         double       fi[3] = {a.y - di * kx, b.y - di * ky, cc.y - di * kzz};
         // u* rebuilt from the (post-NS, truncated) zeta
         cpx<T> us[3];
-        zeta_to_uhat<T>(g, ikx, iky, kz, z0[idx], z1[idx], uk, us);
+        zeta_to_uhat<T>(g, ikx, iky, kz, at(z0, idx), at(z1, idx), uk, us);
         double ur[3], ui[3];
         for (int d = 0; d < 3; d++) {
             ur[d] = (double)us[d].x + fr[d];
@@ -384,8 +375,9 @@ __global__ __launch_bounds__(XTile<T>::NT) void k_x_f_zeta(Grid g, cpx<T> *__res
             c0 = 0;
             c1 = 1;
         }
-        z0[idx] = cmk((T)ore[c0], (T)oim[c0]);
-        z1[idx] = cmk((T)ore[c1], (T)oim[c1]);
+        at(z0, idx) = cmk((T)ore[c0], (T)oim[c0]);
+        at(z1, idx) = cmk((T)ore[c1], (T)oim[c1]);
+        __builtin_amdgcn_sched_barrier(0);  // one mode's FP64 temporaries at a time
     }
 }
 
@@ -397,58 +389,35 @@ __global__ __launch_bounds__(XTile<T>::NT) void k_x_f_zeta(Grid g, cpx<T> *__res
 // (a0, a1), its k = 0 mode into dc; modes beyond the 2/3 rule set to zero;
 // then the inverse x pass of each projected component, in place.
 template <typename T, int L>
-__global__ __launch_bounds__(XTile<T>::NT) void k_x_slip(Grid g, cpx<T> *__restrict__ f0, cpx<T> *__restrict__ f1,
-                                                        cpx<T> *__restrict__ f2, cpx<T> *__restrict__ a0,
-                                                        cpx<T> *__restrict__ a1, double *__restrict__ dc,
-                                                        const int *__restrict__ skip) {
-    constexpr int NT  = XTile<T>::NT;
-    constexpr int C   = XTile<T>::C;
-    constexpr int BS  = ColStride<T, C>::value;
-    constexpr int NPT = (C * L + NT - 1) / NT;
+__global__ __launch_bounds__((ColGeom<T, L>::NT)) void k_x_slip(Grid g, cpx<T> *__restrict__ f0, cpx<T> *__restrict__ f1,
+                                                              cpx<T> *__restrict__ f2, cpx<T> *__restrict__ a0,
+                                                              cpx<T> *__restrict__ a1, double *__restrict__ dc,
+                                                              const int *__restrict__ skip) {
+    using Ff = ColFft<T, L, true, true>;
+    using Fi = ColFft<T, L, false, false>;
+    static_assert(Ff::RN == Fi::R0, "forward output layout must be the inverse input layout");
     if (skip && *skip) return;
-    __shared__ cpx<T> s[L * BS], tw[L];
-    fill_twiddles<T, L, NT>(tw);
-    const int ntiles = (g.trn_z + C - 1) / C;
-    const int o = blockIdx.x / ntiles, kz0 = (blockIdx.x - o * ntiles) * C;
-    const int j = kept_index(o, g.ny, g.trn_y), iky = (j > g.hny) ? j - g.ny : j;
-    const long long lstride = (long long)g.ny * g.nzp;
-    const long long base    = (long long)j * g.nzp + kz0;
-    cpx<T>         *F[3]    = {f0, f1, f2};
-    cpx<T>          Fh[3][NPT];
-    for (int d = 0; d < 3; d++) {
-        cpx<T> v[NPT];
+    __shared__ cpx<T> s[Ff::BUF], twf[Ff::TW], twi[Fi::TW];
+    const XTile<T, L> t(g);
+    cpx<T>           *F[3] = {f0, f1, f2};
+    cpx<T>            Fh[3][Ff::E];
 #pragma unroll
-        for (int i = 0; i < NPT; i++) {
-            const int e = threadIdx.x + i * NT;
-            const int n = e / C, c = e - n * C;
-            v[i]        = (e < C * L && kz0 + c < g.trn_z) ? F[d][base + n * lstride + c] : cmk((T)0, (T)0);
-        }
+    for (int d = 0; d < 3; d++)
 #pragma unroll
-        for (int i = 0; i < NPT; i++) {
-            const int e = threadIdx.x + i * NT;
-            if (e < C * L) s[(e / C) * BS + e % C] = v[i];
-        }
-        __syncthreads();
-        fft_cols_ip<T, L, C, BS, NT, true>(s, tw);
+        for (int i = 0; i < Ff::E; i++)
+            Fh[d][i] = t.ok ? at(F[d], t.elem(Ff::in_point(t.l, i))) : cmk((T)0, (T)0);
+    Ff::fill_tw(twf);  // while the loads are in flight
+    Fi::fill_tw(twi);
 #pragma unroll
-        for (int i = 0; i < NPT; i++) {
-            const int p = threadIdx.x + i * NT;
-            if (p < C * L) Fh[d][i] = s[(p / C) * BS + p % C];
-        }
-        __syncthreads();
-    }
+    for (int d = 0; d < 3; d++) Ff::run(Fh[d], s, twf, t.l, t.c());
 #pragma unroll
-    for (int i = 0; i < NPT; i++) {
-        const int p = threadIdx.x + i * NT;
-        if (p >= C * L) continue;
-        const int n = p / C, c = p - n * C, kz = kz0 + c;
-        const int ikx = (n > g.hnx) ? n - g.nx : n;
-        if (kz >= g.trn_z) continue;
-        if (!kept1(ikx, g.trn_x)) {
+    for (int i = 0; i < Ff::E; i++) {
+        const int n = Ff::out_point(t.l, i), ikx = t.ikx(n), iky = t.iky, kz = t.kz;
+        if (!t.kept(g, n)) {
             Fh[0][i] = Fh[1][i] = Fh[2][i] = cmk((T)0, (T)0);
             continue;
         }
-        const long long idx = base + n * lstride + c;
+        const unsigned idx = t.elem(n);
         const double    kx = ikx * g.wave_x, ky = iky * g.wave_y, kzz = kz * g.wave_z;
         const double    K2  = (g.wave_x * ikx) * (g.wave_x * ikx) + (g.wave_y * iky) * (g.wave_y * iky) +
                           (g.wave_z * kz) * (g.wave_z * kz);
@@ -486,24 +455,16 @@ __global__ __launch_bounds__(XTile<T>::NT) void k_x_slip(Grid g, cpx<T> *__restr
             c0 = 0;
             c1 = 1;
         }
-        a0[idx] = cmk((T)ore[c0], (T)oim[c0]);
-        a1[idx] = cmk((T)ore[c1], (T)oim[c1]);
+        at(a0, idx) = cmk((T)ore[c0], (T)oim[c0]);
+        at(a1, idx) = cmk((T)ore[c1], (T)oim[c1]);
+        __builtin_amdgcn_sched_barrier(0);  // one mode's FP64 temporaries at a time
     }
+#pragma unroll
     for (int d = 0; d < 3; d++) {
+        Fi::run(Fh[d], s, twi, t.l, t.c());
 #pragma unroll
-        for (int i = 0; i < NPT; i++) {
-            const int p = threadIdx.x + i * NT;
-            if (p < C * L) s[(p / C) * BS + p % C] = Fh[d][i];
-        }
-        __syncthreads();
-        fft_cols_ip<T, L, C, BS, NT, false>(s, tw);
-#pragma unroll
-        for (int i = 0; i < NPT; i++) {
-            const int e = threadIdx.x + i * NT;
-            const int n = e / C, c = e - n * C;
-            if (e < C * L && kz0 + c < g.trn_z) F[d][base + n * lstride + c] = s[n * BS + c];
-        }
-        __syncthreads();
+        for (int i = 0; i < Fi::E; i++)
+            if (t.ok) at(F[d], t.elem(Fi::out_point(t.l, i))) = Fh[d][i];
     }
 }
 
@@ -544,16 +505,17 @@ __global__ void k_zeta_add(Grid g, cpx<T> *__restrict__ z0, cpx<T> *__restrict__
 #define KH_FOR_EACH_L(X) X(8) X(12) X(16) X(24) X(32) X(48) X(64) X(96) X(128) X(192) X(256) X(384) X(512)
 
 static inline int nky(const Grid &g) { return 2 * g.trn_y - 1; }
+// kz tiles of a column pass over lines of L points
+template <typename T, int L>
+static inline int ktiles(const Grid &g) { return (g.trn_z + ColGeom<T, L>::C - 1) / ColGeom<T, L>::C; }
 
 template <typename T, bool FWD>
 hipError_t cols_y(const Grid &g, const Comps<T> &data, int ncomp, int in_mask, int out_mask, hipStream_t s,
                   const int *skip) {
-    constexpr int C  = ColTile<T>::C;
-    const int     nt = (g.trn_z + C - 1) / C;
     switch (g.ny) {
 #define KH_CASE(n)                                                                                                 \
     case n:                                                                                                        \
-        hipLaunchKernelGGL((k_cols<T, n, FWD, false>), dim3(g.nx * nt, ncomp, batch_z(g)), dim3(PassThreads<T>::value), 0, s, \
+        hipLaunchKernelGGL((k_cols<T, n, FWD, false>), dim3(g.nx * ktiles<T, n>(g), ncomp, batch_z(g)), dim3(ColGeom<T, n>::NT), 0, s, \
                            data, g, g.trn_z, in_mask, out_mask, skip);                                             \
         return hipGetLastError();
         KH_FOR_EACH_L(KH_CASE)
@@ -564,12 +526,10 @@ hipError_t cols_y(const Grid &g, const Comps<T> &data, int ncomp, int in_mask, i
 
 template <typename T, bool FWD>
 hipError_t cols_x(const Grid &g, const Comps<T> &data, int ncomp, int in_mask, int out_mask, hipStream_t s) {
-    constexpr int C  = ColTile<T>::C;
-    const int     nt = (g.trn_z + C - 1) / C;
     switch (g.nx) {
 #define KH_CASE(n)                                                                                                  \
     case n:                                                                                                         \
-        hipLaunchKernelGGL((k_cols<T, n, FWD, true>), dim3(nky(g) * nt, ncomp, batch_z(g)), dim3(PassThreads<T>::value), 0, s, \
+        hipLaunchKernelGGL((k_cols<T, n, FWD, true>), dim3(nky(g) * ktiles<T, n>(g), ncomp, batch_z(g)), dim3(ColGeom<T, n>::NT), 0, s, \
                            data, g, g.trn_z, in_mask, out_mask, nullptr);                                           \
         return hipGetLastError();
         KH_FOR_EACH_L(KH_CASE)
@@ -581,12 +541,10 @@ hipError_t cols_x(const Grid &g, const Comps<T> &data, int ncomp, int in_mask, i
 template <typename T>
 hipError_t x_zeta2u_inv(const Grid &g, const cpx<T> *z0, const cpx<T> *z1, cpx<T> *const u[3], double *ukdc,
                         int fixmask, hipStream_t s) {
-    constexpr int C  = XZTile<T>::C;
-    const int     nt = (g.trn_z + C - 1) / C;
     switch (g.nx) {
 #define KH_CASE(n)                                                                                                   \
     case n:                                                                                                          \
-        hipLaunchKernelGGL((k_x_zeta2u_inv<T, n>), dim3(nky(g) * nt, 1, batch_z(g)), dim3(XZTile<T>::NT), 0, s, g, z0, z1, u[0], u[1],    \
+        hipLaunchKernelGGL((k_x_zeta2u_inv<T, n>), dim3(nky(g) * ktiles<T, n>(g), 1, batch_z(g)), dim3(ColGeom<T, n>::NT), 0, s, g, z0, z1, u[0], u[1],    \
                            u[2], ukdc, fixmask);                                                                     \
         return hipGetLastError();
         KH_FOR_EACH_L(KH_CASE)
@@ -608,15 +566,13 @@ hipError_t z_force(const Grid &g, T *const up[3], T *phis, T *const us[3], cpx<T
 }
 
 template <typename T>
-hipError_t x_adv_ns(const Grid &g, const Comps<T> &prod, cpx<T> *z0, cpx<T> *z1, double dmy0, double dmy1,
-                    hipStream_t s) {
-    constexpr int C  = XTile<T>::C;
-    const int     nt = (g.trn_z + C - 1) / C;
+hipError_t x_ns_u(const Grid &g, const Comps<T> &prod, cpx<T> *z0, cpx<T> *z1, cpx<T> *const u[3], double *ukdc,
+                  double dmy0, double dmy1, int fixmask, hipStream_t s) {
     switch (g.nx) {
 #define KH_CASE(n)                                                                                                   \
     case n:                                                                                                          \
-        hipLaunchKernelGGL((k_x_adv_ns<T, n>), dim3(nky(g) * nt, 1, batch_z(g)), dim3(XTile<T>::NT), 0, s, g, prod, z0, z1, \
-                           dmy0, dmy1);                                                                              \
+        hipLaunchKernelGGL((k_x_ns_u<T, n>), dim3(nky(g) * ktiles<T, n>(g), 1, batch_z(g)), dim3(ColGeom<T, n>::NT), 0, s, g, prod, z0, z1, \
+                           u[0], u[1], u[2], ukdc, dmy0, dmy1, fixmask);                                             \
         return hipGetLastError();
         KH_FOR_EACH_L(KH_CASE)
 #undef KH_CASE
@@ -626,12 +582,10 @@ hipError_t x_adv_ns(const Grid &g, const Comps<T> &prod, cpx<T> *z0, cpx<T> *z1,
 
 template <typename T>
 hipError_t x_f_zeta(const Grid &g, cpx<T> *const f[3], cpx<T> *z0, cpx<T> *z1, double *ukdc, hipStream_t s) {
-    constexpr int C  = XTile<T>::C;
-    const int     nt = (g.trn_z + C - 1) / C;
     switch (g.nx) {
 #define KH_CASE(n)                                                                                                 \
     case n:                                                                                                        \
-        hipLaunchKernelGGL((k_x_f_zeta<T, n>), dim3(nky(g) * nt, 1, batch_z(g)), dim3(XTile<T>::NT), 0, s, g, f[0], f[1], f[2], z0, z1, \
+        hipLaunchKernelGGL((k_x_f_zeta<T, n>), dim3(nky(g) * ktiles<T, n>(g), 1, batch_z(g)), dim3(ColGeom<T, n>::NT), 0, s, g, f[0], f[1], f[2], z0, z1, \
                            ukdc);                                                                                  \
         return hipGetLastError();
         KH_FOR_EACH_L(KH_CASE)
@@ -643,12 +597,10 @@ hipError_t x_f_zeta(const Grid &g, cpx<T> *const f[3], cpx<T> *z0, cpx<T> *z1, d
 template <typename T>
 hipError_t x_slip(const Grid &g, cpx<T> *const f[3], cpx<T> *a0, cpx<T> *a1, double *dc, const int *skip,
                   hipStream_t s) {
-    constexpr int C  = XTile<T>::C;
-    const int     nt = (g.trn_z + C - 1) / C;
     switch (g.nx) {
 #define KH_CASE(n)                                                                                                  \
     case n:                                                                                                         \
-        hipLaunchKernelGGL((k_x_slip<T, n>), dim3(nky(g) * nt), dim3(XTile<T>::NT), 0, s, g, f[0], f[1], f[2], a0, a1, \
+        hipLaunchKernelGGL((k_x_slip<T, n>), dim3(nky(g) * ktiles<T, n>(g)), dim3(ColGeom<T, n>::NT), 0, s, g, f[0], f[1], f[2], a0, a1, \
                            dc, skip);                                                                               \
         return hipGetLastError();
         KH_FOR_EACH_L(KH_CASE)
@@ -684,7 +636,8 @@ hipError_t zeta_clean(const Grid &g, cpx<T> *z0, cpx<T> *z1, hipStream_t s) {
     template hipError_t x_slip<T>(const Grid &, cpx<T> *const[3], cpx<T> *, cpx<T> *, double *, const int *,          \
                                   hipStream_t);                                                                    \
     template hipError_t x_f_zeta<T>(const Grid &, cpx<T> *const[3], cpx<T> *, cpx<T> *, double *, hipStream_t);    \
-    template hipError_t x_adv_ns<T>(const Grid &, const Comps<T> &, cpx<T> *, cpx<T> *, double, double, hipStream_t); \
+    template hipError_t x_ns_u<T>(const Grid &, const Comps<T> &, cpx<T> *, cpx<T> *, cpx<T> *const[3], double *,    \
+                                  double, double, int, hipStream_t);                                               \
     template hipError_t zeta_clean<T>(const Grid &, cpx<T> *, cpx<T> *, hipStream_t);                               \
     template hipError_t zeta_add<T>(const Grid &, cpx<T> *, cpx<T> *, const cpx<T> *, const cpx<T> *, double *,      \
                                     const double *, hipStream_t);

@@ -49,4 +49,48 @@ __device__ __forceinline__ void slaved_euler_mode(const Grid &g, int ikx, int ik
     x1               = cmk((T)nx1, (T)ny1);
 }
 
+// The same update with the products arriving one at a time: acc[0], acc[1]
+// gather the two rows of -Omega that the mode stores,
+// acc[r] += M[c_r][Q] p_Q (slaved_euler_mode's om is -M p), in FP64.
+template <int Q, typename T>
+__device__ __forceinline__ void adv_fold(const Grid &g, int ikx, int iky, int kz, cpx<T> p, cpx<double> *acc) {
+    const double k1 = ikx * g.wave_x, k2 = iky * g.wave_y, k3 = kz * g.wave_z;
+    double       m0, m1, m2;
+    if constexpr (Q == 0) {
+        m0 = (k3 - k2) * (k3 + k2);
+        m1 = k1 * k2;
+        m2 = -(k3 * k1);
+    } else if constexpr (Q == 1) {
+        m0 = -(k1 * k2);
+        m1 = (k1 - k3) * (k1 + k3);
+        m2 = k2 * k3;
+    } else if constexpr (Q == 2) {
+        m0 = k3 * k1;
+        m1 = -(k2 * k3);
+        m2 = (k2 - k1) * (k2 + k1);
+    } else if constexpr (Q == 3) {
+        m0 = k2 * k3;
+        m1 = 0.0;
+        m2 = -(k1 * k2);
+    } else {
+        m0 = 0.0;
+        m1 = k3 * k1;
+        m2 = -(k1 * k2);
+    }
+    const double a = ikx != 0 ? m1 : iky != 0 ? m2 : m0, b = ikx != 0 ? m2 : iky != 0 ? m0 : m1;
+    acc[0]         = {acc[0].x + a * (double)p.x, acc[0].y + a * (double)p.y};
+    acc[1]         = {acc[1].x + b * (double)p.x, acc[1].y + b * (double)p.y};
+}
+template <typename T>
+__device__ __forceinline__ void slaved_euler_acc(const Grid &g, int ikx, int iky, int kz, const cpx<double> *acc,
+                                                 double dmy0, double dmy1, cpx<T> &x0, cpx<T> &x1) {
+    const double K2 = (g.wave_x * ikx) * (g.wave_x * ikx) + (g.wave_y * iky) * (g.wave_y * iky) +
+                      (g.wave_z * kz) * (g.wave_z * kz);
+    const double IK2 = (K2 > 0.0) ? 1. / K2 : 0.0, dmy = exp(dmy0 * K2) - 1., w = dmy1 * IK2;
+    x0 = cmk((T)((double)x0.x + dmy * ((double)x0.x + w * acc[0].x)),
+             (T)((double)x0.y + dmy * ((double)x0.y + w * acc[0].y)));
+    x1 = cmk((T)((double)x1.x + dmy * ((double)x1.x + w * acc[1].x)),
+             (T)((double)x1.y + dmy * ((double)x1.y + w * acc[1].y)));
+}
+
 }  // namespace kh

@@ -564,14 +564,10 @@ struct Step {
         KH_LAUNCH("y_inv", (cols_y<T, false>(g, c5, 3, 1, 0, s)));
         KH_LAUNCH("z_adv", (z_adv<T>(g, s3, q5, s)));
         KH_LAUNCH("y_fwd_adv", (cols_y<T, true>(g, cq5, 5, 0, 1, s)));
-        if constexpr (sizeof(T) == 8) {  // forward x + slaved Euler in one pass
-            KH_LAUNCH("x_adv_ns", (x_adv_ns<T>(g, cq5, Z(r, 0), Z(r, 1), -r->nu * r->jikan.dt_fluid, 1. / r->nu, s)));
-        } else {  // FP32: the split passes keep more workgroups resident
-            KH_LAUNCH("x_fwd_adv", (cols_x<T, true>(g, cq5, 5, 0, 1, s)));
-            KH_LAUNCH("adv_ns", (adv_ns<T>(g, q5, Z(r, 0), Z(r, 1), -r->nu * r->jikan.dt_fluid, 1. / r->nu, s)));
-        }
-        // FIX_CELL, truncation, Zeta_k2u -> u* in real space
-        KH_LAUNCH("x_zeta2u_inv", (x_zeta2u_inv<T>(g, Z(r, 0), Z(r, 1), s3, r->ukdc, r->fixmask, s)));
+        // forward x, slaved Euler, FIX_CELL, truncation, Zeta_k2u, inverse x
+        KH_LAUNCH("x_ns_u", (x_ns_u<T>(g, cq5, Z(r, 0), Z(r, 1), s3, r->ukdc, -r->nu * r->jikan.dt_fluid, 1. / r->nu,
+                                       r->fixmask, s)));
+        // u* in real space
         KH_LAUNCH("y_inv", (cols_y<T, false>(g, c5, 3, 1, 0, s)));
         ZIO<T> zio{{S(r, 0), S(r, 1), S(r, 2)}, {U(r, 0), U(r, 1), U(r, 2)}};
         KH_LAUNCH("z_c2r", (fft_z_c2r_multi<T>(g, zio, 3, s, g.trn_z, mask, occ)));
