@@ -21,8 +21,8 @@ template <typename T, bool FWD>
 hipError_t cols_x(const Grid &g, const Comps<T> &data, int ncomp, int in_mask, int out_mask, hipStream_t s);
 // zeta -> u_hat (truncated) -> inverse x pass, 3 components
 template <typename T>
-hipError_t x_zeta2u_inv(const Grid &g, const cpx<T> *z0, const cpx<T> *z1, cpx<T> *const u[3], double *ukdc,
-                        int fixmask, hipStream_t s);
+hipError_t x_zeta2u_inv(const Grid &g, const cpx<T> *z0, const cpx<T> *z1, cpx<T> *const u[3], const double *ukdc,
+                        hipStream_t s);
 // inverse z (3) -> products -> forward z (5); p5[2] may be s3[0], p5[1]
 // s3[2] and p5[0] s3[1] (and no other aliasing)
 template <typename T>

@@ -149,12 +149,11 @@ __device__ __forceinline__ void zeta_to_uhat(const Grid &g, int ikx, int iky, in
 }
 
 // zeta -> u_hat (3 components) on the kept (ky,kz) columns, then the
-// inverse x pass of each component. fixmask: FIX_CELL zeroing of uk_dc
-// (sp_3d_ns.cxx:46-52), done by the block holding (ky,kz) = (0,0).
+// inverse x pass of each component.
 template <typename T, int L>
 __global__ __launch_bounds__((ColGeom<T, L>::NT)) void k_x_zeta2u_inv(
     Grid g, const cpx<T> *__restrict__ z0, const cpx<T> *__restrict__ z1, cpx<T> *__restrict__ u0,
-    cpx<T> *__restrict__ u1, cpx<T> *__restrict__ u2, double *__restrict__ ukdc, int fixmask) {
+    cpx<T> *__restrict__ u1, cpx<T> *__restrict__ u2, const double *__restrict__ ukdc) {
     using F = ColFft<T, L, false, false>;
     if (batch_skip(g)) return;
     z0 = brun(z0, g), z1 = brun(z1, g), u0 = brun(u0, g), u1 = brun(u1, g), u2 = brun(u2, g);
@@ -171,11 +170,7 @@ __global__ __launch_bounds__((ColGeom<T, L>::NT)) void k_x_zeta2u_inv(
         D2[i]         = ok ? at(z1, t.elem(n)) : cmk((T)0, (T)0);
     }
     F::fill_tw(tw);
-    if (threadIdx.x < 3) {
-        const bool fixed = fixmask & (1 << threadIdx.x);
-        uk[threadIdx.x]  = fixed ? 0.0 : ukdc[threadIdx.x];
-        if (fixed && t.first()) ukdc[threadIdx.x] = 0.0;
-    }
+    if (threadIdx.x < 3) uk[threadIdx.x] = ukdc[threadIdx.x];
     __syncthreads();
     cpx<T> U[3][F::E];
 #pragma unroll
@@ -539,13 +534,13 @@ hipError_t cols_x(const Grid &g, const Comps<T> &data, int ncomp, int in_mask, i
 }
 
 template <typename T>
-hipError_t x_zeta2u_inv(const Grid &g, const cpx<T> *z0, const cpx<T> *z1, cpx<T> *const u[3], double *ukdc,
-                        int fixmask, hipStream_t s) {
+hipError_t x_zeta2u_inv(const Grid &g, const cpx<T> *z0, const cpx<T> *z1, cpx<T> *const u[3], const double *ukdc,
+                        hipStream_t s) {
     switch (g.nx) {
 #define KH_CASE(n)                                                                                                   \
     case n:                                                                                                          \
         hipLaunchKernelGGL((k_x_zeta2u_inv<T, n>), dim3(nky(g) * ktiles<T, n>(g), 1, batch_z(g)), dim3(ColGeom<T, n>::NT), 0, s, g, z0, z1, u[0], u[1],    \
-                           u[2], ukdc, fixmask);                                                                     \
+                           u[2], ukdc);                                                                     \
         return hipGetLastError();
         KH_FOR_EACH_L(KH_CASE)
 #undef KH_CASE
@@ -628,8 +623,8 @@ hipError_t zeta_clean(const Grid &g, cpx<T> *z0, cpx<T> *z1, hipStream_t s) {
     template hipError_t cols_y<T, false>(const Grid &, const Comps<T> &, int, int, int, hipStream_t, const int *);  \
     template hipError_t cols_x<T, true>(const Grid &, const Comps<T> &, int, int, int, hipStream_t);                \
     template hipError_t cols_x<T, false>(const Grid &, const Comps<T> &, int, int, int, hipStream_t);               \
-    template hipError_t x_zeta2u_inv<T>(const Grid &, const cpx<T> *, const cpx<T> *, cpx<T> *const[3], double *,   \
-                                        int, hipStream_t);                                                          \
+    template hipError_t x_zeta2u_inv<T>(const Grid &, const cpx<T> *, const cpx<T> *, cpx<T> *const[3],              \
+                                        const double *, hipStream_t);                                                          \
     template hipError_t z_adv<T>(const Grid &, cpx<T> *const[3], cpx<T> *const[5], hipStream_t);                   \
     template hipError_t z_force<T>(const Grid &, T *const[3], T *, T *const[3], cpx<T> *const[3], int, int *,          \
                                    hipStream_t, T *const[3], const int *, Occ);                                    \

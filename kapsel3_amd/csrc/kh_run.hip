@@ -560,7 +560,7 @@ struct Step {
         cpx<T>  *q5[5] = {S(r, 1), S(r, 2), S(r, 0), S(r, 4), S(r, 3)};
         Comps<T> cq5{{q5[0], q5[1], q5[2], q5[3], q5[4]}};
         // NS_solver_slavedEuler: zeta -> u -> products -> -Omega -> slaved Euler
-        KH_LAUNCH("x_zeta2u_inv", (x_zeta2u_inv<T>(g, Z(r, 0), Z(r, 1), s3, r->ukdc, 0, s)));
+        KH_LAUNCH("x_zeta2u_inv", (x_zeta2u_inv<T>(g, Z(r, 0), Z(r, 1), s3, r->ukdc, s)));
         KH_LAUNCH("y_inv", (cols_y<T, false>(g, c5, 3, 1, 0, s)));
         KH_LAUNCH("z_adv", (z_adv<T>(g, s3, q5, s)));
         KH_LAUNCH("y_fwd_adv", (cols_y<T, true>(g, cq5, 5, 0, 1, s)));

@@ -26,10 +26,13 @@ struct WaveLane {
     bool      okA, okB;
     int       pitch;  // spectral row pitch (complex elements)
     cpx<T>   *buf;    // this line's LDS strip
-    __device__ __forceinline__ WaveLane(cpx<T> *strips, long long nrows, int pitch_) : pitch(pitch_) {
+    // SPLIT: every wavefront of the workgroup holds the same W lines (each
+    // does its own component of them)
+    __device__ __forceinline__ WaveLane(cpx<T> *strips, long long nrows, int pitch_, bool split = false)
+        : pitch(pitch_) {
         const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, w = lane / Geo::G;
         g              = lane - w * Geo::G;
-        line           = ((long long)blockIdx.x * (Geo::NT / 64) + wv) * Geo::W + w;
+        line           = (split ? (long long)blockIdx.x : (long long)blockIdx.x * (Geo::NT / 64) + wv) * Geo::W + w;
         okA            = 2 * line < nrows;
         okB            = 2 * line + 1 < nrows;
         buf            = strips + (wv * Geo::W + w) * Geo::LP;
@@ -202,7 +205,7 @@ __global__ __launch_bounds__(256) void k_zw_c2r_masked(ZIO<T> io, int ncomp, con
         }
     }
 #pragma unroll 1
-    for (int c = 0; c < ncomp; c++) {
+    for (int c = blockIdx.y; c < ncomp; c += gridDim.y) {
         cpx<T> v[F::E];
         load_pair<T, L, F>(brun(io.in[c], bg), wl, kzv, v);
         F::run(v, wl.buf, tw, wl.g);
@@ -397,6 +400,48 @@ __global__ __launch_bounds__(256) void k_zw_adv(Grid g, const cpx<T> *__restrict
     store_pair<T, L, Ff>(v, wl, kzv, p3);
 }
 
+// The same pass with the work of a line split over five wavefronts: three
+// invert a component each and leave it in their LDS strips, then each of the five
+// forms one product and transforms it. A line's chain is two transforms long
+// instead of eight.
+template <typename T, int L, int E>
+__global__ __launch_bounds__(320) void k_zw_adv_split(Grid g, Comps<T> in, Comps<T> out, T scale) {
+    using Geo = WaveGeom<T, L, E>;
+    using Fi  = WaveFft<T, L, E, false, false>;
+    using Ff  = WaveFft<T, L, E, true, true>;
+    static_assert(Geo::LP >= L, "a strip set holds a wavefront's registers");
+    if (batch_skip(g)) return;
+    __shared__ cpx<T> twi[Fi::TW], twf[Ff::TW], strips[5 * Geo::W * Geo::LP];
+    const WaveLane<T, L, E> wl(strips, (long long)g.nx * g.ny, g.nzp, true);
+    const int               q    = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int               kzv  = g.trn_z;
+    auto                    held = [&](int c) { return strips + c * (Geo::W * Geo::LP) + lane; };
+    cpx<T>                  v[E];
+    if (q < 3) load_pair<T, L, Fi>(brun(in.p[q], g), wl, kzv, v);
+    Fi::template fill_tw<320>(twi);
+    Ff::template fill_tw<320>(twf);
+    __syncthreads();
+    if (q < 3) {
+        Fi::run(v, wl.buf, twi, wl.g);
+        wave_sync();
+        cpx<T> *h = held(q);
+#pragma unroll
+        for (int i = 0; i < E; i++) h[64 * i] = cscale(v[i], scale);
+    }
+    __syncthreads();
+    {  // u2u3, u3u1, u1u2, u2^2 - u3^2, u3^2 - u1^2
+        const cpx<T> *a = held(q == 2 ? 0 : q == 0 || q == 3 ? 1 : 2), *b = held(q == 2 ? 1 : q == 0 || q == 3 ? 2 : 0);
+#pragma unroll
+        for (int i = 0; i < E; i++) {
+            const cpx<T> x = a[64 * i], y = b[64 * i];
+            v[i] = q < 3 ? cmk(x.x * y.x, x.y * y.y) : cmk((x.x - y.x) * (x.x + y.x), (x.y - y.y) * (x.y + y.y));
+        }
+    }
+    __syncthreads();  // the strips are free again
+    Ff::run(v, wl.buf, twf, wl.g);
+    store_pair<T, L, Ff>(v, wl, kzv, brun(out.p[q], g));
+}
+
 // Rigidity force f = up - min(phi_sum, 1) u* (Make_f_particle_dt_nonsole,
 // f_particle.h:35-54; make_phi.cxx:248-259), forward z per component. With
 // us2, u* = us + us2 (the squirmer step's u after the slip iteration, formed
@@ -405,9 +450,11 @@ __global__ __launch_bounds__(256) void k_zw_adv(Grid g, const cpx<T> *__restrict
 // iteration, nonzero on the whole shell |r - a| < xi/2, also where phi has
 // underflowed to 0). clear: bit 0 leaves up zero, bit 1 phi_sum (with
 // phis). A nonzero *skip makes the launch do nothing.
-template <typename T, int L, int E>
-__global__ __launch_bounds__(256) void k_zw_force(Grid g, ZForceIO<T> io, int clear, int *__restrict__ tick,
-                                                  const int *__restrict__ skip) {
+// SPLIT: three wavefronts share a line, one component each.
+template <typename T, int L, int E, bool SPLIT>
+__global__ __launch_bounds__(SPLIT ? 192 : 256) void k_zw_force(Grid g, ZForceIO<T> io, int clear,
+                                                                int *__restrict__ tick,
+                                                                const int *__restrict__ skip) {
     using Geo = WaveGeom<T, L, E>;
     using Ff  = WaveFft<T, L, E, true, true>;
     using RS  = RowStage<T, L>;
@@ -417,12 +464,13 @@ __global__ __launch_bounds__(256) void k_zw_force(Grid g, ZForceIO<T> io, int cl
     // io stays as passed (a modified copy indexed by the loop's d would sit
     // in scratch); each pointer is moved to this block's run at use
     tick = brun(tick, g);
-    __shared__ cpx<T> tw[Ff::TW], strips[(Geo::NT / 64) * Geo::W * Geo::LP];
-    Ff::template fill_tw<Geo::NT>(tw);
+    constexpr int NT = SPLIT ? 192 : Geo::NT;
+    __shared__ cpx<T> tw[Ff::TW], strips[(NT / 64) * Geo::W * Geo::LP];
+    Ff::template fill_tw<NT>(tw);
     __syncthreads();
     if (tick && blockIdx.x == 0 && threadIdx.x == 0) *tick += 1;  // the step counter, after every reader
     const long long         nrows = (long long)g.nx * g.ny;
-    const WaveLane<T, L, E> wl(strips, nrows, g.nzp);
+    const WaveLane<T, L, E> wl(strips, nrows, g.nzp, SPLIT);
     const long long         oa = (2 * wl.line) * L, ob = oa + L;
     using vec                  = typename RS::vec;
     const vec zero             = {(T)0, (T)0, (T)0, (T)0};
@@ -440,10 +488,6 @@ __global__ __launch_bounds__(256) void k_zw_force(Grid g, ZForceIO<T> io, int cl
             na[t]       = wl.okA && occ_bit(ow, io.occ.words, 2 * wl.line, z >> 2);
             nb[t]       = wl.okB && occ_bit(ow, io.occ.words, 2 * wl.line + 1, z >> 2);
             pa[t] = pb[t] = zero;
-            if ((clear & 2) && phis) {
-                if (na[t]) RS::st(phis + oa + z, zero);
-                if (nb[t]) RS::st(phis + ob + z, zero);
-            }
             continue;
         }
         if (!phis) {  // no mask: up is read everywhere (f = up)
@@ -456,15 +500,21 @@ __global__ __launch_bounds__(256) void k_zw_force(Grid g, ZForceIO<T> io, int cl
         vec       a = wl.okA ? RS::ld(phis + oa + z) : zero, b = wl.okB ? RS::ld(phis + ob + z) : zero;
         na[t]       = nonzero(a);
         nb[t]       = nonzero(b);
-        if (clear & 2) {  // leave phi_sum zero for the next step's scatter
-            if (na[t]) RS::st(phis + oa + z, zero);
-            if (nb[t]) RS::st(phis + ob + z, zero);
-        }
         pa[t]       = {fmin(a.x, (T)1), fmin(a.y, (T)1), fmin(a.z, (T)1), fmin(a.w, (T)1)};
         pb[t]       = {fmin(b.x, (T)1), fmin(b.y, (T)1), fmin(b.z, (T)1), fmin(b.w, (T)1)};
     }
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (SPLIT) __syncthreads();  // every component has read the mask
+    if ((clear & 2) && phis && (!SPLIT || wave == 0)) {  // leave phi_sum zero for the next step's scatter
+#pragma unroll
+        for (int t = 0; t < NT4; t++) {
+            const int z = 4 * (wl.g + Geo::G * t);
+            if (na[t]) RS::st(phis + oa + z, zero);
+            if (nb[t]) RS::st(phis + ob + z, zero);
+        }
+    }
 #pragma unroll 1
-    for (int d = 0; d < 3; d++) {
+    for (int d = SPLIT ? wave : 0; d < (SPLIT ? wave + 1 : 3); d++) {
         T *const       UP  = brun(io.up[d], g);
         const T *const US  = brun(io.us[d], g), *const US2 = brun(io.us2[d], g);
         auto     ld_u = [&](long long o) -> vec {
@@ -496,7 +546,7 @@ __global__ __launch_bounds__(256) void k_zw_force(Grid g, ZForceIO<T> io, int cl
         Ff::run(v, wl.buf, tw, wl.g);
         store_pair<T, L, Ff>(v, wl, g.trn_z, brun(io.f[d], g));
     }
-    if (ow && (clear & 2)) {  // leave the bits zero for the next step's scatter
+    if (ow && (clear & 2) && (!SPLIT || wave == 0)) {  // leave the bits zero for the next step's scatter
 #pragma unroll
         for (int t = 0; t < NT4; t++) {
             const int v = wl.g + Geo::G * t;
@@ -552,6 +602,29 @@ static inline unsigned zw_blocks(long long nrows) {
     return (unsigned)((lines + WaveGeom<T, L, E>::LINES - 1) / WaveGeom<T, L, E>::LINES);
 }
 
+// workgroups of the split passes, W lines each
+template <typename T, int L, int E>
+static inline unsigned zw_blocks1(long long nrows) {
+    return (unsigned)(((nrows + 1) / 2 + WaveGeom<T, L, E>::W - 1) / WaveGeom<T, L, E>::W);
+}
+// The advection and inverse passes split a line's components over wavefronts
+// while the lines alone make few wavefronts (four a SIMD fill the chip with
+// one): 64^3 FP64 (256 wavefronts of lines) z_adv 17.6 -> 11.6 us and z_c2r 11.2 ->
+// 7.7, 64 x 96 x 192 (768) even, 128^3 (2048) z_adv 32 -> 41 us.
+template <typename T, int L, int E>
+static inline bool zw_split(long long nrows, unsigned nbatch) {
+    return (long long)zw_blocks1<T, L, E>(nrows) * nbatch <= 1024;
+}
+// The force pass splits in FP64, where the mask is one bit a vector, and at
+// the lengths with 12 points per lane, whose three components in turn take 110
+// to 180 registers: 256^3 FP64 140 -> 131 us, 192^3 mixed 44 -> 39 us, 64^3
+// FP64 13.5 -> 10.4; in FP32 powers of two it would read phi_sum three times
+// (256^3 mixed 78 -> 89 us), so there only small grids do.
+template <typename T, int L, int E>
+static inline bool zw_force_split(long long nrows, unsigned nbatch) {
+    return sizeof(T) == 8 || L % 3 == 0 || zw_split<T, L, E>(nrows, nbatch);
+}
+
 template <typename T>
 hipError_t zw_r2c(int L, const T *in, cpx<T> *out, long long nrows, int pitch, hipStream_t s, int kzv) {
     if (kzv < 0 || kzv > L / 2 + 1) kzv = L / 2 + 1;
@@ -577,7 +650,7 @@ hipError_t zw_c2r(int L, const ZIO<T> &io, int ncomp, long long nrows, T scale, 
         switch (L) {
 #define KH_CASE(n)                                                                                              \
     case n:                                                                                                     \
-        hipLaunchKernelGGL((k_zw_c2r_masked<T, n, ZwE<T, n>::pass>), dim3(zw_blocks<T, n, ZwE<T, n>::pass>(nrows), 1, batch_z(bg)), dim3(256), 0, s, io, ncomp, mask, nrows, scale, kzv, pitch, skip, bg, occ); \
+        hipLaunchKernelGGL((k_zw_c2r_masked<T, n, ZwE<T, n>::pass>), dim3(zw_blocks<T, n, ZwE<T, n>::pass>(nrows), zw_split<T, n, ZwE<T, n>::pass>(nrows, batch_z(bg)) ? ncomp : 1, batch_z(bg)), dim3(256), 0, s, io, ncomp, mask, nrows, scale, kzv, pitch, skip, bg, occ); \
         return hipGetLastError();
             KH_FOR_EACH_WL(KH_CASE)
 #undef KH_CASE
@@ -613,9 +686,14 @@ hipError_t zw_c2r_cross(int L, const ZIO<T> &io, const T *const u[3], long long 
 template <typename T>
 hipError_t zw_adv(const Grid &g, cpx<T> *const s3[3], cpx<T> *const p5[5], T scale, hipStream_t s) {
     const long long nrows = (long long)g.nx * g.ny;
+    const Comps<T>  in{{s3[0], s3[1], s3[2], nullptr, nullptr}}, out{{p5[0], p5[1], p5[2], p5[3], p5[4]}};
     switch (g.nz) {
 #define KH_CASE(n)                                                                                                \
     case n:                                                                                                       \
+        if (zw_split<T, n, ZwE<T, n>::adv>(nrows, batch_z(g))) {                                                  \
+            hipLaunchKernelGGL((k_zw_adv_split<T, n, ZwE<T, n>::adv>), dim3(zw_blocks1<T, n, ZwE<T, n>::adv>(nrows), 1, batch_z(g)), dim3(320), 0, s, g, in, out, scale); \
+            return hipGetLastError();                                                                             \
+        }                                                                                                         \
         hipLaunchKernelGGL((k_zw_adv<T, n, ZwE<T, n>::adv, ZwE<T, n>::live3>), dim3(zw_blocks<T, n, ZwE<T, n>::adv>(nrows), 1, batch_z(g)), dim3(256), 0, s, g, s3[0], s3[1], s3[2], \
                            p5[0], p5[1], p5[2], p5[3], p5[4], scale);                                             \
         return hipGetLastError();
@@ -642,7 +720,12 @@ hipError_t zw_force(const Grid &g, T *const up[3], T *phis, T *const us[3], cpx<
     switch (g.nz) {
 #define KH_CASE(n)                                                                                                  \
     case n:                                                                                                         \
-        hipLaunchKernelGGL((k_zw_force<T, n, ZwE<T, n>::force>), dim3(zw_blocks<T, n, ZwE<T, n>::force>(nrows), 1, batch_z(g)), dim3(256), 0, s, g, io, \
+        if (zw_force_split<T, n, ZwE<T, n>::force>(nrows, batch_z(g))) {                                            \
+            hipLaunchKernelGGL((k_zw_force<T, n, ZwE<T, n>::force, true>), dim3(zw_blocks1<T, n, ZwE<T, n>::force>(nrows), 1, batch_z(g)), dim3(192), 0, s, g, io, \
+                               clear, tick, skip);                                                                  \
+            return hipGetLastError();                                                                               \
+        }                                                                                                           \
+        hipLaunchKernelGGL((k_zw_force<T, n, ZwE<T, n>::force, false>), dim3(zw_blocks<T, n, ZwE<T, n>::force>(nrows), 1, batch_z(g)), dim3(256), 0, s, g, io, \
                            clear, tick, skip);                                                                      \
         return hipGetLastError();
         KH_FOR_EACH_WL(KH_CASE)
