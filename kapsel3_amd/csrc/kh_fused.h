@@ -44,9 +44,10 @@ hipError_t x_slip(const Grid &g, cpx<T> *const f[3], cpx<T> *a0, cpx<T> *a1, dou
 template <typename T>
 hipError_t x_ns_u(const Grid &g, const Comps<T> &prod, cpx<T> *z0, cpx<T> *z1, cpx<T> *const u[3], double *ukdc,
                   double dmy0, double dmy1, int fixmask, hipStream_t s);
-// forward x (3) -> projection + u* + curl -> zeta, uk_dc
+// forward x (3) -> projection + u* + curl -> zeta, uk_dc; next: also the next
+// step's x_zeta2u_inv, its three components in f
 template <typename T>
-hipError_t x_f_zeta(const Grid &g, cpx<T> *const f[3], cpx<T> *z0, cpx<T> *z1, double *ukdc, hipStream_t s);
+hipError_t x_f_zeta(const Grid &g, cpx<T> *const f[3], cpx<T> *z0, cpx<T> *z1, double *ukdc, bool next, hipStream_t s);
 // zeta += (a0, a1) at the kept modes, uk_dc += dc
 template <typename T>
 hipError_t zeta_add(const Grid &g, cpx<T> *z0, cpx<T> *z1, const cpx<T> *a0, const cpx<T> *a1, double *ukdc,

@@ -303,25 +303,31 @@ __global__ __launch_bounds__((ColGeom<T, L>::NT), (ColGeom<T, L>::WAVES)) void k
 // uk_dc += f_hat(0). With the lines in registers 94 to 146 of them instead of
 // 220, so two to three workgroups a CU: 512^3 mixed 1104 -> 381 us (3.5 TB/s),
 // 256^3 mixed 61 -> 52 us, FP64 83 -> 76 us (4.5 TB/s).
-template <typename T, int L>
-__global__ __launch_bounds__((ColGeom<T, L>::NT)) void k_x_f_zeta(Grid g, const cpx<T> *__restrict__ f0,
-                                                                const cpx<T> *__restrict__ f1,
-                                                                const cpx<T> *__restrict__ f2, cpx<T> *__restrict__ z0,
-                                                                cpx<T> *__restrict__ z1, double *__restrict__ ukdc) {
-    using F = ColFft<T, L, true, true>;
+// NEXT: another step follows in the same captured graph, and u_hat of the
+// new zeta is formed here and taken through the inverse x pass, in place of
+// f, instead of by that step's k_x_zeta2u_inv: the new zeta is not read back,
+// and a launch goes (the whole step: 192^3 mixed 324 -> 314 us, 64^3 FP64 88.3 ->
+// 86.0, 256^3 mixed 723 -> 712, 256^3 FP64 1272 -> 1257, 512^3 mixed 6.47 -> 6.36 ms).
+template <typename T, int L, bool NEXT>
+__global__ __launch_bounds__((ColGeom<T, L>::NT)) void k_x_f_zeta(Grid g, cpx<T> *f0, cpx<T> *f1, cpx<T> *f2,
+                                                                  cpx<T> *__restrict__ z0, cpx<T> *__restrict__ z1,
+                                                                  double *__restrict__ ukdc) {
+    using F  = ColFft<T, L, true, true>;
+    using Fi = ColFft<T, L, false, false>;
     if (batch_skip(g)) return;
     f0 = brun(f0, g), f1 = brun(f1, g), f2 = brun(f2, g), z0 = brun(z0, g), z1 = brun(z1, g), ukdc = brun(ukdc, g);
-    __shared__ cpx<T> s[F::BUF], tw[F::TW];
+    __shared__ cpx<T> s[F::BUF], tw[F::TW], twi[NEXT ? Fi::TW : 1];
     __shared__ double uk[3];
     const XTile<T, L> t(g);
-    const cpx<T>     *src[3] = {f0, f1, f2};
+    cpx<T>           *fld[3] = {f0, f1, f2};
     cpx<T>            Fh[3][F::E];
 #pragma unroll
     for (int d = 0; d < 3; d++)
 #pragma unroll
         for (int i = 0; i < F::E; i++)
-            Fh[d][i] = t.ok ? at(src[d], t.elem(F::in_point(t.l, i))) : cmk((T)0, (T)0);
+            Fh[d][i] = t.ok ? at(fld[d], t.elem(F::in_point(t.l, i))) : cmk((T)0, (T)0);
     F::fill_tw(tw);  // while the loads are in flight
+    if constexpr (NEXT) Fi::fill_tw(twi);
     if (threadIdx.x < 3) uk[threadIdx.x] = ukdc[threadIdx.x];
     __syncthreads();
 #pragma unroll
@@ -329,7 +335,10 @@ __global__ __launch_bounds__((ColGeom<T, L>::NT)) void k_x_f_zeta(Grid g, const 
 #pragma unroll
     for (int i = 0; i < F::E; i++) {
         const int n = F::out_point(t.l, i), ikx = t.ikx(n), iky = t.iky, kz = t.kz;
-        if (!t.kept(g, n)) continue;
+        if (!t.kept(g, n)) {
+            if constexpr (NEXT) Fh[0][i] = Fh[1][i] = Fh[2][i] = cmk((T)0, (T)0);
+            continue;
+        }
         const unsigned idx = t.elem(n);
         const double    kx = ikx * g.wave_x, ky = iky * g.wave_y, kzz = kz * g.wave_z;
         const double    K2  = (g.wave_x * ikx) * (g.wave_x * ikx) + (g.wave_y * iky) * (g.wave_y * iky) +
@@ -370,9 +379,27 @@ __global__ __launch_bounds__((ColGeom<T, L>::NT)) void k_x_f_zeta(Grid g, const 
             c0 = 0;
             c1 = 1;
         }
-        at(z0, idx) = cmk((T)ore[c0], (T)oim[c0]);
-        at(z1, idx) = cmk((T)ore[c1], (T)oim[c1]);
+        const cpx<T> x0 = cmk((T)ore[c0], (T)oim[c0]), x1 = cmk((T)ore[c1], (T)oim[c1]);
+        at(z0, idx) = x0;
+        at(z1, idx) = x1;
+        if constexpr (NEXT) {
+            const double un[3] = {uk[0] + fr[0], uk[1] + fr[1], uk[2] + fr[2]};  // uk_dc, read for k = 0 only
+            cpx<T>       u[3];
+            zeta_to_uhat<T>(g, ikx, iky, kz, x0, x1, un, u);
+            Fh[0][i] = u[0];
+            Fh[1][i] = u[1];
+            Fh[2][i] = u[2];
+        }
         __builtin_amdgcn_sched_barrier(0);  // one mode's FP64 temporaries at a time
+    }
+    if constexpr (NEXT) {
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            Fi::run(Fh[d], s, twi, t.l, t.c());
+#pragma unroll
+            for (int i = 0; i < Fi::E; i++)
+                if (t.ok) at(fld[d], t.elem(Fi::out_point(t.l, i))) = Fh[d][i];
+        }
     }
 }
 
@@ -576,13 +603,17 @@ hipError_t x_ns_u(const Grid &g, const Comps<T> &prod, cpx<T> *z0, cpx<T> *z1, c
 }
 
 template <typename T>
-hipError_t x_f_zeta(const Grid &g, cpx<T> *const f[3], cpx<T> *z0, cpx<T> *z1, double *ukdc, hipStream_t s) {
+hipError_t x_f_zeta(const Grid &g, cpx<T> *const f[3], cpx<T> *z0, cpx<T> *z1, double *ukdc, bool next, hipStream_t s) {
     switch (g.nx) {
 #define KH_CASE(n)                                                                                                 \
-    case n:                                                                                                        \
-        hipLaunchKernelGGL((k_x_f_zeta<T, n>), dim3(nky(g) * ktiles<T, n>(g), 1, batch_z(g)), dim3(ColGeom<T, n>::NT), 0, s, g, f[0], f[1], f[2], z0, z1, \
-                           ukdc);                                                                                  \
-        return hipGetLastError();
+    case n: {                                                                                                      \
+        const dim3 grid(nky(g) * ktiles<T, n>(g), 1, batch_z(g)), block(ColGeom<T, n>::NT);                        \
+        if (next)                                                                                                  \
+            hipLaunchKernelGGL((k_x_f_zeta<T, n, true>), grid, block, 0, s, g, f[0], f[1], f[2], z0, z1, ukdc);    \
+        else                                                                                                       \
+            hipLaunchKernelGGL((k_x_f_zeta<T, n, false>), grid, block, 0, s, g, f[0], f[1], f[2], z0, z1, ukdc);   \
+        return hipGetLastError();                                                                                  \
+    }
         KH_FOR_EACH_L(KH_CASE)
 #undef KH_CASE
         default: return hipErrorInvalidValue;
@@ -630,7 +661,7 @@ hipError_t zeta_clean(const Grid &g, cpx<T> *z0, cpx<T> *z1, hipStream_t s) {
                                    hipStream_t, T *const[3], const int *, Occ);                                    \
     template hipError_t x_slip<T>(const Grid &, cpx<T> *const[3], cpx<T> *, cpx<T> *, double *, const int *,          \
                                   hipStream_t);                                                                    \
-    template hipError_t x_f_zeta<T>(const Grid &, cpx<T> *const[3], cpx<T> *, cpx<T> *, double *, hipStream_t);    \
+    template hipError_t x_f_zeta<T>(const Grid &, cpx<T> *const[3], cpx<T> *, cpx<T> *, double *, bool, hipStream_t); \
     template hipError_t x_ns_u<T>(const Grid &, const Comps<T> &, cpx<T> *, cpx<T> *, cpx<T> *const[3], double *,    \
                                   double, double, int, hipStream_t);                                               \
     template hipError_t zeta_clean<T>(const Grid &, cpx<T> *, cpx<T> *, hipStream_t);                               \

@@ -254,6 +254,14 @@ void drop_graph(kh_run *r);
 // the run's occupancy bits of the 4-point z vectors
 static inline Occ occ_of(const kh_run *r) { return Occ{(unsigned long long *)r->occ, r->occw}; }
 
+// A step's place in a chain of fused steps captured into one graph: the step
+// before it left u_hat after the inverse x pass in the transform buffers
+// (have_u), and it does so for the one after it (next).
+struct Chain {
+    bool         have_u = false, next = false;
+    static Chain of(int k, int count) { return {k > 0, k + 1 < count}; }
+};
+
 template <typename T>
 struct Step {
     static cpx<T> *S(kh_run *r, int i) { return (cpx<T> *)r->spec[i]; }
@@ -505,8 +513,8 @@ struct Step {
     // round-off only: FFT(IFFT(a)) = a for the band-limited fields, so the
     // final U2zeta_k of u* + f is taken directly from u*_hat + P f_hat.
     // one step + the device step counter
-    static int step(kh_run *r) {
-        KH_TRY(r->shear ? step_shear(r) : step_body(r));
+    static int step(kh_run *r, Chain c = {}) {
+        KH_TRY(r->shear ? step_shear(r) : step_body(r, c));
         // the fused body ticks inside z_force (or right after it)
         if (r->shear || r->step_path == KH_PATH_REFERENCE_ORDER) KH_LAUNCH("tick", tick(r->d_ts, r->stream));
         if (r->shear) {
@@ -550,7 +558,7 @@ struct Step {
     // step, up to u* in real space (written only where mask != 0 when a mask
     // is given), for the run r or, when g carries a batch, for every run of
     // the batch from r on: one launch per pass covers them all.
-    static int fused_fluid(kh_run *r, const Grid &g, const T *mask, Occ occ = {}) {
+    static int fused_fluid(kh_run *r, const Grid &g, const T *mask, Chain c, Occ occ = {}) {
         hipStream_t s     = r->stream;
         cpx<T>     *s3[3] = {S(r, 0), S(r, 1), S(r, 2)};
         Comps<T>    c5{{S(r, 0), S(r, 1), S(r, 2), S(r, 3), S(r, 4)}};
@@ -560,7 +568,7 @@ struct Step {
         cpx<T>  *q5[5] = {S(r, 1), S(r, 2), S(r, 0), S(r, 4), S(r, 3)};
         Comps<T> cq5{{q5[0], q5[1], q5[2], q5[3], q5[4]}};
         // NS_solver_slavedEuler: zeta -> u -> products -> -Omega -> slaved Euler
-        KH_LAUNCH("x_zeta2u_inv", (x_zeta2u_inv<T>(g, Z(r, 0), Z(r, 1), s3, r->ukdc, s)));
+        if (!c.have_u) KH_LAUNCH("x_zeta2u_inv", (x_zeta2u_inv<T>(g, Z(r, 0), Z(r, 1), s3, r->ukdc, s)));
         KH_LAUNCH("y_inv", (cols_y<T, false>(g, c5, 3, 1, 0, s)));
         KH_LAUNCH("z_adv", (z_adv<T>(g, s3, q5, s)));
         KH_LAUNCH("y_fwd_adv", (cols_y<T, true>(g, cq5, 5, 0, 1, s)));
@@ -576,7 +584,7 @@ struct Step {
     // f = P(up - phi u*), u = u* + f, zeta = curl u (u* = u + us2 when us2
     // is given; up_is_f: the particle step left f itself in up), and the
     // device step counter; for r or r's batch as above
-    static int fused_force(kh_run *r, const Grid &g, T *const us2[3], bool up_is_f, Occ occ = {}) {
+    static int fused_force(kh_run *r, const Grid &g, T *const us2[3], bool up_is_f, Chain c, Occ occ = {}) {
         hipStream_t s      = r->stream;
         cpx<T>     *s3[3]  = {S(r, 0), S(r, 1), S(r, 2)};
         Comps<T>    c5{{S(r, 0), S(r, 1), S(r, 2), S(r, 3), S(r, 4)}};
@@ -584,7 +592,7 @@ struct Step {
         KH_LAUNCH("z_force", (z_force<T>(g, up3, PS(r), up_is_f ? nullptr : u3, s3, 3, r->d_ts, s, us2, nullptr,
                                          occ)));
         KH_LAUNCH("y_fwd_force", (cols_y<T, true>(g, c5, 3, 0, 1, s)));
-        KH_LAUNCH("x_f_zeta", (x_f_zeta<T>(g, s3, Z(r, 0), Z(r, 1), r->ukdc, s)));
+        KH_LAUNCH("x_f_zeta", (x_f_zeta<T>(g, s3, Z(r, 0), Z(r, 1), r->ukdc, c.next, s)));
         return KH_OK;
     }
     // F_H, LJ + gravity, velocity (+ noise), u_p scatter of a run of plain
@@ -600,7 +608,7 @@ struct Step {
         return KH_OK;
     }
 
-    static int step_body(kh_run *r) {
+    static int step_body(kh_run *r, Chain c) {
         if (r->step_path == KH_PATH_REFERENCE_ORDER) return step_reference_order(r);
         const int   ab2 = r->jikan.ts != 0;
         const Grid &g   = r->g;
@@ -620,7 +628,7 @@ struct Step {
         KH_TRY(particles_begin(r, ab2));
         // squirmers read u* on the whole slip shell (|r - a| < xi/2), which
         // reaches points where phi has underflowed to 0: u* is written in full
-        KH_TRY(fused_fluid(r, g, !r->slip ? PS(r) : nullptr, occ));
+        KH_TRY(fused_fluid(r, g, !r->slip ? PS(r) : nullptr, c, occ));
         if (r->slip) {  // the slip loop leaves up zero
             KH_TRY(calc_f_hydro(r));
             KH_TRY(slip_iteration_dev(r, ab2));
@@ -634,7 +642,7 @@ struct Step {
             KH_TRY(plain_particles(r, ab2));
         }
         T *w3[3] = {W(r, 0), W(r, 1), W(r, 2)};  // squirmers: u = u* + the projected slip field
-        KH_TRY(fused_force(r, g, r->slip ? w3 : nullptr, !r->slip && !r->rigid, occ));
+        KH_TRY(fused_force(r, g, r->slip ? w3 : nullptr, !r->slip && !r->rigid, c, occ));
         r->pclean = true;
         return KH_OK;
     }
@@ -645,7 +653,7 @@ struct Step {
     // arena) that supplies the fluid passes' run-0 buffers and the class's
     // constants; the particle launches take each slot's own arguments from
     // the batch's SlotPart table.
-    static int step_batch(kh_batch *b, kh_run *v) {
+    static int step_batch(kh_batch *b, kh_run *v, Chain c) {
         kh_run     *r = v;
         Grid        g = r->g;
         g.nbatch      = b->capacity;
@@ -656,11 +664,11 @@ struct Step {
         KH_LAUNCH("phi_scatter", (phi_scatter_batch<T>(sp, b->active, b->capacity, b->np_cap, r->jikan.dt_md,
                                                        r->jikan.hdt_md, s)));
         const Occ occ = occ_on(r) ? occ_of(r) : Occ{};
-        KH_TRY(fused_fluid(r, g, PS(r), occ));
+        KH_TRY(fused_fluid(r, g, PS(r), c, occ));
         KH_LAUNCH("particle_step", (particle_step_batch<T>(sp, b->active, b->capacity, b->np_cap,
                                                            (-r->dx3 * r->rho) / r->jikan.dt_fluid, r->jikan.hdt_md,
                                                            s)));
-        KH_TRY(fused_force(r, g, nullptr, true, occ));
+        KH_TRY(fused_force(r, g, nullptr, true, c, occ));
         KH_LAUNCH("records", (records_batch<T>(sp, b->active, b->capacity, s)));
         return KH_OK;
     }
@@ -1709,7 +1717,10 @@ static int capture_steps(kh_run *r, int count, hipGraph_t *graph, hipGraphExec_t
     KH_HIP(hipStreamBeginCapture(r->stream, hipStreamCaptureModeThreadLocal));
     r->capturing = true;
     int st       = KH_OK;
-    for (int k = 0; k < count && st == KH_OK; k++) st = r->mixed ? Step<float>::step(r) : Step<double>::step(r);
+    for (int k = 0; k < count && st == KH_OK; k++) {
+        const Chain c = Chain::of(k, count);
+        st            = r->mixed ? Step<float>::step(r, c) : Step<double>::step(r, c);
+    }
     r->capturing = false;
     hipGraph_t g = nullptr;
     hipError_t e = hipStreamEndCapture(r->stream, &g);
@@ -2456,7 +2467,7 @@ static int batch_capture(kh_batch *b, kh_run *m, int count, hipGraph_t *graph, h
     v->event_pool.clear();
     KH_HIP(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
     int st = KH_OK;
-    for (int k = 0; k < count && st == KH_OK; k++) st = Step<T>::step_batch(b, v.get());
+    for (int k = 0; k < count && st == KH_OK; k++) st = Step<T>::step_batch(b, v.get(), Chain::of(k, count));
     hipGraph_t g = nullptr;
     hipError_t e = hipStreamEndCapture(b->stream, &g);
     if (st != KH_OK) {
