@@ -149,6 +149,7 @@ struct kh_run {
     double      *shear_pstress = nullptr;      // np x 6 stress partials of the sheared gather and LJ
     double      *shear_acc     = nullptr;      // Reynolds-stress partials (one per k_obl_to_cart workgroup)
     long long    shear_nacc    = 0;
+    void        *shear_spec    = nullptr;      // two spectral fields: omega_hat's y and z components
     double      *shear_last    = nullptr;      // the last step's stress record (KH_SHEAR_RECORD doubles)
     double      *shear_hist    = nullptr;      // records of shear_hist_n steps from ts = shear_hist_base
     int          shear_hist_n = 0, shear_hist_base = 0;
@@ -740,18 +741,25 @@ struct Step {
         KH_LAUNCH("z_c2r", (fft_z_c2r_multi<T>(g, zio, 3, r->stream, g.trn_z)));
         return KH_OK;
     }
-    // The same inverse transform of omega's three spectra, then u x omega
-    // (contravariant u and omega, covariant product) into out, fused into
-    // the z pass. u holds the real-space u.
-    static int c2r_kept3_cross(kh_run *r, cpx<T> *const sp[3], T *const u[3], T *const out[3]) {
-        const Grid &g = r->g;
-        Comps<T> c{{sp[0], sp[1], sp[2], nullptr, nullptr}};
-        KH_LAUNCH("x_inv_kept", (cols_x<T, false>(g, c, 3, 1, 0, r->stream)));
-        KH_LAUNCH("y_inv_kept", (cols_y<T, false>(g, c, 3, 1, 0, r->stream)));
+    // The nonlinear term of the sheared step on the kept modes: u_hat and
+    // omega_hat of zeta, u x omega in the z pass, its transform into sp (from
+    // u's own buffers); S(3) keeps u_hat^y for the slaved-Euler pass.
+    static int obl_advection(kh_run *r, cpx<T> *const sp[3], int truncate) {
+        const Grid &g     = r->g;
+        hipStream_t s     = r->stream;
+        cpx<T>     *om[3] = {S(r, 4), (cpx<T> *)r->shear_spec, (cpx<T> *)r->shear_spec + g.nspec};
+        Comps<T>    cu{{sp[0], sp[1], sp[2]}}, cw{{om[0], om[1], om[2]}};
+        KH_LAUNCH("obl_zeta_to_u", (obl_zeta_to_u<T>(g, Z(r, 0), Z(r, 1), sp[0], sp[1], sp[2], S(r, 3), r->ukdc, 0,
+                                                     truncate, r->deg, s)));
+        KH_LAUNCH("obl_zeta_to_omega", (obl_zeta_to_omega<T>(g, Z(r, 0), Z(r, 1), om, s)));
+        for (const Comps<T> &c : {cu, cw}) {
+            KH_LAUNCH("x_inv_kept", (cols_x<T, false>(g, c, 3, 1, 0, s)));
+            KH_LAUNCH("y_inv_kept", (cols_y<T, false>(g, c, 3, 1, 0, s)));
+        }
         const T scale = (T)(1.0 / ((double)g.nx * (double)g.ny * (double)g.nz));
-        ZIO<T>  zio{{sp[0], sp[1], sp[2]}, {out[0], out[1], out[2]}};
-        KH_LAUNCH("z_c2r_cross",
-                  (zw_c2r_cross<T>(g.nz, zio, u, (long long)g.nx * g.ny, scale, g.trn_z, g.nzp, r->stream)));
+        KH_LAUNCH("z_obl_adv", (zw_obl_adv<T>(g, sp, om, sp, scale, s)));
+        KH_LAUNCH("y_fwd_kept", (cols_y<T, true>(g, cu, 3, 0, 1, s)));
+        KH_LAUNCH("x_fwd_kept", (cols_x<T, true>(g, cu, 3, 0, 1, s)));
         return KH_OK;
     }
     // Forward transform of three fields whose consumer reads kept modes only:
@@ -791,12 +799,7 @@ struct Step {
         // take the pruned transforms)
         // (zeta's modes beyond the 2/3 rule are left as they are: nothing in
         // the step reads them before U_k2zeta_k_OBL rewrites every mode)
-        KH_LAUNCH("obl_zeta_to_u", (obl_zeta_to_u<T>(g, Z(r, 0), Z(r, 1), s3[0], s3[1], s3[2], S(r, 3), r->ukdc, 0, 0,
-                                                     gd, s)));
-        KH_TRY(c2r_kept3(r, s3, u3));
-        KH_LAUNCH("obl_zeta_to_omega", (obl_zeta_to_omega<T>(g, Z(r, 0), Z(r, 1), s3, s)));
-        KH_TRY(c2r_kept3_cross(r, s3, u3, w3));
-        KH_TRY(r2c_kept3(r, w3, s3));
+        KH_TRY(obl_advection(r, s3, 0));
         KH_LAUNCH("obl_adv_ns", (obl_adv_ns<T>(g, s3, S(r, 3), Z(r, 0), Z(r, 1), r->sre, gd, -r->nu * dt, 1. / r->nu,
                                                s)));
         // FIX_CELL, Zeta_k2u_k_OBL, U_k2u: u* on the oblique grid
@@ -880,12 +883,7 @@ struct Step {
         const double dt    = r->jikan.dt_fluid;
         switch (fn) {
             case KH_FN_OBL_NS_SOLVER:  // Zeta_k2advection_k_OBL + slaved Euler, as in the step
-                KH_LAUNCH("obl_zeta_to_u", (obl_zeta_to_u<T>(g, Z(r, 0), Z(r, 1), s3[0], s3[1], s3[2], S(r, 3),
-                                                             r->ukdc, 0, 1, r->deg, s)));
-                KH_TRY(c2r_kept3(r, s3, u3));
-                KH_LAUNCH("obl_zeta_to_omega", (obl_zeta_to_omega<T>(g, Z(r, 0), Z(r, 1), s3, s)));
-                KH_TRY(c2r_kept3_cross(r, s3, u3, w3));
-                KH_TRY(r2c_kept3(r, w3, s3));
+                KH_TRY(obl_advection(r, s3, 1));
                 KH_LAUNCH("obl_adv_ns", (obl_adv_ns<T>(g, s3, S(r, 3), Z(r, 0), Z(r, 1), r->sre, r->deg,
                                                        -r->nu * dt, 1. / r->nu, s)));
                 return KH_OK;
@@ -1010,6 +1008,7 @@ int free_run(kh_run *r) {
     if (r->frames) (void)hipFreeAsync(r->frames, r->stream);
     for (double *b : {r->shear_pstress, r->shear_acc, r->shear_last, r->shear_hist})
         if (b) (void)hipFreeAsync(b, r->stream);
+    if (r->shear_spec) (void)hipFreeAsync(r->shear_spec, r->stream);
     for (void *b : {(void *)r->ra.B, (void *)r->ra.GR, (void *)r->ra.GRb, (void *)r->bid, (void *)r->flo})
         if (b) (void)hipFreeAsync(b, r->stream);
     if (r->stream) (void)hipStreamSynchronize(r->stream);
@@ -1774,6 +1773,7 @@ int kh_set_shear(kh_run *r, double shear_rate, int ac, double frequency) {
         r->shear_nacc   = obl_to_cart_blocks(r->g);
         if (hipMallocAsync((void **)&r->shear_pstress, sizeof(double) * 6 * np, r->stream) != hipSuccess ||
             hipMallocAsync((void **)&r->shear_acc, sizeof(double) * r->shear_nacc, r->stream) != hipSuccess ||
+            hipMallocAsync(&r->shear_spec, 2 * 2 * r->esz * (size_t)r->g.nspec, r->stream) != hipSuccess ||
             hipMallocAsync((void **)&r->shear_last, sizeof(double) * KH_SHEAR_RECORD, r->stream) != hipSuccess)
             return fail(KH_ERR_NOMEM, "stress record buffers");
         KH_HIP(hipMemsetAsync(r->shear_pstress, 0, sizeof(double) * 6 * np, r->stream));

@@ -18,10 +18,11 @@ template <typename T>
 hipError_t zw_c2r(int L, const ZIO<T> &io, int ncomp, long long nrows, T scale, int kzv, int pitch,
                   hipStream_t s, const T *mask = nullptr, const int *skip = nullptr, const Grid *batch = nullptr,
                   Occ occ = {});
-// inverse z pass of omega fused with u x omega
+// sheared advection: inverse z of u and omega (3 + 3) -> u x omega -> forward
+// z (3), modes kz < TRN_Z; out may be u
 template <typename T>
-hipError_t zw_c2r_cross(int L, const ZIO<T> &io, const T *const u[3], long long nrows, T scale, int kzv, int pitch,
-                        hipStream_t s);
+hipError_t zw_obl_adv(const Grid &g, cpx<T> *const u[3], cpx<T> *const w[3], cpx<T> *const out[3], T scale,
+                      hipStream_t s);
 // inverse z (3) -> advection products -> forward z (5), modes kz < TRN_Z
 template <typename T>
 hipError_t zw_adv(const Grid &g, cpx<T> *const s3[3], cpx<T> *const p5[5], T scale, hipStream_t s);

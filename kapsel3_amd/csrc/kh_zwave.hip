@@ -226,71 +226,59 @@ __global__ __launch_bounds__(256) void k_zw_c2r_masked(ZIO<T> io, int ncomp, con
     }
 }
 
-// p, q, r = a x (x, y, z) per point of four-point vectors
-template <typename V>
-__device__ __forceinline__ void cross4(const V &a, const V &b, const V &c, const V &x, const V &y, const V &z, V &p,
-                                       V &q, V &r) {
-    p = {b.x * z.x - c.x * y.x, b.y * z.y - c.y * y.y, b.z * z.z - c.z * y.z, b.w * z.w - c.w * y.w};
-    q = {c.x * x.x - a.x * z.x, c.y * x.y - a.y * z.y, c.z * x.z - a.z * z.z, c.w * x.w - a.w * z.w};
-    r = {a.x * y.x - b.x * x.x, a.y * y.y - b.y * x.y, a.z * y.z - b.z * x.z, a.w * y.w - b.w * x.w};
-}
-
-// The inverse z pass of omega's three components fused with u x omega
-// (contravariant u and omega, covariant product: operate_omega.cxx:113-137).
-// A line's omega rows stay in registers, u is read once per point, and the
-// product is written to io.out: omega itself never reaches HBM.
+// Sheared advection: inverse z of u (contravariant) and omega, the product
+// u x omega (covariant, operate_omega.cxx:113-137) and its forward z, all in
+// the registers of a line: neither real field reaches HBM, where separate
+// passes wrote u, read it beside omega, and wrote and read the product. u stays live,
+// omega arrives a component at a time and is folded into the product. A line
+// is read before its product is written, so out may be u. Seven components
+// live: 4 points per lane in FP64 (204 registers at 256 points, two wavefronts
+// a SIMD), so it is bound by its transforms' LDS exchanges and by latency. 256^3
+// FP64 294 us (2.8 TB/s) against 488 us of the passes it replaces, 64^3 16.5
+// against 35; 192 points FP64 (12 per lane, spilling 300 bytes) 79 against 112.
 template <typename T, int L, int E>
-__global__ __launch_bounds__(256) void k_zw_c2r_cross(ZIO<T> io, const T *__restrict__ u0, const T *__restrict__ u1,
-                                                      const T *__restrict__ u2, long long nrows, T scale, int kzv,
-                                                      int pitch) {
+__global__ __launch_bounds__(256) void k_zw_obl_adv(Comps<T> u, Comps<T> w, Comps<T> out, long long nrows, T scale,
+                                                    int kzv, int pitch) {
     using Geo = WaveGeom<T, L, E>;
-    using F   = WaveFft<T, L, E, false, false>;
-    using RS  = RowStage<T, L>;
-    using V   = typename RS::vec;
-    static_assert(L >= 4 * Geo::G, "four points per lane per row");
-    constexpr int NT4 = RS::NV / Geo::G;  // vectors per lane per row
-    __shared__ cpx<T> tw[F::TW], strips[(Geo::NT / 64) * Geo::W * Geo::LP];
-    F::template fill_tw<Geo::NT>(tw);
+    using Fi  = WaveFft<T, L, E, false, false>;
+    using Ff  = WaveFft<T, L, E, true, true>;
+    static_assert(Fi::RN == Ff::R0, "inverse output layout must be the forward input layout");
+    __shared__ cpx<T> twi[Fi::TW], twf[Ff::TW], strips[(Geo::NT / 64) * Geo::W * Geo::LP];
+    Fi::template fill_tw<Geo::NT>(twi);
+    Ff::template fill_tw<Geo::NT>(twf);
     __syncthreads();
     const WaveLane<T, L, E> wl(strips, nrows, pitch);
-    const long long         oa = (2 * wl.line) * L, ob = oa + L;
-    V                       wa[3][NT4], wb[3][NT4];
+    cpx<T>                  U[3][E], F[3][E], v[E];
 #pragma unroll
     for (int c = 0; c < 3; c++) {
-        cpx<T> v[F::E];
-        load_pair<T, L, F>(io.in[c], wl, kzv, v);
-        F::run(v, wl.buf, tw, wl.g);
+        load_pair<T, L, Fi>(u.p[c], wl, kzv, U[c]);
+        Fi::run(U[c], wl.buf, twi, wl.g);
 #pragma unroll
-        for (int i = 0; i < F::E; i++) wl.buf[WavePad<T>::at(F::out_point(wl.g, i))] = v[i];
-        wave_sync();
-#pragma unroll
-        for (int t = 0; t < NT4; t++) {
-            const int    z = 4 * (wl.g + Geo::G * t);
-            const cpx<T> a = wl.buf[WavePad<T>::at(z)], b = wl.buf[WavePad<T>::at(z + 1)],
-                         d = wl.buf[WavePad<T>::at(z + 2)], e = wl.buf[WavePad<T>::at(z + 3)];
-            wa[c][t] = {a.x * scale, b.x * scale, d.x * scale, e.x * scale};
-            wb[c][t] = {a.y * scale, b.y * scale, d.y * scale, e.y * scale};
-        }
-        wave_sync();
+        for (int i = 0; i < E; i++) U[c][i] = cscale(U[c][i], scale);
     }
 #pragma unroll
-    for (int t = 0; t < NT4; t++) {
-        const int z = 4 * (wl.g + Geo::G * t);
-        V         p, q, r;
-        if (wl.okA) {
-            const long long o = oa + z;
-            cross4(RS::ld(u0 + o), RS::ld(u1 + o), RS::ld(u2 + o), wa[0][t], wa[1][t], wa[2][t], p, q, r);
-            RS::st(io.out[0] + o, p);
-            RS::st(io.out[1] + o, q);
-            RS::st(io.out[2] + o, r);
+    for (int c = 0; c < 3; c++) {
+        load_pair<T, L, Fi>(w.p[c], wl, kzv, v);
+        Fi::run(v, wl.buf, twi, wl.g);
+#pragma unroll
+        for (int i = 0; i < E; i++) {
+            const cpx<T> o = cscale(v[i], scale), a = U[0][i], b = U[1][i], d = U[2][i];
+            if (c == 0) {
+                F[1][i] = cmk(d.x * o.x, d.y * o.y);
+                F[2][i] = cmk(-(b.x * o.x), -(b.y * o.y));
+            } else if (c == 1) {
+                F[0][i] = cmk(-(d.x * o.x), -(d.y * o.y));
+                F[2][i] = cmk(a.x * o.x + F[2][i].x, a.y * o.y + F[2][i].y);
+            } else {
+                F[0][i] = cmk(b.x * o.x + F[0][i].x, b.y * o.y + F[0][i].y);
+                F[1][i] = cmk(F[1][i].x - a.x * o.x, F[1][i].y - a.y * o.y);
+            }
         }
-        if (wl.okB) {
-            const long long o = ob + z;
-            cross4(RS::ld(u0 + o), RS::ld(u1 + o), RS::ld(u2 + o), wb[0][t], wb[1][t], wb[2][t], p, q, r);
-            RS::st(io.out[0] + o, p);
-            RS::st(io.out[1] + o, q);
-            RS::st(io.out[2] + o, r);
-        }
+    }
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+        Ff::run(F[c], wl.buf, twf, wl.g);
+        store_pair<T, L, Ff>(F[c], wl, kzv, out.p[c]);
     }
 }
 
@@ -594,6 +582,7 @@ struct ZwE {
     static constexpr int  adv   = WaveE<T, L, sizeof(T) == 4 ? KH_ADV_E32 : KH_ADV_E64>::value;
     static constexpr bool live3 = adv <= KH_ADV_LIVE3_E;
     static constexpr int  force = WaveE<T, L, sizeof(T) == 4 ? KH_FORCE_E32 : KH_FORCE_E64>::value;
+    static constexpr int  obl   = WaveE<T, L, sizeof(T) == 4 ? 8 : 4>::value;  // seven components live
 };
 
 template <typename T, int L, int E>
@@ -669,18 +658,19 @@ hipError_t zw_c2r(int L, const ZIO<T> &io, int ncomp, long long nrows, T scale, 
 }
 
 template <typename T>
-hipError_t zw_c2r_cross(int L, const ZIO<T> &io, const T *const u[3], long long nrows, T scale, int kzv, int pitch,
-                        hipStream_t s) {
-    switch (L) {
+hipError_t zw_obl_adv(const Grid &g, cpx<T> *const u[3], cpx<T> *const w[3], cpx<T> *const out[3], T scale,
+                      hipStream_t s) {
+    const long long nrows = (long long)g.nx * g.ny;
+    const Comps<T>  cu{{u[0], u[1], u[2]}}, cw{{w[0], w[1], w[2]}}, co{{out[0], out[1], out[2]}};
+    switch (g.nz) {
 #define KH_CASE(n)                                                                                              \
     case n:                                                                                                     \
-        hipLaunchKernelGGL((k_zw_c2r_cross<T, n, ZwE<T, n>::pass>), dim3(zw_blocks<T, n, ZwE<T, n>::pass>(nrows)), dim3(256), 0, s, io, u[0], u[1], u[2], nrows, scale, kzv, pitch); \
+        hipLaunchKernelGGL((k_zw_obl_adv<T, n, ZwE<T, n>::obl>), dim3(zw_blocks<T, n, ZwE<T, n>::obl>(nrows)), dim3(256), 0, s, cu, cw, co, nrows, scale, g.trn_z, g.nzp); \
         return hipGetLastError();
         KH_FOR_EACH_WL(KH_CASE)
 #undef KH_CASE
-        default: break;
+        default: return hipErrorInvalidValue;
     }
-    return hipErrorInvalidValue;
 }
 
 template <typename T>
@@ -738,7 +728,7 @@ hipError_t zw_force(const Grid &g, T *const up[3], T *phis, T *const us[3], cpx<
     template hipError_t zw_r2c<T>(int, const T *, cpx<T> *, long long, int, hipStream_t, int);               \
     template hipError_t zw_c2r<T>(int, const ZIO<T> &, int, long long, T, int, int, hipStream_t, const T *, \
                                   const int *, const Grid *, Occ);                                         \
-    template hipError_t zw_c2r_cross<T>(int, const ZIO<T> &, const T *const[3], long long, T, int, int, hipStream_t); \
+    template hipError_t zw_obl_adv<T>(const Grid &, cpx<T> *const[3], cpx<T> *const[3], cpx<T> *const[3], T, hipStream_t); \
     template hipError_t zw_adv<T>(const Grid &, cpx<T> *const[3], cpx<T> *const[5], T, hipStream_t);         \
     template hipError_t zw_force<T>(const Grid &, T *const[3], T *, T *const[3], cpx<T> *const[3], int, int *,        \
                                     hipStream_t, T *const[3], const int *, Occ);
