@@ -14,6 +14,14 @@ hipError_t fft_z_r2c(const Grid &g, const T *in, cpx<T> *out, hipStream_t s, int
 // kzvalid >= 0: modes kz >= kzvalid are taken as zero (not read)
 template <typename T>
 hipError_t fft_z_c2r(const Grid &g, const cpx<T> *in, T *out, hipStream_t s, int kzvalid = -1);
+// up to three real fields and their spectra, one launch
+template <typename T>
+struct RIO {
+    const T *in[3];
+    cpx<T>  *out[3];
+};
+template <typename T>
+hipError_t fft_z_r2c_multi(const Grid &g, const RIO<T> &io, int ncomp, hipStream_t s, int kzvalid = -1);
 // up to five components in one launch
 template <typename T>
 struct ZIO {

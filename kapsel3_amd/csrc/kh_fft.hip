@@ -74,8 +74,12 @@ static hipError_t launch_strided(int L, cpx<T> *data, long long lstride, int nco
 }
 
 template <typename T>
+hipError_t fft_z_r2c_multi(const Grid &g, const RIO<T> &io, int ncomp, hipStream_t s, int kzvalid) {
+    return zw_r2c<T>(g.nz, io, ncomp, (long long)g.nx * g.ny, g.nzp, s, kzvalid);
+}
+template <typename T>
 hipError_t fft_z_r2c(const Grid &g, const T *in, cpx<T> *out, hipStream_t s, int kzvalid) {
-    return zw_r2c<T>(g.nz, in, out, (long long)g.nx * g.ny, g.nzp, s, kzvalid);
+    return fft_z_r2c_multi<T>(g, RIO<T>{{in}, {out}}, 1, s, kzvalid);
 }
 template <typename T>
 hipError_t fft_z_c2r(const Grid &g, const cpx<T> *in, T *out, hipStream_t s, int kzvalid) {
@@ -123,6 +127,7 @@ hipError_t fft3d_c2r(const Grid &g, cpx<T> *spec_inout, T *real_out, hipStream_t
 #define KH_INST(T)                                                                   \
     template hipError_t fft_z_r2c<T>(const Grid &, const T *, cpx<T> *, hipStream_t, int); \
     template hipError_t fft_z_c2r<T>(const Grid &, const cpx<T> *, T *, hipStream_t, int); \
+    template hipError_t fft_z_r2c_multi<T>(const Grid &, const RIO<T> &, int, hipStream_t, int); \
     template hipError_t fft_z_c2r_multi<T>(const Grid &, const ZIO<T> &, int, hipStream_t, int, const T *, Occ); \
     template hipError_t fft_y<T, true>(const Grid &, cpx<T> *, hipStream_t);          \
     template hipError_t fft_y<T, false>(const Grid &, cpx<T> *, hipStream_t);         \

@@ -27,6 +27,8 @@ template <typename T>
 hipError_t add3(long long n, T *const u[3], T *const f[3], hipStream_t s);
 template <typename T>
 hipError_t fill(long long n, T *p, T v, hipStream_t s);
+template <typename T>
+hipError_t fill3(long long n, T *const p[3], T v, hipStream_t s);  // three fields, one launch
 
 // kh_shear.hip (the Lees-Edwards step; gd = strain of the oblique grid)
 template <typename T>

@@ -401,7 +401,8 @@ struct Step {
         return KH_OK;
     }
     static int make_up(kh_run *r) {
-        for (int d = 0; d < 3; d++) KH_TRY(zero(r, UP(r, d)));
+        T *up3[3] = {UP(r, 0), UP(r, 1), UP(r, 2)};
+        KH_LAUNCH("fill", (fill3<T>(r->g.nreal, up3, (T)0, r->stream)));
         return scatter_up(r);
     }
     // Make_f_particle_dt_sole (f_particle.h:60-67) into W[0..2]
@@ -766,7 +767,8 @@ struct Step {
     // y and x passes write only the kept rows of the kept columns.
     static int r2c_kept3(kh_run *r, T *const in[3], cpx<T> *const sp[3]) {
         const Grid &g = r->g;
-        for (int d = 0; d < 3; d++) KH_LAUNCH("fft_z_r2c", (fft_z_r2c<T>(g, in[d], sp[d], r->stream, g.trn_z)));
+        const RIO<T> rio{{in[0], in[1], in[2]}, {sp[0], sp[1], sp[2]}};
+        KH_LAUNCH("fft_z_r2c", (fft_z_r2c_multi<T>(g, rio, 3, r->stream, g.trn_z)));
         Comps<T> c{{sp[0], sp[1], sp[2], nullptr, nullptr}};
         KH_LAUNCH("y_fwd_kept", (cols_y<T, true>(g, c, 3, 0, 1, r->stream)));
         KH_LAUNCH("x_fwd_kept", (cols_x<T, true>(g, c, 3, 0, 1, r->stream)));

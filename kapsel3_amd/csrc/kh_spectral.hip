@@ -221,7 +221,8 @@ __global__ __launch_bounds__(PW_NT) void k_add3(long long n, T *__restrict__ u0,
 
 // 16-byte stores; fields are hipMalloc'd (256-byte aligned)
 template <typename T>
-__global__ __launch_bounds__(PW_NT) void k_fill(long long n, T *__restrict__ p, T v) {
+__global__ __launch_bounds__(PW_NT) void k_fill(long long n, T *p0, T *p1, T *p2, T v) {
+    T *const        p  = blockIdx.y == 0 ? p0 : blockIdx.y == 1 ? p1 : p2;
     constexpr int   W  = 16 / sizeof(T);
     const long long i  = ((long long)blockIdx.x * PW_NT + threadIdx.x) * W;
     if (i + W <= n) {
@@ -279,10 +280,18 @@ hipError_t add3(long long n, T *const u[3], T *const f[3], hipStream_t s) {
     return hipGetLastError();
 }
 template <typename T>
-hipError_t fill(long long n, T *p, T v, hipStream_t s) {
+static hipError_t fill_n(long long n, T *p0, T *p1, T *p2, int fields, T v, hipStream_t s) {
     constexpr int W = 16 / sizeof(T);
-    hipLaunchKernelGGL(k_fill<T>, dim3(nblocks((n + W - 1) / W)), dim3(PW_NT), 0, s, n, p, v);
+    hipLaunchKernelGGL(k_fill<T>, dim3(nblocks((n + W - 1) / W), fields), dim3(PW_NT), 0, s, n, p0, p1, p2, v);
     return hipGetLastError();
+}
+template <typename T>
+hipError_t fill(long long n, T *p, T v, hipStream_t s) {
+    return fill_n<T>(n, p, nullptr, nullptr, 1, v, s);
+}
+template <typename T>
+hipError_t fill3(long long n, T *const p[3], T v, hipStream_t s) {
+    return fill_n<T>(n, p[0], p[1], p[2], 3, v, s);
 }
 
 #define KH_INST(T)                                                                                                 \
@@ -295,7 +304,8 @@ hipError_t fill(long long n, T *p, T v, hipStream_t s) {
                                      cpx<T> *, double *, hipStream_t);                                             \
     template hipError_t f_nonsole<T>(long long, T *const[3], const T *, T *const[3], T *const[3], hipStream_t);    \
     template hipError_t add3<T>(long long, T *const[3], T *const[3], hipStream_t);                                 \
-    template hipError_t fill<T>(long long, T *, T, hipStream_t);
+    template hipError_t fill<T>(long long, T *, T, hipStream_t);                                                   \
+    template hipError_t fill3<T>(long long, T *const[3], T, hipStream_t);
 KH_INST(double)
 KH_INST(float)
 #undef KH_INST

@@ -6,9 +6,10 @@
 
 namespace kh {
 
-// rows of L reals -> half spectra (all L/2+1 modes); spectral rows `pitch` complex apart
+// rows of L reals -> half spectra (modes kz < kzv, < 0: all L/2+1), ncomp
+// components in one launch; spectral rows `pitch` complex apart
 template <typename T>
-hipError_t zw_r2c(int L, const T *in, cpx<T> *out, long long nrows, int pitch, hipStream_t s, int kzv = -1);
+hipError_t zw_r2c(int L, const RIO<T> &io, int ncomp, long long nrows, int pitch, hipStream_t s, int kzv = -1);
 // half spectra (modes kz < kzv, rest zero) -> rows of L reals * scale; grid y = component.
 // mask (a real field): only 4-point vectors where it is nonzero are written
 // (a non-null skip, masked passes only: nothing is done once *skip is nonzero;

@@ -94,15 +94,14 @@ __device__ __forceinline__ void store_pair(const cpx<T> *v, const WaveLane<T, L,
 
 // ------------------------------------------------------------- kernels
 template <typename T, int L, int E>
-__global__ __launch_bounds__(256) void k_zw_r2c(const T *__restrict__ in, cpx<T> *__restrict__ out, long long nrows,
-                                                int pitch, int kzv) {
+__global__ __launch_bounds__(256) void k_zw_r2c(RIO<T> io, long long nrows, int pitch, int kzv) {
     using Geo = WaveGeom<T, L, E>;
     using F   = WaveFft<T, L, E, true, true>;
     __shared__ cpx<T> tw[F::TW], strips[(Geo::NT / 64) * Geo::W * Geo::LP];
     F::template fill_tw<Geo::NT>(tw);
     __syncthreads();
     const WaveLane<T, L, E> wl(strips, nrows, pitch);
-    const T             *ra = in + (2 * wl.line) * L;
+    const T             *ra = io.in[blockIdx.y] + (2 * wl.line) * L;  // one component per grid row
     const T             *rb = ra + L;
     cpx<T>               v[F::E];
 #pragma unroll
@@ -111,7 +110,7 @@ __global__ __launch_bounds__(256) void k_zw_r2c(const T *__restrict__ in, cpx<T>
         v[i]        = cmk(wl.okA ? ra[n] : (T)0, wl.okB ? rb[n] : (T)0);
     }
     F::run(v, wl.buf, tw, wl.g);
-    store_pair<T, L, F>(v, wl, kzv, out);
+    store_pair<T, L, F>(v, wl, kzv, io.out[blockIdx.y]);
 }
 
 // Real rows of a line <-> its LDS strip as (row 2p, row 2p+1) pairs, four
@@ -615,12 +614,12 @@ static inline bool zw_force_split(long long nrows, unsigned nbatch) {
 }
 
 template <typename T>
-hipError_t zw_r2c(int L, const T *in, cpx<T> *out, long long nrows, int pitch, hipStream_t s, int kzv) {
+hipError_t zw_r2c(int L, const RIO<T> &io, int ncomp, long long nrows, int pitch, hipStream_t s, int kzv) {
     if (kzv < 0 || kzv > L / 2 + 1) kzv = L / 2 + 1;
     switch (L) {
 #define KH_CASE(n)                                                                                   \
     case n:                                                                                          \
-        hipLaunchKernelGGL((k_zw_r2c<T, n, ZwE<T, n>::pass>), dim3(zw_blocks<T, n, ZwE<T, n>::pass>(nrows)), dim3(256), 0, s, in, out, nrows, pitch, kzv); \
+        hipLaunchKernelGGL((k_zw_r2c<T, n, ZwE<T, n>::pass>), dim3(zw_blocks<T, n, ZwE<T, n>::pass>(nrows), ncomp), dim3(256), 0, s, io, nrows, pitch, kzv); \
         return hipGetLastError();
         KH_FOR_EACH_WL(KH_CASE)
 #undef KH_CASE
@@ -725,7 +724,7 @@ hipError_t zw_force(const Grid &g, T *const up[3], T *phis, T *const us[3], cpx<
 }
 
 #define KH_INST(T)                                                                                           \
-    template hipError_t zw_r2c<T>(int, const T *, cpx<T> *, long long, int, hipStream_t, int);               \
+    template hipError_t zw_r2c<T>(int, const RIO<T> &, int, long long, int, hipStream_t, int);               \
     template hipError_t zw_c2r<T>(int, const ZIO<T> &, int, long long, T, int, int, hipStream_t, const T *, \
                                   const int *, const Grid *, Occ);                                         \
     template hipError_t zw_obl_adv<T>(const Grid &, cpx<T> *const[3], cpx<T> *const[3], cpx<T> *const[3], T, hipStream_t); \
