@@ -71,6 +71,12 @@ struct Grid {
     const int *bactive;
 };
 
+// up to five spectral components transformed by one launch (grid row = component)
+template <typename T>
+struct Comps {
+    cpx<T> *p[5];
+};
+
 // Launch grid z of a pass over g's batch.
 inline unsigned batch_z(const Grid &g) { return g.nbatch > 1 ? (unsigned)g.nbatch : 1u; }
 // This block's run of the batch is not stepped.

@@ -14,11 +14,11 @@ hipError_t fft_z_r2c(const Grid &g, const T *in, cpx<T> *out, hipStream_t s, int
 // kzvalid >= 0: modes kz >= kzvalid are taken as zero (not read)
 template <typename T>
 hipError_t fft_z_c2r(const Grid &g, const cpx<T> *in, T *out, hipStream_t s, int kzvalid = -1);
-// up to three real fields and their spectra, one launch
+// up to five real fields and their spectra, one launch
 template <typename T>
 struct RIO {
-    const T *in[3];
-    cpx<T>  *out[3];
+    const T *in[5];
+    cpx<T>  *out[5];
 };
 template <typename T>
 hipError_t fft_z_r2c_multi(const Grid &g, const RIO<T> &io, int ncomp, hipStream_t s, int kzvalid = -1);
@@ -33,9 +33,9 @@ template <typename T>
 hipError_t fft_z_c2r_multi(const Grid &g, const ZIO<T> &io, int ncomp, hipStream_t s, int kzvalid = -1,
                            const T *mask = nullptr, Occ occ = {});
 template <typename T, bool FWD>
-hipError_t fft_y(const Grid &g, cpx<T> *data, hipStream_t s);
+hipError_t fft_y(const Grid &g, const Comps<T> &data, int ncomp, hipStream_t s);
 template <typename T, bool FWD>
-hipError_t fft_x(const Grid &g, cpx<T> *data, hipStream_t s);
+hipError_t fft_x(const Grid &g, const Comps<T> &data, int ncomp, hipStream_t s);
 
 // Forward: real R[x][y][z] -> spectral S[x][y][kz] (unnormalised, exp(-i k.x)).
 template <typename T>

@@ -24,14 +24,14 @@ namespace kh {
 // Tile t of outer block o starts at data + o*ostride + t*C; `ncols` columns
 // are valid per outer block.
 template <typename T, int L, bool FWD>
-__global__ __launch_bounds__((ColGeom<T, L>::NT)) void k_fft_strided(cpx<T> *__restrict__ data, long long lstride,
+__global__ __launch_bounds__((ColGeom<T, L>::NT)) void k_fft_strided(Comps<T> data, long long lstride,
                                                                    int ncols, long long ostride, int tiles) {
     using F = ColFft<T, L, FWD, FWD>;
     __shared__ cpx<T> s[F::BUF], tw[F::TW];
     const int  o = blockIdx.x / tiles, t = blockIdx.x - o * tiles;
     const int  g = threadIdx.x / F::C, c = threadIdx.x - g * F::C;
     const bool ok   = t * F::C + c < ncols;
-    cpx<T>    *base = data + (long long)o * ostride + t * F::C + c;
+    cpx<T>    *base = data.p[blockIdx.y] + (long long)o * ostride + t * F::C + c;  // one component per grid row
     cpx<T>     v[F::E];
 #pragma unroll
     for (int i = 0; i < F::E; i++) v[i] = ok ? base[(long long)F::in_point(g, i) * lstride] : cmk((T)0, (T)0);
@@ -56,14 +56,14 @@ bool fft_length_supported(int L) {
 }
 
 template <typename T, bool FWD>
-static hipError_t launch_strided(int L, cpx<T> *data, long long lstride, int ncols, long long ostride, int nouter,
-                                 hipStream_t s) {
+static hipError_t launch_strided(int L, const Comps<T> &data, int ncomp, long long lstride, int ncols,
+                                 long long ostride, int nouter, hipStream_t s) {
     switch (L) {
 #define KH_CASE(n)                                                                                                 \
     case n: {                                                                                                      \
         using Geo       = ColGeom<T, n>;                                                                           \
         const int tiles = (ncols + Geo::C - 1) / Geo::C;                                                           \
-        hipLaunchKernelGGL((k_fft_strided<T, n, FWD>), dim3((unsigned)((long long)tiles * nouter)), dim3(Geo::NT), \
+        hipLaunchKernelGGL((k_fft_strided<T, n, FWD>), dim3((unsigned)((long long)tiles * nouter), ncomp), dim3(Geo::NT), \
                            0, s, data, lstride, ncols, ostride, tiles);                                            \
         return hipGetLastError();                                                                                  \
     }
@@ -97,30 +97,30 @@ hipError_t fft_z_c2r_multi(const Grid &g, const ZIO<T> &io, int ncomp, hipStream
 }
 // y: lines along y at stride nzp, columns kz < nzh, one outer block per x
 template <typename T, bool FWD>
-hipError_t fft_y(const Grid &g, cpx<T> *data, hipStream_t s) {
-    return launch_strided<T, FWD>(g.ny, data, g.nzp, g.nzh, (long long)g.ny * g.nzp, g.nx, s);
+hipError_t fft_y(const Grid &g, const Comps<T> &data, int ncomp, hipStream_t s) {
+    return launch_strided<T, FWD>(g.ny, data, ncomp, g.nzp, g.nzh, (long long)g.ny * g.nzp, g.nx, s);
 }
 // x: lines along x at stride ny*nzp, columns (y,kz) flattened (the row
 // padding columns are transformed too: they hold zeros)
 template <typename T, bool FWD>
-hipError_t fft_x(const Grid &g, cpx<T> *data, hipStream_t s) {
+hipError_t fft_x(const Grid &g, const Comps<T> &data, int ncomp, hipStream_t s) {
     const int M = g.ny * g.nzp;
-    return launch_strided<T, FWD>(g.nx, data, M, M, 0, 1, s);
+    return launch_strided<T, FWD>(g.nx, data, ncomp, M, M, 0, 1, s);
 }
 
 template <typename T>
 hipError_t fft3d_r2c(const Grid &g, const T *real_in, cpx<T> *spec_out, hipStream_t s) {
     hipError_t e;
     if ((e = fft_z_r2c<T>(g, real_in, spec_out, s)) != hipSuccess) return e;
-    if ((e = fft_y<T, true>(g, spec_out, s)) != hipSuccess) return e;
-    return fft_x<T, true>(g, spec_out, s);
+    if ((e = fft_y<T, true>(g, Comps<T>{{spec_out}}, 1, s)) != hipSuccess) return e;
+    return fft_x<T, true>(g, Comps<T>{{spec_out}}, 1, s);
 }
 
 template <typename T>
 hipError_t fft3d_c2r(const Grid &g, cpx<T> *spec_inout, T *real_out, hipStream_t s) {
     hipError_t e;
-    if ((e = fft_x<T, false>(g, spec_inout, s)) != hipSuccess) return e;
-    if ((e = fft_y<T, false>(g, spec_inout, s)) != hipSuccess) return e;
+    if ((e = fft_x<T, false>(g, Comps<T>{{spec_inout}}, 1, s)) != hipSuccess) return e;
+    if ((e = fft_y<T, false>(g, Comps<T>{{spec_inout}}, 1, s)) != hipSuccess) return e;
     return fft_z_c2r<T>(g, spec_inout, real_out, s);
 }
 
@@ -129,10 +129,10 @@ hipError_t fft3d_c2r(const Grid &g, cpx<T> *spec_inout, T *real_out, hipStream_t
     template hipError_t fft_z_c2r<T>(const Grid &, const cpx<T> *, T *, hipStream_t, int); \
     template hipError_t fft_z_r2c_multi<T>(const Grid &, const RIO<T> &, int, hipStream_t, int); \
     template hipError_t fft_z_c2r_multi<T>(const Grid &, const ZIO<T> &, int, hipStream_t, int, const T *, Occ); \
-    template hipError_t fft_y<T, true>(const Grid &, cpx<T> *, hipStream_t);          \
-    template hipError_t fft_y<T, false>(const Grid &, cpx<T> *, hipStream_t);         \
-    template hipError_t fft_x<T, true>(const Grid &, cpx<T> *, hipStream_t);          \
-    template hipError_t fft_x<T, false>(const Grid &, cpx<T> *, hipStream_t);
+    template hipError_t fft_y<T, true>(const Grid &, const Comps<T> &, int, hipStream_t);          \
+    template hipError_t fft_y<T, false>(const Grid &, const Comps<T> &, int, hipStream_t);         \
+    template hipError_t fft_x<T, true>(const Grid &, const Comps<T> &, int, hipStream_t);          \
+    template hipError_t fft_x<T, false>(const Grid &, const Comps<T> &, int, hipStream_t);
 KH_INST(double)
 KH_INST(float)
 #undef KH_INST

@@ -6,12 +6,6 @@
 
 namespace kh {
 
-// up to five spectral components transformed by one launch (grid row = component)
-template <typename T>
-struct Comps {
-    cpx<T> *p[5];
-};
-
 // y passes on columns kz < TRN_Z; x passes on kept (ky,kz) columns (a
 // non-null skip: nothing is done once *skip is nonzero)
 template <typename T, bool FWD>

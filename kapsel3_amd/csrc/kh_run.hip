@@ -7,6 +7,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <initializer_list>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -272,16 +273,29 @@ struct Step {
     static T      *W(kh_run *r, int i) { return (T *)r->work[i]; }
     static T      *PS(kh_run *r) { return (T *)r->phisum; }
 
-    static int r2c(kh_run *r, const T *in, cpx<T> *out) {
-        KH_LAUNCH("fft_z_r2c", (fft_z_r2c<T>(r->g, in, out, r->stream)));
-        KH_LAUNCH("fft_y_fwd", (fft_y<T, true>(r->g, out, r->stream)));
-        KH_LAUNCH("fft_x_fwd", (fft_x<T, true>(r->g, out, r->stream)));
+    // full transforms of n fields, each pass one launch over all of them
+    static int r2c(kh_run *r, std::initializer_list<T *> in, std::initializer_list<cpx<T> *> out) {
+        RIO<T>    io{};
+        Comps<T>  c{};
+        const int n = (int)in.size();
+        std::copy(in.begin(), in.end(), io.in);
+        std::copy(out.begin(), out.end(), io.out);
+        std::copy(out.begin(), out.end(), c.p);
+        KH_LAUNCH("fft_z_r2c", (fft_z_r2c_multi<T>(r->g, io, n, r->stream)));
+        KH_LAUNCH("fft_y_fwd", (fft_y<T, true>(r->g, c, n, r->stream)));
+        KH_LAUNCH("fft_x_fwd", (fft_x<T, true>(r->g, c, n, r->stream)));
         return KH_OK;
     }
-    static int c2r(kh_run *r, cpx<T> *in, T *out) {
-        KH_LAUNCH("fft_x_inv", (fft_x<T, false>(r->g, in, r->stream)));
-        KH_LAUNCH("fft_y_inv", (fft_y<T, false>(r->g, in, r->stream)));
-        KH_LAUNCH("fft_z_c2r", (fft_z_c2r<T>(r->g, in, out, r->stream)));
+    static int c2r(kh_run *r, std::initializer_list<cpx<T> *> in, std::initializer_list<T *> out) {
+        ZIO<T>    io{};
+        Comps<T>  c{};
+        const int n = (int)in.size();
+        std::copy(in.begin(), in.end(), io.in);
+        std::copy(out.begin(), out.end(), io.out);
+        std::copy(in.begin(), in.end(), c.p);
+        KH_LAUNCH("fft_x_inv", (fft_x<T, false>(r->g, c, n, r->stream)));
+        KH_LAUNCH("fft_y_inv", (fft_y<T, false>(r->g, c, n, r->stream)));
+        KH_LAUNCH("fft_z_c2r", (fft_z_c2r_multi<T>(r->g, io, n, r->stream)));
         return KH_OK;
     }
     // The occupancy bits replace phi_sum as the mask of z_c2r and z_force
@@ -302,7 +316,7 @@ struct Step {
     static int zeta_k2u(kh_run *r, int fixmask, int truncate = 1) {
         KH_LAUNCH("zeta_to_u", (zeta_to_u<T>(r->g, Z(r, 0), Z(r, 1), S(r, 0), S(r, 1), S(r, 2), r->ukdc, fixmask,
                                              truncate, r->stream)));
-        for (int d = 0; d < 3; d++) KH_TRY(c2r(r, S(r, d), U(r, d)));
+        KH_TRY(c2r(r, {S(r, 0), S(r, 1), S(r, 2)}, {U(r, 0), U(r, 1), U(r, 2)}));
         return KH_OK;
     }
 
@@ -311,7 +325,8 @@ struct Step {
         KH_TRY(zeta_k2u(r, 0));
         T *p[5] = {W(r, 0), W(r, 1), W(r, 2), W(r, 3), W(r, 4)};
         KH_LAUNCH("products", (products<T>(r->g.nreal, U(r, 0), U(r, 1), U(r, 2), p, r->stream)));
-        for (int c = 0; c < 5; c++) KH_TRY(r2c(r, W(r, c), S(r, c)));
+        KH_TRY(r2c(r, {W(r, 0), W(r, 1), W(r, 2), W(r, 3), W(r, 4)},
+                   {S(r, 0), S(r, 1), S(r, 2), S(r, 3), S(r, 4)}));
         cpx<T> *P5[5] = {S(r, 0), S(r, 1), S(r, 2), S(r, 3), S(r, 4)};
         KH_LAUNCH("adv_ns", (adv_ns<T>(r->g, P5, Z(r, 0), Z(r, 1), -r->nu * r->jikan.dt_fluid, 1. / r->nu,
                                        r->stream)));
@@ -320,7 +335,7 @@ struct Step {
 
     // U2zeta_k (operate_omega.h:208-211)
     static int u2zeta_k(kh_run *r) {
-        for (int d = 0; d < 3; d++) KH_TRY(r2c(r, U(r, d), S(r, d)));
+        KH_TRY(r2c(r, {U(r, 0), U(r, 1), U(r, 2)}, {S(r, 0), S(r, 1), S(r, 2)}));
         KH_LAUNCH("u_to_zeta", (u_to_zeta<T>(r->g, S(r, 0), S(r, 1), S(r, 2), Z(r, 0), Z(r, 1), r->ukdc, r->stream)));
         return KH_OK;
     }
@@ -410,9 +425,9 @@ struct Step {
         T *up3[3] = {UP(r, 0), UP(r, 1), UP(r, 2)}, *u[3] = {U(r, 0), U(r, 1), U(r, 2)};
         T *f[3]   = {W(r, 0), W(r, 1), W(r, 2)};
         KH_LAUNCH("f_nonsole", (f_nonsole<T>(r->g.nreal, up3, PS(r), u, f, r->stream)));
-        for (int d = 0; d < 3; d++) KH_TRY(r2c(r, W(r, d), S(r, d)));
+        KH_TRY(r2c(r, {W(r, 0), W(r, 1), W(r, 2)}, {S(r, 0), S(r, 1), S(r, 2)}));
         KH_LAUNCH("solenoidal", (solenoidal<T>(r->g, S(r, 0), S(r, 1), S(r, 2), r->stream)));
-        for (int d = 0; d < 3; d++) KH_TRY(c2r(r, S(r, d), W(r, d)));
+        KH_TRY(c2r(r, {S(r, 0), S(r, 1), S(r, 2)}, {W(r, 0), W(r, 1), W(r, 2)}));
         return KH_OK;
     }
     // The slip iteration of Time_evolution_hydro (sp_3d_ns.cxx:121-161):
@@ -429,9 +444,9 @@ struct Step {
         for (;;) {
             for (int d = 0; d < 3; d++) KH_TRY(zero(r, up[d]));
             KH_LAUNCH("slip_scatter", slip_scatter<T>(r->pp, r->dp, u, up, r->stream));
-            for (int d = 0; d < 3; d++) KH_TRY(r2c(r, up[d], S(r, d)));
+            KH_TRY(r2c(r, {up[0], up[1], up[2]}, {S(r, 0), S(r, 1), S(r, 2)}));
             KH_LAUNCH("solenoidal", (solenoidal<T>(r->g, S(r, 0), S(r, 1), S(r, 2), r->stream)));
-            for (int d = 0; d < 3; d++) KH_TRY(c2r(r, S(r, d), up[d]));
+            KH_TRY(c2r(r, {S(r, 0), S(r, 1), S(r, 2)}, {up[0], up[1], up[2]}));
             KH_LAUNCH("f_slip", f_slip<T>(r->pp, r->dp, up, coef, r->stream));
             KH_LAUNCH("add3", (add3<T>(r->g.nreal, up, u, r->stream)));
             if (iter == 0) KH_LAUNCH("forces", forces(r->pp, r->dp, r->stream));
@@ -844,7 +859,7 @@ struct Step {
     static int settle(kh_run *r) {
         const Grid &g     = r->g;
         cpx<T>     *s3[3] = {S(r, 0), S(r, 1), S(r, 2)};
-        for (int d = 0; d < 3; d++) KH_TRY(r2c(r, U(r, d), s3[d]));
+        KH_TRY(r2c(r, {U(r, 0), U(r, 1), U(r, 2)}, {s3[0], s3[1], s3[2]}));
         KH_LAUNCH("obl_u_to_zeta",
                   (obl_u_to_zeta<T>(g, s3[0], s3[1], s3[2], Z(r, 0), Z(r, 1), r->ukdc, r->deg, r->stream)));
         r->zeta_lazy = 0;
@@ -892,10 +907,10 @@ struct Step {
             case KH_FN_OBL_ZETA_K2U:  // Zeta_k2u_k_OBL + U_k2u on every mode of zeta
                 KH_LAUNCH("obl_zeta_to_u", (obl_zeta_to_u<T>(g, Z(r, 0), Z(r, 1), s3[0], s3[1], s3[2], nullptr,
                                                              r->ukdc, 0, -1, r->deg, s)));
-                for (int d = 0; d < 3; d++) KH_TRY(c2r(r, s3[d], u3[d]));
+                KH_TRY(c2r(r, {s3[0], s3[1], s3[2]}, {u3[0], u3[1], u3[2]}));
                 return KH_OK;
             case KH_FN_OBL_U2ZETA_K:  // U2u_k + Solenoidal_uk_OBL + U_k2zeta_k_OBL
-                for (int d = 0; d < 3; d++) KH_TRY(r2c(r, u3[d], s3[d]));
+                KH_TRY(r2c(r, {u3[0], u3[1], u3[2]}, {s3[0], s3[1], s3[2]}));
                 KH_LAUNCH("obl_u_to_zeta", (obl_u_to_zeta<T>(g, s3[0], s3[1], s3[2], Z(r, 0), Z(r, 1), r->ukdc,
                                                              r->deg, s)));
                 return KH_OK;
@@ -1448,22 +1463,28 @@ int run_create(const kh_params *P, int np, char *arena, size_t arena_bytes, kh_r
     if (st != KH_OK) return bail(st);
     hipStream_t  cs  = r->stream;
     const size_t psz = sizeof(DevParticle) * (size_t)(np > 0 ? np : 1);
-    if (hipMemcpyAsync(r->ds, hs.data(), sizeof(DevSpecies) * hs.size(), hipMemcpyHostToDevice, cs) != hipSuccess ||
-        hipMemcpyAsync(r->sek, sek.data(), sizeof(int) * sek.size(), hipMemcpyHostToDevice, cs) != hipSuccess ||
-        hipMemsetAsync(r->ukdc, 0, 3 * sizeof(double), cs) != hipSuccess ||
-        hipMemsetAsync(r->d_ts, 0, sizeof(int), cs) != hipSuccess || hipMemsetAsync(r->dp, 0, psz, cs) != hipSuccess ||
-        hipMemsetAsync(r->slipflag, 0, 32, cs) != hipSuccess)
-        return bail(fail(KH_ERR_HIP, "initial upload failed"));
-    for (int i = 0; i < 2; i++)
-        if (hipMemsetAsync(r->zeta[i], 0, sb, cs) != hipSuccess) return bail(fail(KH_ERR_HIP, "hipMemset failed"));
-    for (int i = 0; i < 5; i++)  // the row padding stays zero for good
-        if (hipMemsetAsync(r->spec[i], 0, sb, cs) != hipSuccess) return bail(fail(KH_ERR_HIP, "hipMemset failed"));
-    void *zr[] = {r->ureal[0], r->ureal[1], r->ureal[2], r->up[0], r->up[1], r->up[2],
-                  r->work[0], r->work[1], r->work[2], r->work[3], r->work[4], r->phisum};
-    for (void *b : zr)
-        if (hipMemsetAsync(b, 0, rb, cs) != hipSuccess) return bail(fail(KH_ERR_HIP, "hipMemset failed"));
-    if (hipMemsetAsync(r->occ, 0, sizeof(unsigned long long) * (size_t)r->occw * (size_t)g.nx * g.ny, cs) != hipSuccess)
-        return bail(fail(KH_ERR_HIP, "hipMemset failed"));
+    // every buffer starts zeroed (the spectral rows' padding stays zero for
+    // good): the buffers of an arena, one after the other in it, by one fill
+    // (served runs are created one by one while others step: with the initial
+    // block's three-component transforms 32 of them take 60.7 -> 58.4 ms)
+    bool ok = true;
+    auto clear = [&](void *p, size_t bytes) {
+        if (!arena) ok = ok && hipMemsetAsync(p, 0, bytes, cs) == hipSuccess;
+    };
+    if (arena) ok = hipMemsetAsync(arena, 0, r->arena_used, cs) == hipSuccess;
+    clear(r->ukdc, 3 * sizeof(double));
+    clear(r->d_ts, sizeof(int));
+    clear(r->dp, psz);
+    clear(r->slipflag, 32);
+    for (void *b : r->zeta) clear(b, sb);
+    for (void *b : r->spec) clear(b, sb);
+    for (void *b : {r->ureal[0], r->ureal[1], r->ureal[2], r->up[0], r->up[1], r->up[2], r->work[0], r->work[1],
+                    r->work[2], r->work[3], r->work[4], r->phisum})
+        clear(b, rb);
+    clear(r->occ, sizeof(unsigned long long) * (size_t)r->occw * (size_t)g.nx * g.ny);
+    ok = ok && hipMemcpyAsync(r->ds, hs.data(), sizeof(DevSpecies) * hs.size(), hipMemcpyHostToDevice, cs) == hipSuccess &&
+         hipMemcpyAsync(r->sek, sek.data(), sizeof(int) * sek.size(), hipMemcpyHostToDevice, cs) == hipSuccess;
+    if (!ok) return bail(fail(KH_ERR_HIP, "initial upload failed"));
     if (hipStreamSynchronize(cs) != hipSuccess) return bail(fail(KH_ERR_HIP, "initial upload failed"));
 
     PParams &pp        = r->pp;
@@ -2156,9 +2177,9 @@ int kh_A2a_k(kh_run *r, double *a) {
     if (!r || !a) return fail(KH_ERR_ARG, "NULL argument");
     KH_TRY(upload_real(r, r->work[4], a));
     if (r->mixed) {
-        KH_TRY(Step<float>::r2c(r, (float *)r->work[4], (cpx<float> *)r->spec[4]));
+        KH_TRY(Step<float>::r2c(r, {(float *)r->work[4]}, {(cpx<float> *)r->spec[4]}));
     } else {
-        KH_TRY(Step<double>::r2c(r, (double *)r->work[4], (cpx<double> *)r->spec[4]));
+        KH_TRY(Step<double>::r2c(r, {(double *)r->work[4]}, {(cpx<double> *)r->spec[4]}));
     }
     return download_spec(r, a, r->spec[4]);
 }
@@ -2167,9 +2188,9 @@ int kh_A_k2a(kh_run *r, double *a) {
     if (!r || !a) return fail(KH_ERR_ARG, "NULL argument");
     KH_TRY(upload_spec(r, r->spec[4], a));
     if (r->mixed) {
-        KH_TRY(Step<float>::c2r(r, (cpx<float> *)r->spec[4], (float *)r->work[4]));
+        KH_TRY(Step<float>::c2r(r, {(cpx<float> *)r->spec[4]}, {(float *)r->work[4]}));
     } else {
-        KH_TRY(Step<double>::c2r(r, (cpx<double> *)r->spec[4], (double *)r->work[4]));
+        KH_TRY(Step<double>::c2r(r, {(cpx<double> *)r->spec[4]}, {(double *)r->work[4]}));
     }
     return download_real(r, a, r->work[4]);
 }

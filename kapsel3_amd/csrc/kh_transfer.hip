@@ -149,8 +149,7 @@ void RowStage::release() {
 // Measured on kh_get_fluid (two spectral fields), against the strided copies
 // by the runtime: 256^3 FP64 903 -> 6.0 ms (45 GB/s), 128^3 FP64 218 -> 1.5 ms,
 // 32^3 FP64 14.2 -> 0.11 ms, 256^3 mixed (which converted on the host) 57 -> 6.1
-// ms, 512^3 mixed 422 -> 44 ms. One thread's copies and page faults alone would
-// take 30 ms at 256^3; with WORKERS = 8 the link is the slower side.
+// ms, 512^3 mixed 422 -> 44 ms.
 hipError_t move_rows(RowStage &st, int device, const RowField *f, int nfields, bool to_host, hipStream_t s) {
     std::vector<Chunk> c;
     size_t             most = 0;
