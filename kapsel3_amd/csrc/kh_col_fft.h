@@ -97,7 +97,7 @@ struct ColFft {
         // The results are formed here. Without this the compiler moves the last
         // stage below the conditions the results are used under, and keeps its
         // inputs and twiddles of every component alive until then (340
-        // registers instead of 160 in the FP64 x_adv_ns).
+        // registers instead of 160 in the FP64 x_ns_u).
 #pragma unroll
         for (int i = 0; i < E; i++) asm volatile("" : "+v"(v[i].x), "+v"(v[i].y));
     }

@@ -1,0 +1,77 @@
+"""The column passes at every kind of length (one stage, radix 8 with and
+without a shorter last stage, 12 points per lane; tiles that hold more columns
+than there are kept modes) along x and along y, through the whole plain step
+and the squirmers' slip loop, against the oracle; and captured steps, which go
+from one step's zeta straight to the next one's u_hat, against the same steps
+taken one by one."""
+import numpy as np
+import pytest
+
+from oracle import kref
+from kapsel3_amd import workloads
+from kapsel3_amd._abi import FP64, JAX_Z, JP_SLIP, MIXED, Params, make_species
+
+from test_gpu_step import cmp_particles, rel
+
+pytestmark = pytest.mark.gpu
+
+
+def system(n, slip=False, precision=FP64, a=2.0):
+    sp = [make_species(mass_ratio=1.0, propulsion=JP_SLIP, janus_axis=JAX_Z, slip_vel=0.01, slip_mode=1.3)
+          if slip else make_species(mass_ratio=2.0)]
+    # (the reference's link cells are 16 points: no pair forces on a shorter axis)
+    P = Params(n, a=a, a_xi=2.0, dt=0.05, species=sp, rotation=1, g=0.0 if slip else 1e-3, fix_cell=(0, 1, 1),
+               lj_truncate=1 if min(n) >= 16 else -1, precision=precision)
+    box = np.array(n, float)
+    x = np.mod(np.array([[0.2, 0.3, 0.9], [0.2, 0.3, 0.9], [0.7, 0.8, 0.4]]) * box + [[0, 0, 0], [3.1, 1.2, 2.2], [0, 0, 0]],
+               box)
+    p = workloads.particles_at(x, spec=np.zeros(3, int), q=workloads.random_quaternions(3, 3))
+    rng = np.random.default_rng(4)
+    p["v"], p["omega"] = rng.normal(0, 1e-2, (3, 3)), rng.normal(0, 1e-3, (3, 3))
+    return P, p
+
+
+@pytest.mark.parametrize("slip", [False, True], ids=["plain", "slip"])
+@pytest.mark.parametrize("n", [(512, 16, 16), (16, 512, 24), (384, 24, 16), (24, 384, 16), (256, 12, 32), (16, 192, 12),
+                               (128, 96, 16), (64, 48, 24), (12, 64, 128), (8, 24, 32)],
+                         ids=lambda n: "x".join(map(str, n)))
+def test_steps_against_oracle(gpu, n, slip):
+    import kapsel3_amd
+    print(f"columns {n} slip {slip}", flush=True)
+    P, p = system(n, slip, a=2.0 if min(n) > 8 else 1.0)
+    o, g = kref.Run(P, 3), kapsel3_amd.Run(P, 3)
+    for r in (o, g):
+        r.set_particles(p)
+        r.init_fluid()
+        r.step(10)
+    cmp_particles(g.get_particles(), o.get_particles(), 1e-10,
+                  ["x_nopbc", "v", "omega", "q", "f_hydro_previous", "torque_hydro_previous"], p0=p, a=2.0)
+    zo, zg = o.get_fluid(), g.get_fluid()
+    assert rel(zg[0], zo[0]) < 1e-10 and rel(zg[1], zo[1]) < 1e-10
+    # FIX_CELL leaves x free: its mean velocity is carried from step to step
+    assert np.abs(zg[2] - zo[2]).max() < 1e-10 * max(np.abs(zo[2]).max(), 1.0)
+
+
+@pytest.mark.parametrize("precision", [FP64, MIXED], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("n", [(32, 32, 32), (24, 48, 96), (64, 64, 64)], ids=lambda n: "x".join(map(str, n)))
+def test_captured_chain_is_the_steps_one_by_one(gpu, n, precision):
+    """Sixteen steps replayed as two graphs of eight against sixteen launched
+    singly: the same arithmetic, so the same bits (overlapping spheres add two
+    contributions to a zeroed point, in either order the same sum)."""
+    import kapsel3_amd
+    print(f"chain {n} precision {precision}", flush=True)
+    out = []
+    for graph in (True, False):
+        P, p = system(n, precision=precision)
+        with kapsel3_amd.Run(P, 3) as r:
+            r.set_particles(p)
+            r.init_fluid()
+            r.set_graph(graph)
+            r.step(1)
+            r.step(16)
+            r.step(16)
+            out.append((r.get_particles(), r.get_fluid()))
+    (pa, za), (pb, zb) = out
+    for k in ("x", "v", "omega", "q"):
+        assert np.array_equal(pa[k], pb[k]), k
+    assert all(np.array_equal(a, b) for a, b in zip(za, zb))
