@@ -55,9 +55,10 @@ def test_steps_against_oracle(gpu, n, slip):
 @pytest.mark.parametrize("precision", [FP64, MIXED], ids=["fp64", "mixed"])
 @pytest.mark.parametrize("n", [(32, 32, 32), (24, 48, 96), (64, 64, 64)], ids=lambda n: "x".join(map(str, n)))
 def test_captured_chain_is_the_steps_one_by_one(gpu, n, precision):
-    """Sixteen steps replayed as two graphs of eight against sixteen launched
-    singly: the same arithmetic, so the same bits (overlapping spheres add two
-    contributions to a zeroed point, in either order the same sum)."""
+    """Steps replayed as graphs of eight against steps launched singly: the
+    same formulas in other kernels, whose multiply-adds the compiler contracts
+    differently, so equal to rounding over the 33 steps (FP64 1e-12, some
+    thousand ulps; FP32 fields 1e-5)."""
     import kapsel3_amd
     print(f"chain {n} precision {precision}", flush=True)
     out = []
@@ -72,6 +73,7 @@ def test_captured_chain_is_the_steps_one_by_one(gpu, n, precision):
             r.step(16)
             out.append((r.get_particles(), r.get_fluid()))
     (pa, za), (pb, zb) = out
+    tol = 1e-12 if precision == FP64 else 1e-5
     for k in ("x", "v", "omega", "q"):
-        assert np.array_equal(pa[k], pb[k]), k
-    assert all(np.array_equal(a, b) for a, b in zip(za, zb))
+        assert rel(pa[k], pb[k]) < tol, k
+    assert rel(za[0], zb[0]) < tol and rel(za[1], zb[1]) < tol
