@@ -89,6 +89,13 @@ struct XTile {
         const int ntiles = (g.trn_z + Geo::C - 1) / Geo::C;
         const int o      = blockIdx.x / ntiles;
         l                = threadIdx.x / Geo::C;
+        // Lines of 8 and 12 points sit whole in one lane, so l is 0 and every
+        // wavenumber a constant, but the compiler finds that out late, when the
+        // test for the mean mode has become (ikx | iky | kz) == 0: it then drops an
+        // ikx of -1 from the OR instead of making the result -1, and mode
+        // (-1, 0, 0) was taken for the mean mode (zeta and uk_dc wrong after a
+        // step). With l kept unknown nothing is folded, as at the longer lengths.
+        if constexpr (Geo::G == 1) asm volatile("" : "+v"(l));
         kz               = (blockIdx.x - o * ntiles) * Geo::C + (threadIdx.x - l * Geo::C);
         j                = kept_index(o, g.ny, g.trn_y);
         iky              = ky_of(g, j);

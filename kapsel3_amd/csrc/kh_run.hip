@@ -54,10 +54,6 @@ int fail(int status, const char *fmt, ...) {
     } while (0)
 
 constexpr double KH_PI     = 3.14159265358979323846;
-// The fused x passes hold a line of 8 or 12 points whole in one lane; at 12
-// the mean mode's column came out wrong (the cause is not known), so runs on
-// such an x axis step in the reference's order on the full transforms.
-constexpr int FUSED_MIN_NX = 16;
 constexpr double kT_snap_v = 1.439;  // input.cxx:309
 constexpr double kT_snap_o = 1.22;   // input.cxx:311
 
@@ -1524,7 +1520,6 @@ int run_create(const kh_params *P, int np, char *arena, size_t arena_bytes, kh_r
         pp.direct_dist = 2 * (nh + 2) <= nmin;
     }
 
-    if (g.nx < FUSED_MIN_NX) r->step_path = KH_PATH_REFERENCE_ORDER;
     CTime t0  = {0, 0.0, P->dt, P->dt * 0.5, P->dt, P->dt * 0.5};  // sp_3d_ns.cxx:782
     r->jikan  = t0;
     *out      = r;
@@ -2214,7 +2209,7 @@ int kh_set_step_path(kh_run *r, int path) {
     if (!r) return fail(KH_ERR_ARG, "NULL run");
     if (path != KH_PATH_FUSED && path != KH_PATH_REFERENCE_ORDER) return fail(KH_ERR_ARG, "unknown step path %d", path);
     KH_TRY(settle_zeta(r));
-    r->step_path = r->g.nx < FUSED_MIN_NX ? KH_PATH_REFERENCE_ORDER : path;
+    r->step_path = path;
     drop_graph(r);
     return KH_OK;
 }

@@ -148,7 +148,6 @@ int leave(Request *q) {
 
 bool batchable(const kh_server *S, const Request *q) {
     if (S->cfg.batch_slots < 2 || (int)q->parts.size() > KH_BATCH_NP_CAP) return false;
-    if (q->P.nx < 16) return false;  // a batch runs the fused passes, which such an x axis does not take
     for (const kh_species &sp : q->species)
         if (sp.propulsion == KH_JP_SLIP) return false;
     return true;
