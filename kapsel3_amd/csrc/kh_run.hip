@@ -759,14 +759,15 @@ struct Step {
     }
     // The nonlinear term of the sheared step on the kept modes: u_hat and
     // omega_hat of zeta, u x omega in the z pass, its transform into sp (from
-    // u's own buffers); S(3) keeps u_hat^y for the slaved-Euler pass.
-    static int obl_advection(kh_run *r, cpx<T> *const sp[3], int truncate) {
+    // u's own buffers); S(3) keeps u_hat^y for the slaved-Euler pass. zeta's
+    // modes beyond the 2/3 rule are not read and stay as they are.
+    static int obl_advection(kh_run *r, cpx<T> *const sp[3]) {
         const Grid &g     = r->g;
         hipStream_t s     = r->stream;
         cpx<T>     *om[3] = {S(r, 4), (cpx<T> *)r->shear_spec, (cpx<T> *)r->shear_spec + g.nspec};
         Comps<T>    cu{{sp[0], sp[1], sp[2]}}, cw{{om[0], om[1], om[2]}};
-        KH_LAUNCH("obl_zeta_to_u", (obl_zeta_to_u<T>(g, Z(r, 0), Z(r, 1), sp[0], sp[1], sp[2], S(r, 3), r->ukdc, 0,
-                                                     truncate, r->deg, s)));
+        KH_LAUNCH("obl_zeta_to_u", (obl_zeta_to_u<T>(g, Z(r, 0), Z(r, 1), sp[0], sp[1], sp[2], S(r, 3), r->ukdc, 0, 0,
+                                                     r->deg, s)));
         KH_LAUNCH("obl_zeta_to_omega", (obl_zeta_to_omega<T>(g, Z(r, 0), Z(r, 1), om, s)));
         for (const Comps<T> &c : {cu, cw}) {
             KH_LAUNCH("x_inv_kept", (cols_x<T, false>(g, c, 3, 1, 0, s)));
@@ -816,7 +817,7 @@ struct Step {
         // take the pruned transforms)
         // (zeta's modes beyond the 2/3 rule are left as they are: nothing in
         // the step reads them before U_k2zeta_k_OBL rewrites every mode)
-        KH_TRY(obl_advection(r, s3, 0));
+        KH_TRY(obl_advection(r, s3));
         KH_LAUNCH("obl_adv_ns", (obl_adv_ns<T>(g, s3, S(r, 3), Z(r, 0), Z(r, 1), r->sre, gd, -r->nu * dt, 1. / r->nu,
                                                s)));
         // FIX_CELL, Zeta_k2u_k_OBL, U_k2u: u* on the oblique grid
@@ -900,7 +901,11 @@ struct Step {
         const double dt    = r->jikan.dt_fluid;
         switch (fn) {
             case KH_FN_OBL_NS_SOLVER:  // Zeta_k2advection_k_OBL + slaved Euler, as in the step
-                KH_TRY(obl_advection(r, s3, 1));
+                // (the step's z pass leaves no real u: here the truncated zeta's u is left in the field)
+                KH_LAUNCH("obl_zeta_to_u", (obl_zeta_to_u<T>(g, Z(r, 0), Z(r, 1), s3[0], s3[1], s3[2], nullptr,
+                                                             r->ukdc, 0, 1, r->deg, s)));
+                KH_TRY(c2r_kept3(r, s3, u3));
+                KH_TRY(obl_advection(r, s3));
                 KH_LAUNCH("obl_adv_ns", (obl_adv_ns<T>(g, s3, S(r, 3), Z(r, 0), Z(r, 1), r->sre, r->deg,
                                                        -r->nu * dt, 1. / r->nu, s)));
                 return KH_OK;

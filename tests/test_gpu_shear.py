@@ -263,6 +263,23 @@ def test_sheared_functions_fp64(gpu):
     gr.close()
 
 
+def test_ns_solver_leaves_u(gpu):
+    """kh_apply of the sheared NS solver leaves the velocity it was given
+    (zeta_k2u of the truncated zeta) in u."""
+    n, rate = 32, 0.05
+    P, p, g0 = sheared_system(n)
+    z = initial_fluid(P, n, g0, rate)
+    gr, orc = _pair(P, p, z, rate, g0)
+    print("u after the sheared NS solver", flush=True)
+    for d in range(3):  # something else in the field
+        gr.set_field("u%d" % d, np.full((n, n, n + 2), 7.0))
+    gr.apply("obl_ns_solver")
+    orc.le_apply("zeta_k2u")
+    for d in range(3):
+        assert rel(gr.get_field(f"u{d}")[..., :n], orc.get_field(f"u{d}")[..., :n]) < 1e-12, d
+    gr.close()
+
+
 def test_deferred_modes_after_remap_and_transitions(gpu):
     """zeta's modes beyond the 2/3 rule, which sheared steps leave to be
     formed when the state is read, against the oracle (1e-10, uk_dc
