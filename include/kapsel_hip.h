@@ -94,7 +94,8 @@ typedef struct kh_params {
                               0: count every pair once */
     int               nspecies;
     const kh_species *species; /* nspecies entries, copied at kh_run_create */
-    int    slip_iter_max;      /* switch.SLIP_iter (MAX_SLIP_ITER) */
+    int    slip_iter_max;      /* switch.SLIP_iter (MAX_SLIP_ITER); beyond 16 kh_step
+                                  waits for the device a few times a step */
     double slip_tol;           /* switch.SLIP_tol (MAX_SLIP_TOL) */
     int    precision;          /* KH_FP64 or KH_MIXED */
     uint64_t seed;             /* thermal-noise stream key */

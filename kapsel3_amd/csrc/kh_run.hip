@@ -54,6 +54,16 @@ int fail(int status, const char *fmt, ...) {
     } while (0)
 
 constexpr double KH_PI     = 3.14159265358979323846;
+// Squirmer steps launch every slip iteration up to a slip_iter_max of
+// SLIP_ALL and are captured. Beyond it, where the launches of the iterations
+// after convergence (15 us an iteration, at any grid) set the time, the
+// iterations go uncaptured in rounds, 4 and then 8 at a time, and the host reads
+// the loop's flag between them. us/step at 48^3, 64^3 and 128^3 FP64, converging
+// in 3 iterations: all of 16 launched 461, 471, 681, all of 64 1192, 1204, 1438,
+// in rounds 340, 340, 537; with 17 to 24 allowed and never converging the captured step
+// is the faster one (1006, 1039, 1807 against 1143, 1210, 1907 at 17).
+constexpr int  SLIP_ALL = 16;
+constexpr bool slip_round_ends(int launched) { return launched % 8 == 4; }
 constexpr double kT_snap_v = 1.439;  // input.cxx:309
 constexpr double kT_snap_o = 1.22;   // input.cxx:311
 
@@ -473,7 +483,8 @@ struct Step {
     // The same slip iteration in the fused step with its length decided on
     // the device: every iteration up to slip_iter_max is launched and those
     // after convergence return at once (slip_conv sets the flag the others
-    // read), so squirmer steps are captured as graphs like the plain step.
+    // read), so squirmer steps are captured as graphs like the plain step (a
+    // slip_iter_max beyond SLIP_ALL: in rounds, see there).
     // The projection of the slip force field runs on the pruned transforms
     // (Solenoidal_u truncates to the 2/3 modes): forward z of the scattered
     // field (read at every point: the shell slip force is nonzero also where
@@ -513,6 +524,12 @@ struct Step {
             KH_LAUNCH("slip_conv", slip_conv(r->pp, r->dp, r->slipeps, s, &loop));
             if (iter + 1 < r->P.slip_iter_max)
                 KH_LAUNCH("slip_update", slip_update(r->pp, r->dp, iter + 1, 1, s, skip));
+            if (r->P.slip_iter_max > SLIP_ALL && slip_round_ends(iter + 1)) {
+                int done = 0;
+                KH_HIP(hipMemcpyAsync(&done, r->slipflag, sizeof(int), hipMemcpyDeviceToHost, s));
+                KH_HIP(hipStreamSynchronize(s));
+                if (done) break;
+            }
         }
         KH_LAUNCH("reset_forces", reset_forces(r->pp, r->dp, s));
         KH_LAUNCH("zeta_add", (zeta_add<T>(g, Z(r, 0), Z(r, 1), S(r, 3), S(r, 4), r->ukdc, r->slipdc, s)));
@@ -1767,7 +1784,8 @@ int kh_step(kh_run *r, int nsteps) {
     if (!r->shear) KH_TRY(settle_zeta(r));
     for (int s = 0; s < nsteps;) {
         const bool graph_ok = r->use_graph && !r->timing && r->step_path == KH_PATH_FUSED && r->jikan.ts > 0 &&
-                              !r->zeta_dirty && !r->shear && r->pclean;
+                              !r->zeta_dirty && !r->shear && r->pclean &&
+                              !(r->slip && r->P.slip_iter_max > SLIP_ALL);
         int done = 1;
         if (graph_ok && nsteps - s >= GRAPH_STEPS) {
             if (!r->graph_exec_k) KH_TRY(capture_steps(r, GRAPH_STEPS, &r->graph_k, &r->graph_exec_k));

@@ -94,6 +94,35 @@ def test_squirmer_steps_fp64(gpu, path, n):
     g.close()
 
 
+@pytest.mark.parametrize("n", [32, 48])
+@pytest.mark.parametrize("iters,tol", [(16, 0.005), (17, 0.005), (100000, 0.005), (17, 0.0), (30, 0.0)])
+def test_large_slip_iter_max(gpu, n, iters, tol):
+    """slip_iter_max is a bound, not a count: beyond 16 the launches stop with
+    the round (of at most 8 iterations) that converges, and a loop that does not
+    converge runs its slip_iter_max iterations, across the ends of the rounds."""
+    print(f"squirmers {n}^3, slip_iter_max {iters}, tol {tol}", flush=True)
+    steps = 10
+    P, parts = squirmer_system(n=n, scale=n / 32, iters=iters, tol=tol)
+    o, g = both(P, parts)
+    o.init_fluid()
+    g.init_fluid()
+    g.timing(True)
+    g.step(1)
+    launched, it = g.timing_stats()["slip_scatter"][0], g.slip_iterations()[0]
+    assert launched == 16 if iters == 16 else it <= launched < it + 8
+    g.timing(False)
+    g.step(steps - 1)
+    o.step(steps)
+    it, loops = g.slip_iterations()
+    assert loops == steps and (it == steps * iters if tol == 0.0 else it < steps * iters)
+    cmp_particles(g.get_particles(), o.get_particles(), 1e-10,
+                  keys=["x", "x_nopbc", "v", "omega", "q", "v_slip", "omega_slip"], p0=parts, a=4.0)
+    zo, zg = o.get_fluid(), g.get_fluid()
+    assert rel(zg[0], zo[0]) < 1e-10 and rel(zg[1], zo[1]) < 1e-10
+    o.close()
+    g.close()
+
+
 def test_squirmers_mixed_vs_fp64(gpu):
     print("squirmers mixed vs fp64, 64^3 x 12, 60 steps", flush=True)
     import kapsel3_amd
