@@ -156,6 +156,9 @@ int kh_set_fluid(kh_run *run, const double *zeta0, const double *zeta1, const do
 int kh_get_fluid(kh_run *run, double *zeta0, double *zeta1, double uk_dc[3]);
 int kh_set_time(kh_run *run, const CTime *jikan);
 int kh_get_time(kh_run *run, CTime *jikan);
+/* Fields and fluid go through pinned host memory, up to 32 MB that the run
+ * allocates at its first such call and keeps until it is destroyed; where it
+ * cannot be allocated the runtime copies row by row, with the same result. */
 int kh_get_field(kh_run *run, int field, double *out);
 int kh_set_field(kh_run *run, int field, const double *in);
 

@@ -16,7 +16,8 @@
 
 #include <algorithm>
 #include <atomic>
-#include <system_error>
+#include <exception>
+#include <new>
 #include <thread>
 #include <vector>
 
@@ -84,6 +85,7 @@ hipError_t reserve(RowStage &st, int slots, size_t slot_bytes) {
         st.release();
         hipError_t e = hipHostMalloc((void **)&st.buf, (size_t)slots * slot_bytes, hipHostMallocDefault);
         if (e != hipSuccess) {
+            (void)hipGetLastError();  // not the next launch's
             st.buf = nullptr;
             return e;
         }
@@ -94,11 +96,40 @@ hipError_t reserve(RowStage &st, int slots, size_t slot_bytes) {
         if (!st.done[i]) {
             hipError_t e = hipEventCreateWithFlags(&st.done[i], hipEventDisableTiming);
             if (e != hipSuccess) {
+                (void)hipGetLastError();
                 st.done[i] = nullptr;
                 return e;
             }
         }
     return hipSuccess;
+}
+
+// Without pinned memory: copies by the runtime, row by row where the rows
+// have gaps, converted on the host where the device holds floats.
+hipError_t move_pageable(const RowField &f, bool out, hipStream_t s) {
+    const size_t esz = f.fp32 ? sizeof(float) : sizeof(double), dpitch = esz * f.pitch, w = esz * f.width;
+    const size_t hpitch = sizeof(double) * f.hwidth;
+    hipError_t   e;
+    if (!f.fp32) {
+        e = out ? hipMemcpy2DAsync(f.host, hpitch, f.dev, dpitch, w, f.rows, hipMemcpyDeviceToHost, s)
+                : hipMemcpy2DAsync(f.dev, dpitch, f.host, hpitch, w, f.rows, hipMemcpyHostToDevice, s);
+        if (e == hipSuccess) e = hipStreamSynchronize(s);
+    } else {
+        std::vector<float> tmp((size_t)f.rows * f.width);
+        if (!out)
+            for (long long r = 0; r < f.rows; r++)
+                for (int k = 0; k < f.width; k++) tmp[(size_t)r * f.width + k] = (float)f.host[r * f.hwidth + k];
+        e = out ? hipMemcpy2DAsync(tmp.data(), w, f.dev, dpitch, w, f.rows, hipMemcpyDeviceToHost, s)
+                : hipMemcpy2DAsync(f.dev, dpitch, tmp.data(), w, w, f.rows, hipMemcpyHostToDevice, s);
+        const hipError_t e2 = hipStreamSynchronize(s);  // also after an error: tmp goes
+        if (e == hipSuccess) e = e2;
+        if (out && e == hipSuccess)
+            for (long long r = 0; r < f.rows; r++)
+                for (int k = 0; k < f.width; k++) f.host[r * f.hwidth + k] = tmp[(size_t)r * f.width + k];
+    }
+    if (out && e == hipSuccess)
+        for (long long r = 0; r < f.rows; r++) std::fill(f.host + r * f.hwidth + f.width, f.host + (r + 1) * f.hwidth, 0.0);
+    return e;
 }
 
 // chunks w, w + step, w + 2 step, ... through slots w * SLOTS ..
@@ -149,8 +180,9 @@ void RowStage::release() {
 // Measured on kh_get_fluid (two spectral fields), against the strided copies
 // by the runtime: 256^3 FP64 903 -> 6.0 ms (45 GB/s), 128^3 FP64 218 -> 1.5 ms,
 // 32^3 FP64 14.2 -> 0.11 ms, 256^3 mixed (which converted on the host) 57 -> 6.1
-// ms, 512^3 mixed 422 -> 44 ms.
-hipError_t move_rows(RowStage &st, int device, const RowField *f, int nfields, bool to_host, hipStream_t s) {
+// ms, 512^3 mixed 422 -> 44 ms. Where the pinned memory is not to be had for
+// every worker one worker takes its two slots, and without those the runtime copies.
+static hipError_t move_rows_on(RowStage &st, int device, const RowField *f, int nfields, bool to_host, hipStream_t s) {
     std::vector<Chunk> c;
     size_t             most = 0;
     for (int i = 0; i < nfields; i++) {
@@ -163,33 +195,53 @@ hipError_t move_rows(RowStage &st, int device, const RowField *f, int nfields, b
     }
     const int n = (int)c.size();
     if (n == 0) return hipSuccess;
+    most = (most + 4095) / 4096 * 4096;
     // one worker, the calling thread, while all chunks fit its slots
-    const int  workers = std::max(1, std::min(RowStage::WORKERS, n / RowStage::SLOTS));
-    hipError_t e       = reserve(st, workers * RowStage::SLOTS, (most + 4095) / 4096 * 4096);
-    if (e != hipSuccess) return e;
+    int workers = std::max(1, std::min(RowStage::WORKERS, n / RowStage::SLOTS));
+    if (reserve(st, workers * RowStage::SLOTS, most) != hipSuccess) {
+        workers = 1;
+        if (reserve(st, RowStage::SLOTS, most) != hipSuccess) {
+            hipError_t e = hipSuccess;
+            for (int i = 0; i < nfields && e == hipSuccess; i++) e = move_pageable(f[i], to_host, s);
+            return e;
+        }
+    }
     if (workers == 1) return work(st, c.data(), n, 0, 1, to_host, s);
-    std::atomic<int>         err{(int)hipSuccess};
-    auto                     run = [&](int w) {
+    std::atomic<int> err{(int)hipSuccess};
+    auto             run = [&](int w) {
         hipError_t r = hipSetDevice(device);
         if (r == hipSuccess) r = work(st, c.data(), n, w, workers, to_host, s);
         if (r != hipSuccess) err.store((int)r);
     };
     std::vector<std::thread> t;
+    std::vector<int>         here;  // the calling thread's share
     t.reserve(workers);
-    std::vector<int> here = {0};  // the calling thread's share
+    here.reserve(workers);
+    here.push_back(0);
     for (int w = 1; w < workers; w++) {
         try {
             t.emplace_back(run, w);
-        } catch (const std::system_error &) {  // no thread to be had: the caller does it
+        } catch (const std::exception &) {  // no thread to be had: the caller does it
             here.push_back(w);
         }
     }
-    int dev = device;
-    (void)hipGetDevice(&dev);
     for (int w : here) run(w);
     for (std::thread &x : t) x.join();
-    if (dev != device) (void)hipSetDevice(dev);
     return (hipError_t)err.load();
+}
+
+hipError_t move_rows(RowStage &st, int device, const RowField *f, int nfields, bool to_host, hipStream_t s) {
+    int        dev = device;
+    hipError_t e   = hipGetDevice(&dev);
+    if (e == hipSuccess && dev != device) e = hipSetDevice(device);  // the caller's may be another
+    if (e != hipSuccess) return e;
+    try {
+        e = move_rows_on(st, device, f, nfields, to_host, s);
+    } catch (const std::bad_alloc &) {  // no exception leaves a C entry
+        e = hipErrorOutOfMemory;
+    }
+    if (dev != device) (void)hipSetDevice(dev);
+    return e;
 }
 
 }  // namespace kh
