@@ -1038,7 +1038,7 @@ int free_run(kh_run *r) {
     drop_graph(r);
     void *bufs[] = {r->zeta[0], r->zeta[1], r->spec[0], r->spec[1], r->spec[2], r->spec[3], r->spec[4],
                     r->ureal[0], r->ureal[1], r->ureal[2], r->up[0], r->up[1], r->up[2], r->work[0], r->work[1],
-                    r->work[2], r->work[3], r->work[4], r->phisum, r->ukdc, r->dp, r->ds, r->sek, r->cphi, r->cidx,
+                    r->work[2], r->work[3], r->work[4], r->phisum, r->occ, r->ukdc, r->dp, r->ds, r->sek, r->cphi, r->cidx,
                     r->ccode, r->ccnt, r->d_ts, r->slipeps, r->slipdc, r->slipflag, r->xs};
     if (!r->arena)  // buffers carved from a batch arena stay with the arena
         for (void *b : bufs)

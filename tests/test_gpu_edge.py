@@ -11,6 +11,7 @@ from oracle import kref
 from kapsel3_amd import workloads
 from kapsel3_amd._abi import FP64, MIXED, Params, make_species
 
+import interposed
 from test_gpu_step import cmp_particles, rel, run_both
 
 pytestmark = pytest.mark.gpu
@@ -114,3 +115,35 @@ def test_largest_grid_mixed_vs_fp64(gpu):
     vs = np.abs(out[0]["v"]).max()
     assert vs > 0
     assert np.abs(out[1]["v"] - out[0]["v"]).max() <= 1e-4 * vs
+
+
+LIVE = """
+live = ctypes.c_int.in_dll(fake, "live")
+import numpy as np
+import kapsel3_amd
+from kapsel3_amd import workloads
+from kapsel3_amd._abi import JAX_Z, JP_SLIP, MIXED, Params, make_species
+for kind in ("plain", "mixed", "slip", "sheared"):
+    sp = [make_species(mass_ratio=1.0, propulsion=JP_SLIP, janus_axis=JAX_Z, slip_vel=0.01, slip_mode=1.3)
+          if kind == "slip" else make_species(mass_ratio=2.0)]
+    P = Params((32, 16, 16), a=2.0, a_xi=2.0, dt=0.05, species=sp, precision=MIXED if kind == "mixed" else 0)
+    with kapsel3_amd.Run(P, 2) as r:
+        r.set_particles(workloads.particles_at(np.array([[5.1, 6.2, 7.3], [20.4, 9.5, 3.6]]), spec=np.zeros(2, int),
+                                               q=workloads.random_quaternions(2, 3)))
+        r.init_fluid()
+        if kind == "sheared":
+            r.set_shear(0.01)
+            r.set_shear_history(4)
+        r.set_trajectory(4)
+        r.set_output(2, 2)
+        r.step(4)
+        r.get_fluid()
+        assert live.value > 0
+    print(kind, live.value)
+"""
+
+
+def test_run_gives_back_its_device_memory(gpu, tmp_path):
+    print("device memory after the runs", flush=True)
+    out = interposed.run(tmp_path, interposed.COUNTED, LIVE)
+    assert out.splitlines() == [k + " 0" for k in ("plain", "mixed", "slip", "sheared")], out
