@@ -190,7 +190,9 @@ int kh_get_slip_iterations(kh_run *run, long long *iterations, long long *loops)
  * min((SIGMA + XI)/2^(1/2n), SIGMA) as the reference's sheared runs take it
  * (input.cxx:549-566). Not for squirmer (slip) runs. The strain
  * degree_oblique (in (-NX/NY, NX/NY)) and Shear_rate_eff are run state,
- * saved and restored like zeta (resume.cxx:72, 566-580). */
+ * saved and restored like zeta (resume.cxx:72, 566-580). The first call
+ * allocates two more spectral fields than kh_run_bytes counts (285 MB at 256^3
+ * FP64); KH_ERR_NOMEM leaves the run as it was. */
 int kh_set_shear(kh_run *run, double shear_rate, int ac, double frequency);
 int kh_get_shear_state(kh_run *run, double *degree_oblique, double *shear_rate_eff);
 int kh_set_shear_state(kh_run *run, double degree_oblique, double shear_rate_eff);

@@ -1814,14 +1814,21 @@ int kh_set_shear(kh_run *r, double shear_rate, int ac, double frequency) {
     if (r->slip) return fail(KH_ERR_UNSUPPORTED, "the sheared step has no squirmer slip iteration");
     KH_TRY(settle_zeta(r));  // at the strain the last step left
     drop_graph(r);
-    if (!r->shear_last) {  // the stress record's device buffers
+    if (!r->shear_last) {  // the stress record's device buffers, omega_hat's two spectral fields
         const size_t np = (size_t)(r->np > 0 ? r->np : 1);
         r->shear_nacc   = obl_to_cart_blocks(r->g);
         if (hipMallocAsync((void **)&r->shear_pstress, sizeof(double) * 6 * np, r->stream) != hipSuccess ||
             hipMallocAsync((void **)&r->shear_acc, sizeof(double) * r->shear_nacc, r->stream) != hipSuccess ||
             hipMallocAsync(&r->shear_spec, 2 * 2 * r->esz * (size_t)r->g.nspec, r->stream) != hipSuccess ||
-            hipMallocAsync((void **)&r->shear_last, sizeof(double) * KH_SHEAR_RECORD, r->stream) != hipSuccess)
-            return fail(KH_ERR_NOMEM, "stress record buffers");
+            hipMallocAsync((void **)&r->shear_last, sizeof(double) * KH_SHEAR_RECORD, r->stream) != hipSuccess) {
+            (void)hipGetLastError();  // not the next launch's
+            for (void *b : {(void *)r->shear_pstress, (void *)r->shear_acc, r->shear_spec})
+                if (b) (void)hipFreeAsync(b, r->stream);
+            r->shear_pstress = r->shear_acc = nullptr;
+            r->shear_spec    = nullptr;
+            r->shear_last    = nullptr;
+            return fail(KH_ERR_NOMEM, "buffers of the sheared step");
+        }
         KH_HIP(hipMemsetAsync(r->shear_pstress, 0, sizeof(double) * 6 * np, r->stream));
         KH_HIP(hipMemsetAsync(r->shear_acc, 0, sizeof(double) * r->shear_nacc, r->stream));
         KH_HIP(hipMemsetAsync(r->shear_last, 0, sizeof(double) * KH_SHEAR_RECORD, r->stream));

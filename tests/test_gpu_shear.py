@@ -11,6 +11,7 @@ from oracle import kref
 from kapsel3_amd import workloads
 from kapsel3_amd._abi import FP64, MIXED, Params, make_species
 
+import interposed
 from test_gpu_step import cmp_particles, kept_mask, rel
 
 pytestmark = pytest.mark.gpu
@@ -278,6 +279,42 @@ def test_ns_solver_leaves_u(gpu):
     for d in range(3):
         assert rel(gr.get_field(f"u{d}")[..., :n], orc.get_field(f"u{d}")[..., :n]) < 1e-12, d
     gr.close()
+
+
+REFUSED = """
+calls, live, fail_at = (ctypes.c_int.in_dll(fake, k) for k in ("calls", "live", "fail_at"))
+import numpy as np
+import kapsel3_amd
+from kapsel3_amd._abi import Params
+out = []
+for refuse in (0, 1, 2, 3, 4):
+    with kapsel3_amd.Run(Params((16, 16, 16), a=1.0, a_xi=1.0, dt=0.05), 0) as r:
+        z = np.random.default_rng(3).standard_normal(r.shape)
+        r.set_fluid(z, z[::-1], [1.0, 2.0, 3.0])
+        if refuse:
+            fail_at.value = calls.value + refuse
+            try:
+                r.set_shear(0.1)
+                raise SystemExit("accepted")
+            except kapsel3_amd.KhError:
+                pass
+        r.step(2)  # still the plain step
+        r.set_shear(0.1)
+        r.step(2)
+        out.append(r.get_fluid())
+    print("live after the run", live.value)
+for f in out[1:]:
+    assert all(np.array_equal(a, b) for a, b in zip(f, out[0]))
+"""
+
+
+def test_refused_buffers_leave_the_run(gpu, tmp_path):
+    """kh_set_shear that cannot allocate one of its buffers says so, the run
+    goes on as it was, a later call is accepted, and the run gives back all
+    that was allocated."""
+    print("set_shear without memory", flush=True)
+    out = interposed.run(tmp_path, interposed.COUNTED, REFUSED)
+    assert out.splitlines() == 5 * ["live after the run 0"], out
 
 
 def test_deferred_modes_after_remap_and_transitions(gpu):
