@@ -603,14 +603,15 @@ template <typename T, int L, int E>
 static inline bool zw_split(long long nrows, unsigned nbatch) {
     return (long long)zw_blocks1<T, L, E>(nrows) * nbatch <= 1024;
 }
-// The force pass splits in FP64, where the mask is one bit a vector, and at
-// the lengths with 12 points per lane, whose three components in turn take 110
-// to 180 registers: 256^3 FP64 140 -> 131 us, 192^3 mixed 44 -> 39 us, 64^3
-// FP64 13.5 -> 10.4; in FP32 powers of two it would read phi_sum three times
-// (256^3 mixed 78 -> 89 us), so there only small grids do.
+// The force pass splits at the lengths with 12 points per lane, whose three
+// components in turn take 110 to 180 registers (192^3 mixed 40 -> 35 us, FP64 74 -> 70,
+// 192^3 squirmers 84 -> 82), and in FP64 where the mask is one bit a vector (256^3
+// 140 -> 131 us, 64^3 13.5 -> 10.4). Otherwise every wavefront of a line would read
+// all of phi_sum (256^3 mixed 78 -> 89 us, rigid FP64 125 -> 138, squirmers FP64
+// 137 -> 143), so there only small grids do.
 template <typename T, int L, int E>
-static inline bool zw_force_split(long long nrows, unsigned nbatch) {
-    return sizeof(T) == 8 || L % 3 == 0 || zw_split<T, L, E>(nrows, nbatch);
+static inline bool zw_force_split(long long nrows, unsigned nbatch, bool bits) {
+    return L % 3 == 0 || (sizeof(T) == 8 && bits) || zw_split<T, L, E>(nrows, nbatch);
 }
 
 template <typename T>
@@ -709,7 +710,7 @@ hipError_t zw_force(const Grid &g, T *const up[3], T *phis, T *const us[3], cpx<
     switch (g.nz) {
 #define KH_CASE(n)                                                                                                  \
     case n:                                                                                                         \
-        if (zw_force_split<T, n, ZwE<T, n>::force>(nrows, batch_z(g))) {                                            \
+        if (zw_force_split<T, n, ZwE<T, n>::force>(nrows, batch_z(g), occ.w != nullptr)) {                           \
             hipLaunchKernelGGL((k_zw_force<T, n, ZwE<T, n>::force, true>), dim3(zw_blocks1<T, n, ZwE<T, n>::force>(nrows), 1, batch_z(g)), dim3(192), 0, s, g, io, \
                                clear, tick, skip);                                                                  \
             return hipGetLastError();                                                                               \
