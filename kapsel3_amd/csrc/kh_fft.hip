@@ -12,7 +12,8 @@
 // with the 1/(NX NY NZ) normalisation folded into the last pass. Every pass
 // reads and writes each field element once: the z passes on the
 // wavefront-scope engine (kh_zwave.hip), the y and x passes a tile of C
-// neighbouring columns (C*elem = 128 B per row) staged in LDS.
+// neighbouring columns (C*elem = 128 B per row) in a workgroup's registers
+// (kh_col_fft.h).
 #include "kh_col_fft.h"
 #include "kh_fft.h"
 #include "kh_zwave.h"
@@ -78,17 +79,6 @@ hipError_t fft_z_r2c_multi(const Grid &g, const RIO<T> &io, int ncomp, hipStream
     return zw_r2c<T>(g.nz, io, ncomp, (long long)g.nx * g.ny, g.nzp, s, kzvalid);
 }
 template <typename T>
-hipError_t fft_z_r2c(const Grid &g, const T *in, cpx<T> *out, hipStream_t s, int kzvalid) {
-    return fft_z_r2c_multi<T>(g, RIO<T>{{in}, {out}}, 1, s, kzvalid);
-}
-template <typename T>
-hipError_t fft_z_c2r(const Grid &g, const cpx<T> *in, T *out, hipStream_t s, int kzvalid) {
-    ZIO<T> io{};
-    io.in[0]  = in;
-    io.out[0] = out;
-    return fft_z_c2r_multi<T>(g, io, 1, s, kzvalid);
-}
-template <typename T>
 hipError_t fft_z_c2r_multi(const Grid &g, const ZIO<T> &io, int ncomp, hipStream_t s, int kzvalid, const T *mask,
                            Occ occ) {
     const T   scale = (T)(1.0 / ((double)g.nx * (double)g.ny * (double)g.nz));
@@ -111,22 +101,12 @@ hipError_t fft_x(const Grid &g, const Comps<T> &data, int ncomp, hipStream_t s) 
 template <typename T>
 hipError_t fft3d_r2c(const Grid &g, const T *real_in, cpx<T> *spec_out, hipStream_t s) {
     hipError_t e;
-    if ((e = fft_z_r2c<T>(g, real_in, spec_out, s)) != hipSuccess) return e;
+    if ((e = fft_z_r2c_multi<T>(g, RIO<T>{{real_in}, {spec_out}}, 1, s, -1)) != hipSuccess) return e;
     if ((e = fft_y<T, true>(g, Comps<T>{{spec_out}}, 1, s)) != hipSuccess) return e;
     return fft_x<T, true>(g, Comps<T>{{spec_out}}, 1, s);
 }
 
-template <typename T>
-hipError_t fft3d_c2r(const Grid &g, cpx<T> *spec_inout, T *real_out, hipStream_t s) {
-    hipError_t e;
-    if ((e = fft_x<T, false>(g, Comps<T>{{spec_inout}}, 1, s)) != hipSuccess) return e;
-    if ((e = fft_y<T, false>(g, Comps<T>{{spec_inout}}, 1, s)) != hipSuccess) return e;
-    return fft_z_c2r<T>(g, spec_inout, real_out, s);
-}
-
 #define KH_INST(T)                                                                   \
-    template hipError_t fft_z_r2c<T>(const Grid &, const T *, cpx<T> *, hipStream_t, int); \
-    template hipError_t fft_z_c2r<T>(const Grid &, const cpx<T> *, T *, hipStream_t, int); \
     template hipError_t fft_z_r2c_multi<T>(const Grid &, const RIO<T> &, int, hipStream_t, int); \
     template hipError_t fft_z_c2r_multi<T>(const Grid &, const ZIO<T> &, int, hipStream_t, int, const T *, Occ); \
     template hipError_t fft_y<T, true>(const Grid &, const Comps<T> &, int, hipStream_t);          \
@@ -138,8 +118,5 @@ KH_INST(float)
 #undef KH_INST
 
 template hipError_t fft3d_r2c<double>(const Grid &, const double *, cpx<double> *, hipStream_t);
-template hipError_t fft3d_r2c<float>(const Grid &, const float *, cpx<float> *, hipStream_t);
-template hipError_t fft3d_c2r<double>(const Grid &, cpx<double> *, double *, hipStream_t);
-template hipError_t fft3d_c2r<float>(const Grid &, cpx<float> *, float *, hipStream_t);
 
 }  // namespace kh

@@ -12,8 +12,11 @@
 // Pointwise work between two passes on the same axis is fused into one
 // kernel: the real-space quadratic products sit between the inverse and the
 // forward z pass (k_zw_adv), the construction of u_hat from zeta sits in
-// front of the inverse x pass (k_x_zeta2u_inv), and the projection, the
-// addition of u* and the curl sit behind the forward x pass (k_x_f_zeta).
+// front of the inverse x pass (k_x_zeta2u_inv), -Omega, the slaved-Euler update
+// of zeta and u*_hat of the new zeta sit between the products' forward and the
+// inverse x pass (k_x_ns_u), and the projection, the addition of u* and the curl
+// sit behind the forward x pass (k_x_f_zeta), which in a captured chain of steps
+// goes on to the next step's u_hat and inverse x pass.
 #include "kh_col_fft.h"
 #include "kh_fused.h"
 #include "kh_modes.h"

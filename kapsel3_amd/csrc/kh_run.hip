@@ -170,7 +170,7 @@ struct kh_run {
     int             *bid   = nullptr;   // np: body of each bead
     double          *flo   = nullptr;   // np x 3: LJ force from partners of higher index
     std::vector<int> sek_host;          // the packed Sekibun offsets (host copy, for the initial block)
-    RowStage         stage;             // pinned staging of the field transfers
+    PinnedRows       stage;             // pinned staging of the field transfers
     // measurement
     bool                               timing = false;
     std::map<std::string, KernelTimes> times;
@@ -1485,9 +1485,9 @@ int run_create(const kh_params *P, int np, char *arena, size_t arena_bytes, kh_r
     if (st != KH_OK) return bail(st);
     hipStream_t  cs  = r->stream;
     const size_t psz = sizeof(DevParticle) * (size_t)(np > 0 ? np : 1);
-    // every buffer starts zeroed (the spectral rows' padding stays zero for
-    // good): the buffers of an arena, one after the other in it, by one fill
-    // (served runs are created one by one while others step: with the initial
+    // fields, spectra (whose rows' padding stays zero for good), particles and
+    // counters start zeroed; an arena, its buffers one after the other, whole by one
+    // fill (served runs are created one by one while others step: with the initial
     // block's three-component transforms 32 of them take 60.7 -> 58.4 ms)
     bool ok = true;
     auto clear = [&](void *p, size_t bytes) {

@@ -21,7 +21,7 @@ struct RowField {
 
 // Pinned staging of one run's transfers: allocated by the first, kept for
 // the next ones, given back with the run (release).
-struct RowStage {
+struct PinnedRows {
     static constexpr int WORKERS = 8, SLOTS = 2;  // slots per worker
     char      *buf       = nullptr;               // pinned, `slots` slots of slot_bytes
     size_t     slot_bytes = 0;
@@ -33,6 +33,6 @@ struct RowStage {
 // Moves nfields fields, ordered after the work on s; returns once the host
 // arrays are complete (to_host) or the rows are enqueued and the host arrays
 // no longer needed (to the device).
-hipError_t move_rows(RowStage &st, int device, const RowField *f, int nfields, bool to_host, hipStream_t s);
+hipError_t move_rows(PinnedRows &st, int device, const RowField *f, int nfields, bool to_host, hipStream_t s);
 
 }  // namespace kh

@@ -80,7 +80,7 @@ hipError_t launch(const Chunk &c, void *slot, bool out, hipStream_t s) {
     return out ? launch<double, true>(c, slot, s) : launch<double, false>(c, slot, s);
 }
 
-hipError_t reserve(RowStage &st, int slots, size_t slot_bytes) {
+hipError_t reserve(PinnedRows &st, int slots, size_t slot_bytes) {
     if (st.slots < slots || st.slot_bytes < slot_bytes) {
         st.release();
         hipError_t e = hipHostMalloc((void **)&st.buf, (size_t)slots * slot_bytes, hipHostMallocDefault);
@@ -133,8 +133,8 @@ hipError_t move_pageable(const RowField &f, bool out, hipStream_t s) {
 }
 
 // chunks w, w + step, w + 2 step, ... through slots w * SLOTS ..
-hipError_t work(RowStage &st, const Chunk *c, int n, int w, int step, bool out, hipStream_t s) {
-    constexpr int B = RowStage::SLOTS;
+hipError_t work(PinnedRows &st, const Chunk *c, int n, int w, int step, bool out, hipStream_t s) {
+    constexpr int B = PinnedRows::SLOTS;
     hipError_t    e = hipSuccess;
     auto          slot = [&](int k) { return w * B + k % B; };
     auto          buf  = [&](int k) { return st.buf + (size_t)slot(k) * st.slot_bytes; };
@@ -166,7 +166,7 @@ hipError_t work(RowStage &st, const Chunk *c, int n, int w, int step, bool out, 
 
 }  // namespace
 
-void RowStage::release() {
+void PinnedRows::release() {
     if (buf) (void)hipHostFree(buf);
     buf        = nullptr;
     slot_bytes = 0;
@@ -182,7 +182,7 @@ void RowStage::release() {
 // 32^3 FP64 14.2 -> 0.11 ms, 256^3 mixed (which converted on the host) 57 -> 6.1
 // ms, 512^3 mixed 422 -> 44 ms. Where the pinned memory is not to be had for
 // every worker one worker takes its two slots, and without those the runtime copies.
-static hipError_t move_rows_on(RowStage &st, int device, const RowField *f, int nfields, bool to_host, hipStream_t s) {
+static hipError_t move_rows_on(PinnedRows &st, int device, const RowField *f, int nfields, bool to_host, hipStream_t s) {
     std::vector<Chunk> c;
     size_t             most = 0;
     for (int i = 0; i < nfields; i++) {
@@ -197,10 +197,10 @@ static hipError_t move_rows_on(RowStage &st, int device, const RowField *f, int 
     if (n == 0) return hipSuccess;
     most = (most + 4095) / 4096 * 4096;
     // one worker, the calling thread, while all chunks fit its slots
-    int workers = std::max(1, std::min(RowStage::WORKERS, n / RowStage::SLOTS));
-    if (reserve(st, workers * RowStage::SLOTS, most) != hipSuccess) {
+    int workers = std::max(1, std::min(PinnedRows::WORKERS, n / PinnedRows::SLOTS));
+    if (reserve(st, workers * PinnedRows::SLOTS, most) != hipSuccess) {
         workers = 1;
-        if (reserve(st, RowStage::SLOTS, most) != hipSuccess) {
+        if (reserve(st, PinnedRows::SLOTS, most) != hipSuccess) {
             hipError_t e = hipSuccess;
             for (int i = 0; i < nfields && e == hipSuccess; i++) e = move_pageable(f[i], to_host, s);
             return e;
@@ -230,7 +230,7 @@ static hipError_t move_rows_on(RowStage &st, int device, const RowField *f, int 
     return (hipError_t)err.load();
 }
 
-hipError_t move_rows(RowStage &st, int device, const RowField *f, int nfields, bool to_host, hipStream_t s) {
+hipError_t move_rows(PinnedRows &st, int device, const RowField *f, int nfields, bool to_host, hipStream_t s) {
     int        dev = device;
     hipError_t e   = hipGetDevice(&dev);
     if (e == hipSuccess && dev != device) e = hipSetDevice(device);  // the caller's may be another

@@ -180,11 +180,6 @@ struct WaveE {
     static constexpr int value = L % 3 == 0 ? 12 : L < PREF ? L : (L / PREF > 64 ? L / 64 : PREF);
 };
 
-__host__ __device__ constexpr bool wave_fft_ok(int L) {
-    if (L % 3 == 0) return L >= 12 && L <= 384 && ((L / 3) & (L / 3 - 1)) == 0;
-    return L >= 8 && L <= 512 && (L & (L - 1)) == 0;
-}
-
 // LDS strip of one line in 128-byte groups (8 FP64 / 16 FP32 complex).
 // KH_WAVE_SWIZZLE 0: each group padded by one element; 1: no padding, the
 // element's slot within its group XORed with the group number, so that

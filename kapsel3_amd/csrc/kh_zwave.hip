@@ -117,7 +117,7 @@ __global__ __launch_bounds__(256) void k_zw_r2c(RIO<T> io, long long nrows, int 
 // consecutive points per lane per access: each lane moves 16-byte vectors
 // of both rows, so the HBM side of the z passes is fully coalesced.
 template <typename T, int L>
-struct RowStage {
+struct ZRow {
     static constexpr int V  = 4;      // points per vector
     static constexpr int NV = L / V;  // vectors per row
     using vec = typename std::conditional<sizeof(T) == 4, float4, double4>::type;
@@ -133,7 +133,7 @@ template <typename T, int L, int E>
 __global__ __launch_bounds__(256) void k_zw_c2r(ZIO<T> io, long long nrows, T scale, int kzv, int pitch) {
     using Geo = WaveGeom<T, L, E>;
     using F   = WaveFft<T, L, E, false, false>;
-    using RS  = RowStage<T, L>;
+    using RS  = ZRow<T, L>;
     __shared__ cpx<T> tw[F::TW], strips[(Geo::NT / 64) * Geo::W * Geo::LP];
     F::template fill_tw<Geo::NT>(tw);
     __syncthreads();
@@ -178,7 +178,7 @@ __global__ __launch_bounds__(256) void k_zw_c2r_masked(ZIO<T> io, int ncomp, con
                                                        const int *__restrict__ skip, Grid bg, Occ occ) {
     using Geo = WaveGeom<T, L, E>;
     using F   = WaveFft<T, L, E, false, false>;
-    using RS  = RowStage<T, L>;
+    using RS  = ZRow<T, L>;
     static_assert(L >= 4 * Geo::G, "four points per lane per row");
     constexpr int NT4 = RS::NV / Geo::G;  // vectors per lane per row
     if ((skip && *skip) || batch_skip(bg)) return;
@@ -234,7 +234,9 @@ __global__ __launch_bounds__(256) void k_zw_c2r_masked(ZIO<T> io, int ncomp, con
 // live: 4 points per lane in FP64 (204 registers at 256 points, two wavefronts
 // a SIMD), so it is bound by its transforms' LDS exchanges and by latency. 256^3
 // FP64 294 us (2.8 TB/s) against 488 us of the passes it replaces, 64^3 16.5
-// against 35; 192 points FP64 (12 per lane, spilling 300 bytes) 79 against 112.
+// against 35. At every FP64 length 3 * 2^a, 12 points per lane, it takes all 512 registers,
+// one wavefront a SIMD, and spills 152 to 348 bytes a lane; still 192 points 79
+// against 112.
 template <typename T, int L, int E>
 __global__ __launch_bounds__(256) void k_zw_obl_adv(Comps<T> u, Comps<T> w, Comps<T> out, long long nrows, T scale,
                                                     int kzv, int pitch) {
@@ -283,13 +285,14 @@ __global__ __launch_bounds__(256) void k_zw_obl_adv(Comps<T> u, Comps<T> w, Comp
 
 // Advection products (U2advection_k, operate_omega.cxx:31-47): inverse z
 // transforms of u1 (s0), u2 (s1), u3 (s2), the five products in registers,
-// forward z transforms into p0..p4. With LIVE3 all three components stay in
-// registers and each is read once; otherwise two are live at a time, so u2
-// is read and transformed twice; the order is u1 u2 -> p2, then u3 -> p1, p4,
-// then u2 again -> p0, p3. Either way a line's inputs are read before its
-// products are written, so a product buffer may be an input buffer:
-// p2 = s0, p1 = s2, p0 = s1 are allowed.
-template <typename T, int L, int E, bool LIVE3>
+// forward z transforms into p0..p4. All three components stay in registers, each
+// read and transformed once; with two of them live u2 is transformed twice,
+// which costs more than the registers save, also at 12 points per lane, where
+// FP64 takes 272 to 328, one wavefront a SIMD (192^3 134 us against 141, 128 x 128 x 384 129 against
+// 131, 192 x 192 x 96 74 against 81, 192^3 mixed 54 against 58). A line's inputs
+// are read before its products are written, so a product buffer may be an
+// input buffer: p2 = s0, p1 = s2, p0 = s1 are allowed.
+template <typename T, int L, int E>
 __global__ __launch_bounds__(256) void k_zw_adv(Grid g, const cpx<T> *__restrict__ s0, const cpx<T> *__restrict__ s1,
                                                 const cpx<T> *__restrict__ s2, cpx<T> *__restrict__ p0,
                                                 cpx<T> *__restrict__ p1, cpx<T> *__restrict__ p2,
@@ -307,82 +310,38 @@ __global__ __launch_bounds__(256) void k_zw_adv(Grid g, const cpx<T> *__restrict
     __syncthreads();
     const WaveLane<T, L, E> wl(strips, (long long)g.nx * g.ny, g.nzp);
     const int            kzv = g.trn_z;
-    if constexpr (LIVE3) {
-        cpx<T> a[E], b[E], c[E], v[E];
-        load_pair<T, L, Fi>(s0, wl, kzv, a);
-        load_pair<T, L, Fi>(s1, wl, kzv, b);
-        load_pair<T, L, Fi>(s2, wl, kzv, c);
-        Fi::run(a, wl.buf, twi, wl.g);
-        Fi::run(b, wl.buf, twi, wl.g);
-        Fi::run(c, wl.buf, twi, wl.g);
-#pragma unroll
-        for (int i = 0; i < E; i++) {
-            a[i] = cscale(a[i], scale);
-            b[i] = cscale(b[i], scale);
-            c[i] = cscale(c[i], scale);
-            v[i] = cmk(a[i].x * b[i].x, a[i].y * b[i].y);  // u1 u2
-        }
-        Ff::run(v, wl.buf, twf, wl.g);
-        store_pair<T, L, Ff>(v, wl, kzv, p2);
-#pragma unroll
-        for (int i = 0; i < E; i++) v[i] = cmk(c[i].x * a[i].x, c[i].y * a[i].y);  // u3 u1
-        Ff::run(v, wl.buf, twf, wl.g);
-        store_pair<T, L, Ff>(v, wl, kzv, p1);
-#pragma unroll
-        for (int i = 0; i < E; i++)  // u3^2 - u1^2
-            v[i] = cmk((c[i].x - a[i].x) * (c[i].x + a[i].x), (c[i].y - a[i].y) * (c[i].y + a[i].y));
-        Ff::run(v, wl.buf, twf, wl.g);
-        store_pair<T, L, Ff>(v, wl, kzv, p4);
-#pragma unroll
-        for (int i = 0; i < E; i++) v[i] = cmk(b[i].x * c[i].x, b[i].y * c[i].y);  // u2 u3
-        Ff::run(v, wl.buf, twf, wl.g);
-        store_pair<T, L, Ff>(v, wl, kzv, p0);
-#pragma unroll
-        for (int i = 0; i < E; i++)  // u2^2 - u3^2
-            v[i] = cmk((b[i].x - c[i].x) * (b[i].x + c[i].x), (b[i].y - c[i].y) * (b[i].y + c[i].y));
-        Ff::run(v, wl.buf, twf, wl.g);
-        store_pair<T, L, Ff>(v, wl, kzv, p3);
-        return;
-    }
-    cpx<T> ua[E], ub[E], v[E];
-    load_pair<T, L, Fi>(s0, wl, kzv, ua);
-    Fi::run(ua, wl.buf, twi, wl.g);
-    load_pair<T, L, Fi>(s1, wl, kzv, ub);
-    Fi::run(ub, wl.buf, twi, wl.g);
+    cpx<T> a[E], b[E], c[E], v[E];
+    load_pair<T, L, Fi>(s0, wl, kzv, a);
+    load_pair<T, L, Fi>(s1, wl, kzv, b);
+    load_pair<T, L, Fi>(s2, wl, kzv, c);
+    Fi::run(a, wl.buf, twi, wl.g);
+    Fi::run(b, wl.buf, twi, wl.g);
+    Fi::run(c, wl.buf, twi, wl.g);
 #pragma unroll
     for (int i = 0; i < E; i++) {
-        ua[i] = cscale(ua[i], scale);
-        ub[i] = cscale(ub[i], scale);
-        v[i]  = cmk(ua[i].x * ub[i].x, ua[i].y * ub[i].y);  // u1 u2
+        a[i] = cscale(a[i], scale);
+        b[i] = cscale(b[i], scale);
+        c[i] = cscale(c[i], scale);
+        v[i] = cmk(a[i].x * b[i].x, a[i].y * b[i].y);  // u1 u2
     }
     Ff::run(v, wl.buf, twf, wl.g);
     store_pair<T, L, Ff>(v, wl, kzv, p2);
-    load_pair<T, L, Fi>(s2, wl, kzv, ub);  // ub := u3
-    Fi::run(ub, wl.buf, twi, wl.g);
 #pragma unroll
-    for (int i = 0; i < E; i++) {
-        ub[i] = cscale(ub[i], scale);
-        v[i]  = cmk(ub[i].x * ua[i].x, ub[i].y * ua[i].y);  // u3 u1
-    }
+    for (int i = 0; i < E; i++) v[i] = cmk(c[i].x * a[i].x, c[i].y * a[i].y);  // u3 u1
     Ff::run(v, wl.buf, twf, wl.g);
     store_pair<T, L, Ff>(v, wl, kzv, p1);
 #pragma unroll
     for (int i = 0; i < E; i++)  // u3^2 - u1^2
-        v[i] = cmk((ub[i].x - ua[i].x) * (ub[i].x + ua[i].x), (ub[i].y - ua[i].y) * (ub[i].y + ua[i].y));
+        v[i] = cmk((c[i].x - a[i].x) * (c[i].x + a[i].x), (c[i].y - a[i].y) * (c[i].y + a[i].y));
     Ff::run(v, wl.buf, twf, wl.g);
     store_pair<T, L, Ff>(v, wl, kzv, p4);
-    load_pair<T, L, Fi>(s1, wl, kzv, ua);  // ua := u2 again
-    Fi::run(ua, wl.buf, twi, wl.g);
 #pragma unroll
-    for (int i = 0; i < E; i++) {
-        ua[i] = cscale(ua[i], scale);
-        v[i]  = cmk(ua[i].x * ub[i].x, ua[i].y * ub[i].y);  // u2 u3
-    }
+    for (int i = 0; i < E; i++) v[i] = cmk(b[i].x * c[i].x, b[i].y * c[i].y);  // u2 u3
     Ff::run(v, wl.buf, twf, wl.g);
     store_pair<T, L, Ff>(v, wl, kzv, p0);
 #pragma unroll
     for (int i = 0; i < E; i++)  // u2^2 - u3^2
-        v[i] = cmk((ua[i].x - ub[i].x) * (ua[i].x + ub[i].x), (ua[i].y - ub[i].y) * (ua[i].y + ub[i].y));
+        v[i] = cmk((b[i].x - c[i].x) * (b[i].x + c[i].x), (b[i].y - c[i].y) * (b[i].y + c[i].y));
     Ff::run(v, wl.buf, twf, wl.g);
     store_pair<T, L, Ff>(v, wl, kzv, p3);
 }
@@ -444,7 +403,7 @@ __global__ __launch_bounds__(SPLIT ? 192 : 256) void k_zw_force(Grid g, ZForceIO
                                                                 const int *__restrict__ skip) {
     using Geo = WaveGeom<T, L, E>;
     using Ff  = WaveFft<T, L, E, true, true>;
-    using RS  = RowStage<T, L>;
+    using RS  = ZRow<T, L>;
     static_assert(L >= 4 * Geo::G, "four points per lane per row");
     constexpr int NT4 = RS::NV / Geo::G;  // vectors per lane per row
     if ((skip && *skip) || batch_skip(g)) return;
@@ -569,17 +528,10 @@ __global__ __launch_bounds__(SPLIT ? 192 : 256) void k_zw_force(Grid g, ZForceIO
 #ifndef KH_FORCE_E32
 #define KH_FORCE_E32 4
 #endif
-// the advection pass keeps all three components live (each read once) at
-// this many points per lane or fewer: at 8 (FP32 and FP64) the extra
-// registers cost less than the second read and transform of u2
-#ifndef KH_ADV_LIVE3_E
-#define KH_ADV_LIVE3_E 12
-#endif
 template <typename T, int L>
 struct ZwE {
     static constexpr int  pass  = WaveE<T, L, sizeof(T) == 4 ? KH_PASS_E32 : KH_PASS_E64>::value;
     static constexpr int  adv   = WaveE<T, L, sizeof(T) == 4 ? KH_ADV_E32 : KH_ADV_E64>::value;
-    static constexpr bool live3 = adv <= KH_ADV_LIVE3_E;
     static constexpr int  force = WaveE<T, L, sizeof(T) == 4 ? KH_FORCE_E32 : KH_FORCE_E64>::value;
     static constexpr int  obl   = WaveE<T, L, sizeof(T) == 4 ? 8 : 4>::value;  // seven components live
 };
@@ -684,7 +636,7 @@ hipError_t zw_adv(const Grid &g, cpx<T> *const s3[3], cpx<T> *const p5[5], T sca
             hipLaunchKernelGGL((k_zw_adv_split<T, n, ZwE<T, n>::adv>), dim3(zw_blocks1<T, n, ZwE<T, n>::adv>(nrows), 1, batch_z(g)), dim3(320), 0, s, g, in, out, scale); \
             return hipGetLastError();                                                                             \
         }                                                                                                         \
-        hipLaunchKernelGGL((k_zw_adv<T, n, ZwE<T, n>::adv, ZwE<T, n>::live3>), dim3(zw_blocks<T, n, ZwE<T, n>::adv>(nrows), 1, batch_z(g)), dim3(256), 0, s, g, s3[0], s3[1], s3[2], \
+        hipLaunchKernelGGL((k_zw_adv<T, n, ZwE<T, n>::adv>), dim3(zw_blocks<T, n, ZwE<T, n>::adv>(nrows), 1, batch_z(g)), dim3(256), 0, s, g, s3[0], s3[1], s3[2], \
                            p5[0], p5[1], p5[2], p5[3], p5[4], scale);                                             \
         return hipGetLastError();
         KH_FOR_EACH_WL(KH_CASE)
