@@ -70,9 +70,8 @@ def test_slip_functions_fp64(gpu):
     g.close()
 
 
-# 32^3: the fused step's slip loop decided on the device (captured as
-# graphs); 48^3: the same step with the loop decided on the host (NZ not a
-# power of two)
+# the fused step's slip loop is decided on the device (captured as graphs), at
+# powers of two and at 3 * 2^a; the reference-order path's on the host
 @pytest.mark.parametrize("path,n", [("fused", 32), ("reference", 32), ("fused", 48)])
 def test_squirmer_steps_fp64(gpu, path, n):
     print(f"squirmers {n}^3 x 4, 40 steps, {path}", flush=True)
