@@ -4,6 +4,9 @@
 
 #include <hip/hip_runtime.h>
 
+#include <memory>
+#include <mutex>
+
 namespace kh {
 
 // One field: `rows` rows of `width` elements, `pitch` elements apart on the
@@ -27,6 +30,8 @@ struct PinnedRows {
     size_t     slot_bytes = 0;
     int        slots      = 0;
     hipEvent_t done[WORKERS * SLOTS] = {};
+    // held by each transfer: threads that read one run at a time share the slots
+    std::shared_ptr<std::mutex> lock = std::make_shared<std::mutex>();
     void       release();
 };
 

@@ -231,8 +231,9 @@ static hipError_t move_rows_on(PinnedRows &st, int device, const RowField *f, in
 }
 
 hipError_t move_rows(PinnedRows &st, int device, const RowField *f, int nfields, bool to_host, hipStream_t s) {
-    int        dev = device;
-    hipError_t e   = hipGetDevice(&dev);
+    std::lock_guard<std::mutex> held(*st.lock);
+    int                         dev = device;
+    hipError_t                  e   = hipGetDevice(&dev);
     if (e == hipSuccess && dev != device) e = hipSetDevice(device);  // the caller's may be another
     if (e != hipSuccess) return e;
     try {

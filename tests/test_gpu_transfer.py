@@ -3,6 +3,8 @@ kh_get_fluid): the rows come back as they went in, bit for bit in FP64 and
 rounded once to FP32 in a mixed run, with the real fields' padding columns
 zero. Sizes with one chunk, with a last chunk of a few rows and with several
 worker threads; and the same without the pinned staging."""
+import concurrent.futures
+
 import numpy as np
 import pytest
 
@@ -31,6 +33,32 @@ def test_fields_round_trip(gpu, n, precision):
             u = r.get_field("u1")
             assert np.array_equal(u[..., :n[2]], stored(z[2])[..., :n[2]])
             assert not u[..., n[2]:].any()
+
+
+def test_threads_read_one_run(gpu):
+    """Several threads at once, fluid and fields of different sizes of staging:
+    each gets what a single thread gets."""
+    n = (64, 64, 96)
+    print(f"transfer {n}, four threads", flush=True)
+    rng = np.random.default_rng(8)
+    with gpu.Run(Params(n, a=1.0, a_xi=1.0), 0) as r:
+        z = [rng.standard_normal(r.shape) for _ in range(4)]
+        r.set_fluid(z[0], z[1], [1.0, 2.0, 3.0])
+        r.set_field("u1", z[2])
+        r.set_field("u2", z[3])
+
+        def read(k):
+            for _ in range(6):
+                if k % 2:
+                    z0, z1, uk = r.get_fluid()
+                    assert np.array_equal(z0, z[0]) and np.array_equal(z1, z[1]) and np.array_equal(uk, [1.0, 2.0, 3.0])
+                else:
+                    u = r.get_field("u%d" % (1 + k // 2))[..., :n[2]]
+                    assert np.array_equal(u, z[2 + k // 2][..., :n[2]])
+            return True
+
+        with concurrent.futures.ThreadPoolExecutor(4) as ex:
+            assert list(ex.map(read, range(4))) == 4 * [True]
 
 
 # hipHostMalloc that fails (hipErrorOutOfMemory) beyond `limit` bytes
