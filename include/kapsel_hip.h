@@ -105,7 +105,10 @@ typedef struct kh_params {
 typedef struct kh_run kh_run;
 
 /* Fields that can be read or written in the reference's real-space layout
- * (NX*NY*NZ_ doubles, NZ_ = 2*(NZ/2+1), padding columns ignored). */
+ * (NX*NY*NZ_ doubles, NZ_ = 2*(NZ/2+1), padding columns ignored). A fused
+ * step (KH_PATH_FUSED) leaves u* in u, and that only around the particles
+ * (everywhere in squirmer runs), and zeros in up and phi_sum, on every grid:
+ * kh_apply forms them whole (KH_FN_ZETA_K2U, KH_FN_MAKE_PHI, KH_FN_MAKE_UP). */
 enum kh_field {
     KH_FIELD_U0 = 0, KH_FIELD_U1, KH_FIELD_U2,    /* u   (fft_wrapper.cxx:20) */
     KH_FIELD_UP0, KH_FIELD_UP1, KH_FIELD_UP2,     /* up  (fft_wrapper.cxx:20) */
