@@ -11,7 +11,10 @@
 // shear) on the fused step path join.
 #pragma once
 
+#include <hip/hip_runtime.h>
 #include <stddef.h>
+
+#include <vector>
 
 #include "../../include/kapsel_hip.h"
 
@@ -19,10 +22,36 @@ struct kh_batch;
 
 namespace kh {
 
+// Streams that the runs and batches of one server use one after the other:
+// creating and destroying one costs 0.2 to 0.7 ms (hardware queues come and go
+// with them), and a served run of small size lives for some ms. One thread's; no
+// more of them than runs and batches were ever resident at once; given back with
+// the server.
+class RunStreams {
+  public:
+    hipError_t take(hipStream_t *s) {
+        if (idle_.empty()) return hipStreamCreateWithFlags(s, hipStreamNonBlocking);
+        *s = idle_.back();
+        idle_.pop_back();
+        return hipSuccess;
+    }
+    void give(hipStream_t s) { idle_.push_back(s); }  // s is drained
+    void release() {
+        for (hipStream_t s : idle_) (void)hipStreamDestroy(s);
+        idle_.clear();
+    }
+
+  private:
+    std::vector<hipStream_t> idle_;
+};
+
+// kh_run_create on a stream of `streams`, which takes it back when the run is destroyed
+int run_create_on(RunStreams *streams, const kh_params *P, int np, kh_run **out);
+
 // arena bytes per slot for runs of P's class with up to np_cap particles
 size_t batch_stride(const kh_params &P, int np_cap);
 // P's grid, precision, dx, rho, eta, dt, FIX_CELL, a and a_xi define the class
-int  batch_create(const kh_params &P, int np_cap, int capacity, kh_batch **out);
+int  batch_create(RunStreams *streams, const kh_params &P, int np_cap, int capacity, kh_batch **out);
 bool batch_accepts(const kh_batch *b, const kh_params &P, int np);
 int  batch_free_slot(const kh_batch *b);  // -1: none
 int  batch_run_create(kh_batch *b, int slot, const kh_params *P, int np, kh_run **out);

@@ -90,6 +90,7 @@ struct kh_run {
     int                     device = 0;
     hipStream_t             stream = nullptr;
     hipStream_t             own_stream = nullptr;  // stream created with the run (stream differs while batched)
+    RunStreams             *streams    = nullptr;  // where own_stream came from and goes back to (nullptr: the run's)
     // a run inside a batch arena (kh_batch): its device buffers are
     // sub-allocated from arena in a fixed order, slot * stride after the
     // batch's first arena
@@ -197,6 +198,7 @@ struct kh_batch {
     void                 *dslots = nullptr;    // device SlotPart<T> per slot
     std::vector<char>     hslots;              // its host copy
     hipStream_t           stream = nullptr;
+    kh::RunStreams       *streams = nullptr;   // where stream and its runs' streams came from and go back to
     std::vector<kh_run *> slot_run;  // the run created in each slot (nullptr: free)
     bool                  dirty  = true;
     hipGraph_t            graph1 = nullptr, graphk = nullptr;
@@ -1057,7 +1059,12 @@ int free_run(kh_run *r) {
     }
     for (auto e : r->event_pool) (void)hipEventDestroy(e);
     r->stage.release();
-    if (r->stream) (void)hipStreamDestroy(r->stream);
+    if (r->stream) {
+        if (r->streams)
+            r->streams->give(r->stream);
+        else
+            (void)hipStreamDestroy(r->stream);
+    }
     delete r;
     return KH_OK;
 }
@@ -1340,7 +1347,7 @@ const char *kh_strerror(int s) {
 // (in the same order and sizes for every run of one grid and precision, so
 // the field buffers sit at the same offsets in every arena) and not freed
 // with the run.
-int run_create(const kh_params *P, int np, char *arena, size_t arena_bytes, kh_run **out) {
+int run_create(RunStreams *streams, const kh_params *P, int np, char *arena, size_t arena_bytes, kh_run **out) {
     if (!out) return fail(KH_ERR_ARG, "out is NULL");
     *out = nullptr;
     KH_TRY(check_params(P, np));
@@ -1358,8 +1365,11 @@ int run_create(const kh_params *P, int np, char *arena, size_t arena_bytes, kh_r
         return s;
     };
     if (hipGetDevice(&r->device) != hipSuccess) return bail(fail(KH_ERR_HIP, "no HIP device"));
-    if (hipStreamCreateWithFlags(&r->stream, hipStreamNonBlocking) != hipSuccess)
+    r->streams = streams;
+    if ((streams ? streams->take(&r->stream) : hipStreamCreateWithFlags(&r->stream, hipStreamNonBlocking)) != hipSuccess) {
+        r->stream = nullptr;
         return bail(fail(KH_ERR_HIP, "hipStreamCreate failed"));
+    }
     r->own_stream = r->stream;
 
     // Set_global_parameters (input.cxx:424-600)
@@ -1550,7 +1560,7 @@ int run_create(const kh_params *P, int np, char *arena, size_t arena_bytes, kh_r
 
 extern "C" {
 
-int kh_run_create(const kh_params *P, int np, kh_run **out) { return run_create(P, np, nullptr, 0, out); }
+int kh_run_create(const kh_params *P, int np, kh_run **out) { return run_create(nullptr, P, np, nullptr, 0, out); }
 
 int kh_run_destroy(kh_run *r) { return free_run(r); }
 
@@ -2379,8 +2389,8 @@ bool batch_accepts(const kh_batch *b, const kh_params &P, int np) {
     return run_footprint(P, np) <= b->stride;
 }
 
-int batch_create(const kh_params &P, int np_cap, int capacity, kh_batch **out) {
-    if (!out || capacity < 1 || np_cap < 1 || np_cap > 256) return fail(KH_ERR_ARG, "bad batch arguments");
+int batch_create(RunStreams *streams, const kh_params &P, int np_cap, int capacity, kh_batch **out) {
+    if (!out || !streams || capacity < 1 || np_cap < 1 || np_cap > 256) return fail(KH_ERR_ARG, "bad batch arguments");
     *out        = nullptr;
     kh_batch *b = new kh_batch();
     b->P        = P;
@@ -2388,6 +2398,7 @@ int batch_create(const kh_params &P, int np_cap, int capacity, kh_batch **out) {
     b->P.nspecies = 0;
     b->capacity = capacity;
     b->np_cap   = np_cap;
+    b->streams  = streams;
     b->stride   = batch_stride(P, np_cap);
     b->hactive.assign(capacity, 0);
     b->hslots.assign(sizeof(SlotPart<double>) * (size_t)capacity, 0);
@@ -2397,12 +2408,14 @@ int batch_create(const kh_params &P, int np_cap, int capacity, kh_batch **out) {
         if (b->base) (void)hipFree(b->base);
         if (b->active) (void)hipFree(b->active);
         if (b->dslots) (void)hipFree(b->dslots);
-        if (b->stream) (void)hipStreamDestroy(b->stream);
+        if (b->stream) streams->give(b->stream);
         delete b;
         return st;
     };
-    if (hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess)
+    if (streams->take(&b->stream) != hipSuccess) {
+        b->stream = nullptr;
         return bail(fail(KH_ERR_HIP, "hipStreamCreate failed"));
+    }
     if (hipMallocAsync((void **)&b->base, b->stride * (size_t)capacity, b->stream) != hipSuccess) {
         b->base = nullptr;
         return bail(fail(KH_ERR_NOMEM, "batch arena of %zu bytes", b->stride * (size_t)capacity));
@@ -2423,6 +2436,10 @@ int batch_create(const kh_params &P, int np_cap, int capacity, kh_batch **out) {
     return KH_OK;
 }
 
+int run_create_on(RunStreams *streams, const kh_params *P, int np, kh_run **out) {
+    return run_create(streams, P, np, nullptr, 0, out);
+}
+
 int batch_free_slot(const kh_batch *b) {
     for (int k = 0; k < b->capacity; k++)
         if (!b->slot_run[k]) return k;
@@ -2433,7 +2450,7 @@ int batch_run_create(kh_batch *b, int slot, const kh_params *P, int np, kh_run *
     if (!b || !P || !out || slot < 0 || slot >= b->capacity || b->slot_run[slot])
         return fail(KH_ERR_ARG, "slot %d is not free", slot);
     if (!batch_accepts(b, *P, np)) return fail(KH_ERR_ARG, "run is not of the batch's class");
-    KH_TRY(run_create(P, np, b->base + (size_t)slot * b->stride, b->stride, out));
+    KH_TRY(run_create(b->streams, P, np, b->base + (size_t)slot * b->stride, b->stride, out));
     (*out)->slot     = slot;
     b->slot_run[slot] = *out;
     return KH_OK;
@@ -2590,7 +2607,7 @@ int batch_destroy(kh_batch *b) {
     (void)hipFreeAsync(b->active, b->stream);
     (void)hipFreeAsync(b->dslots, b->stream);
     (void)hipStreamSynchronize(b->stream);
-    (void)hipStreamDestroy(b->stream);
+    b->streams->give(b->stream);
     delete b;
     return KH_OK;
 }

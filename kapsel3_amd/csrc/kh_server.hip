@@ -78,6 +78,7 @@ struct kh_server {
     std::map<long long, std::unique_ptr<Request>> all;
     std::vector<Request *>                 active;  // scheduler thread only
     std::vector<std::pair<kh_batch *, long long>> batches;  // with their arena bytes (scheduler thread only)
+    kh::RunStreams                         streams;  // of finished runs, for the next ones (scheduler thread only)
     long long                              used = 0, peak_bytes = 0, next_id = 1;
     int                                    peak_active = 0, nactive = 0;
     bool                                   stop = false, started = false;
@@ -122,10 +123,10 @@ void finish(kh_server *S, Request *q, int status, const char *err) {
 
 // Device side of admission: create the run (in its batch slot, if any),
 // upload, initial constraint block; a batched run takes its first step alone.
-int start(Request *q) {
+int start(kh_server *S, Request *q) {
     const int np = (int)q->parts.size();
     int       st = q->batch ? kh::batch_run_create(q->batch, q->slot, &q->P, np, &q->run)
-                            : kh_run_create(&q->P, np, &q->run);
+                            : kh::run_create_on(&S->streams, &q->P, np, &q->run);
     if (st == KH_OK) st = kh_set_particles(q->run, q->parts.data(), np);
     if (st == KH_OK) st = kh_init_fluid(q->run);
     if (st == KH_OK) st = kh_set_trajectory(q->run, q->nsteps);
@@ -204,7 +205,7 @@ void loop(kh_server *S) {
                 q              = h;
             }
             if (new_slots) {
-                const int bst = kh::batch_create(q->P, KH_BATCH_NP_CAP, new_slots, &b);
+                const int bst = kh::batch_create(&S->streams, q->P, KH_BATCH_NP_CAP, new_slots, &b);
                 if (bst != KH_OK) {
                     const std::string e = kh_last_error();
                     {
@@ -219,7 +220,7 @@ void loop(kh_server *S) {
             }
             q->batch  = b;
             q->slot   = slot;
-            const int st = start(q);
+            const int st = start(S, q);
             if (st != KH_OK) {
                 const std::string e = kh_last_error();
                 leave(q);
@@ -346,6 +347,7 @@ void loop(kh_server *S) {
             }
         }
     }
+    S->streams.release();
 }
 
 }  // namespace

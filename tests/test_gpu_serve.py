@@ -9,6 +9,8 @@ from oracle import kref
 from kapsel3_amd import serving, workloads
 from kapsel3_amd._abi import MIXED, FP64
 
+import interposed
+
 pytestmark = pytest.mark.gpu
 
 
@@ -104,3 +106,48 @@ def test_admission_by_budget(gpu):
             srv.wait(rid)
         st = srv.stats()
     assert st["completed"] == 6 and st["peak_active"] <= 2 and st["peak_bytes"] <= st["budget"]
+
+
+STREAMS = """
+int made = 0, live = 0;
+int hipStreamCreateWithFlags(void **s, unsigned flags) {
+    int e = ((int (*)(void **, unsigned))hip("hipStreamCreateWithFlags"))(s, flags);
+    made += e == 0, live += e == 0;
+    return e;
+}
+int hipStreamDestroy(void *s) {
+    live--;
+    return ((int (*)(void *))hip("hipStreamDestroy"))(s);
+}
+"""
+
+SERVED = """
+made, live = (ctypes.c_int.in_dll(fake, k) for k in ("made", "live"))
+import numpy as np
+import kapsel3_amd
+from kapsel3_amd import workloads
+from kapsel3_amd._abi import FP64
+runs = [workloads.sedimentation(n, 4, a=2.0, kbt=0.0, precision=FP64, seed=s, gap=1.0) for s in range(6) for n in (16, 32)]
+out = []
+for rep in range(2):
+    with kapsel3_amd.Server(max_active=4, chunk_steps=8, batch_slots=4) as srv:
+        for burst in range(3):
+            ids = [srv.submit(P, p, 24) for P, p in runs]
+            for rid, _ in ids:
+                srv.wait(rid)
+            out.append([t for _, t in ids])
+    print(made.value <= 4 + 2, live.value)
+    made.value = 0
+vs = max(np.abs(t[..., 3:]).max() for t in out[0])
+for o in out[1:]:
+    for a, b in zip(o, out[0]):
+        assert np.abs(a[..., 3:] - b[..., 3:]).max() < 1e-10 * vs
+"""
+
+
+def test_streams_are_reused_and_given_back(gpu, tmp_path):
+    """A server makes as many streams as runs and batches are resident at once
+    (4 and 2 here, for 36 runs), and destroys them with it; later runs on the same
+    streams go as the first ones."""
+    print("served runs, streams", flush=True)
+    assert interposed.run(tmp_path, STREAMS, SERVED).splitlines() == 2 * ["True 0"]
